@@ -193,8 +193,10 @@ int ds5_hip_kv_append(ds5_hip_ctx* ctx, const ds5_kv_append_args* args);
  * not the valid length. Replaces kernels_b.zig:29-133 gqaAttention (Metal:
  * kernels/gpu/kernels.zig:254-286). n_tokens == 1 runs the split-K
  * flash-decoding kernels, n_tokens > 1 the causal MFMA prefill kernel
- * (f16 cache, head_dim 64 or 128); other shapes and f32 caches run a generic
- * streaming kernel. All paths are device code. */
+ * (f16 cache, head_dim 64 or 128), f32 caches of head_dim 64 or 128 the f32
+ * matrix-core kernel (one or many tokens; split over positions, and merged, where
+ * the context workspace has or may get room for the partials, else one split);
+ * other shapes run a generic streaming kernel. All paths are device code. */
 typedef struct ds5_attn_args {
     ds5_buf q;       /* f32 [n_tokens, n_q_heads, head_dim], post-norm post-rope */
     ds5_buf k_cache; /* kv_dtype [n_kv_heads, max_ctx, head_dim] */

@@ -97,6 +97,9 @@ int ds5_fail(ds5_hip_ctx* ctx, int code, const char* fmt, ...) __attribute__((fo
 int ds5_hip_status(ds5_hip_ctx* ctx, hipError_t err, const char* what);
 int ds5_after_launch(ds5_hip_ctx* ctx, const char* what);
 int ds5_workspace(ds5_hip_ctx* ctx, size_t bytes, void** out);
+// The workspace if `bytes` of it can be had: false, with no error left behind, where a
+// stream capture would have to allocate, the static scratch is smaller, or memory is out.
+bool ds5_workspace_if(ds5_hip_ctx* ctx, size_t bytes, void** out);
 int ds5_aux_workspace(ds5_hip_ctx* ctx, size_t bytes, void** out);
 // Looks up (once per device) the address of the static scratch array on the
 // context's device, which must be current, and records it in the context.
@@ -290,6 +293,24 @@ struct KvAppendLaunch {
 };
 int launch_kv_append(ds5_hip_ctx* ctx, const KvAppendLaunch& a);
 
+// rmsNorm of q and k, rope of q (in place) and k, and the append of k and v, one launch:
+// what launch_rms_norm, launch_rope and launch_kv_append write (k itself stays as it was),
+// bit for bit. head_dim <= kRmsSerialMaxDim; q, k and v disjoint.
+struct StepPrepLaunch {
+    float* q;
+    const float* k;
+    const float* v;
+    const float* q_norm;
+    const float* k_norm;
+    const int32_t* positions;
+    void* k_cache;
+    void* v_cache;
+    uint32_t kv_dtype, pos, n_tokens, n_q_heads, n_kv_heads, head_dim, max_ctx;
+    float eps, freq_scale;
+    const RopeTable* table;
+};
+int launch_step_prep(ds5_hip_ctx* ctx, const StepPrepLaunch& a);
+
 // Prefill pre-pass of the fused step: per token, the norm + rope + f16 append
 // of every kv head's k row, f16 append of v, and the rope cos/sin of the token
 // into cs [n_tokens, head_dim] (cos of pairs 0 .. head_dim/2 - 1, then sin),
@@ -321,6 +342,17 @@ struct GenericAttnLaunch {
     float scale;
 };
 int launch_generic_attention(ds5_hip_ctx* ctx, const GenericAttnLaunch& a);
+// The same over f32 caches with head_dim 64 or 128, q, caches and out 16-byte aligned, on
+// the f32 matrix cores (k_attn_f32.hip). chunk positions per split, at most kAttnF32MaxSplits
+// splits; wave_rows: a wavefront per 16-row tile instead of a workgroup.
+constexpr uint32_t kAttnF32MaxSplits = 64;
+struct AttnF32Plan {
+    uint32_t row_tiles, chunk, n_splits;
+    bool wave_rows;
+};
+AttnF32Plan attn_f32_plan(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads);
+size_t attn_f32_workspace_bytes(uint32_t n_tokens, uint32_t n_q_heads, uint32_t head_dim, uint32_t n_splits);
+int launch_attn_f32(ds5_hip_ctx* ctx, const GenericAttnLaunch& a);
 
 // Split-K MFMA decode (one query token per sequence), f16 cache, head_dim 64
 // or 128. Covers the contiguous and paged caches, with or without the fused

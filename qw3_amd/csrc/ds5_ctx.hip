@@ -76,6 +76,26 @@ int ds5_workspace(ds5_hip_ctx* ctx, size_t bytes, void** out) {
     return DS5_OK;
 }
 
+bool ds5_workspace_if(ds5_hip_ctx* ctx, size_t bytes, void** out) {
+    if (ctx->use_scratch) {
+        *out = ctx->scratch;
+        return bytes <= ctx->scratch_bytes;
+    }
+    if (bytes > ctx->workspace_bytes) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return false;
+        const std::string before = ctx->last_error;
+        void* ws = nullptr;
+        if (ds5_workspace(ctx, bytes, &ws)) {
+            (void)hipGetLastError();
+            ctx->last_error = before;
+            return false;
+        }
+    }
+    *out = ctx->workspace;
+    return true;
+}
+
 int ds5_aux_workspace(ds5_hip_ctx* ctx, size_t bytes, void** out) {
     if (int rc = grow_buffer(ctx, bytes, ctx->aux, ctx->aux_bytes, "workspace")) return rc;
     *out = ctx->aux;

@@ -117,6 +117,11 @@ bool covers(ds5_buf b, uint64_t bytes) { return b.len >= bytes && (bytes == 0 ||
 
 bool aligned16(ds5_buf b) { return ((uintptr_t)ds5_ptr(b) & 15u) == 0; }
 
+bool disjoint(ds5_buf a, uint64_t a_bytes, ds5_buf b, uint64_t b_bytes) {
+    const uintptr_t p = (uintptr_t)ds5_ptr(a), q = (uintptr_t)ds5_ptr(b);
+    return p + a_bytes <= q || q + b_bytes <= p;
+}
+
 uint64_t cache_elem_bytes(uint32_t kv_dtype) {
     return kv_dtype == DS5_DTYPE_F32 ? 4 : kv_dtype == DS5_DTYPE_F16 ? 2 : 0;
 }
@@ -643,6 +648,9 @@ int ds5_hip_gqa_attention(ds5_hip_ctx* ctx, const ds5_attn_args* a) {
     GenericAttnLaunch g{(const float*)ds5_ptr(a->q), ds5_ptr(a->k_cache), ds5_ptr(a->v_cache), (float*)ds5_ptr(a->out),
                         a->kv_dtype, a->pos, a->n_tokens, a->n_q_heads, a->n_kv_heads, a->head_dim, a->max_ctx,
                         a->scale};
+    if (a->kv_dtype == DS5_DTYPE_F32 && (a->head_dim == 64 || a->head_dim == 128) && aligned16(a->q) &&
+        aligned16(a->k_cache) && aligned16(a->v_cache) && aligned16(a->out))
+        return launch_attn_f32(ctx, g);
     return launch_generic_attention(ctx, g);
 }
 
@@ -754,9 +762,42 @@ int ds5_hip_attention_step(ds5_hip_ctx* ctx, const ds5_attention_step_args* a) {
         }
     }
 
-    // Other shapes: the six separate device ops, in place on q and k.
+    // Other shapes (f32 caches, other head sizes): norm, rope and append in one launch,
+    // then the attention op. Views that overlap, longer heads: the six separate ops, in
+    // place on q and k.
     float* q = (float*)ds5_ptr(a->q);
     float* k = (float*)ds5_ptr(a->k);
+    const uint64_t q_bytes = T * hq * hd * 4, kv_bytes = T * hkv * hd * 4;
+    const uint64_t cache_bytes = hkv * a->max_ctx * hd * cache_elem_bytes(a->kv_dtype);
+    const struct { ds5_buf b; uint64_t n; } views[] = {{a->q, q_bytes}, {a->k_cache, cache_bytes}, {a->v_cache, cache_bytes},
+                                                      {a->k, kv_bytes}, {a->v, kv_bytes}, {a->q_norm, hd * 4},
+                                                      {a->k_norm, hd * 4}, {a->positions, T * 4}};
+    bool apart = hd <= kRmsSerialMaxDim;
+    for (int i = 0; i < 3; i++)  // the first three are written
+        for (int j = i + 1; j < 8; j++) apart = apart && disjoint(views[i].b, views[i].n, views[j].b, views[j].n);
+    if (apart) {
+        StepPrepLaunch sp{};
+        sp.q = q;
+        sp.k = k;
+        sp.v = (const float*)ds5_ptr(a->v);
+        sp.q_norm = (const float*)ds5_ptr(a->q_norm);
+        sp.k_norm = (const float*)ds5_ptr(a->k_norm);
+        sp.positions = (const int32_t*)ds5_ptr(a->positions);
+        sp.k_cache = ds5_ptr(a->k_cache);
+        sp.v_cache = ds5_ptr(a->v_cache);
+        sp.kv_dtype = a->kv_dtype;
+        sp.pos = a->pos;
+        sp.n_tokens = a->n_tokens;
+        sp.n_q_heads = a->n_q_heads;
+        sp.n_kv_heads = a->n_kv_heads;
+        sp.head_dim = a->head_dim;
+        sp.max_ctx = a->max_ctx;
+        sp.eps = a->eps;
+        sp.freq_scale = a->freq_scale;
+        sp.table = table;
+        if (int rc = launch_step_prep(ctx, sp)) return rc;
+        return ds5_hip_gqa_attention(ctx, &at);
+    }
     int rc = launch_rms_norm(ctx, RmsNormLaunch{q, (const float*)ds5_ptr(a->q_norm), q, (uint32_t)(T * hq),
                                                 a->head_dim, a->eps});
     if (!rc) rc = launch_rms_norm(ctx, RmsNormLaunch{k, (const float*)ds5_ptr(a->k_norm), k, (uint32_t)(T * hkv),

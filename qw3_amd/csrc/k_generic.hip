@@ -1,5 +1,5 @@
-// k_generic.hip -- causal GQA attention for every shape the MFMA kernels do
-// not take: f32 caches, head_dim other than 64/128, misaligned views.
+// k_generic.hip -- causal GQA attention for every shape the f16 matrix-core
+// and f32 kernels do not take: head_dim other than 64/128, misaligned views.
 //
 // Semantics are those of kernels_b.zig:29-133: query token t (absolute
 // position pos + t) of q head h attends cache positions 0..pos+t of kv head

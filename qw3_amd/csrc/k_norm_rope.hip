@@ -28,6 +28,50 @@ constexpr int kNormTile = 4096;  // floats of a block's rows staged in LDS
 // reference GPU kernel's reduction order (rms_norm_tree_kernel).
 constexpr uint32_t kSerialMaxDim = kRmsSerialMaxDim;
 
+// The serial sum of a row's squares staged in LDS (16-byte aligned), in element order.
+__device__ __forceinline__ float staged_sumsq(const float* row, uint32_t dim) {
+            float sumsq = 0.0f;
+            // 32 squares per batch in two alternating register sets: a batch's reads are
+            // issued before the previous batch's adds (the scheduling fences keep them
+            // there), so the dependent chain never waits for LDS
+            constexpr int B = 8;  // float4 per batch
+            const uint32_t nb = dim / (4 * B), db = nb * 4 * B;
+            float4 ba[B], bb[B];
+            auto rd = [&](float4(&d)[B], uint32_t batch) {
+    #pragma unroll
+                for (int b = 0; b < B; b++) d[b] = *(const float4*)(row + 4 * B * batch + 4 * b);
+            };
+            auto add = [&](const float4(&d)[B]) {
+    #pragma unroll
+                for (int b = 0; b < B; b++) {
+                    sumsq += d[b].x;
+                    sumsq += d[b].y;
+                    sumsq += d[b].z;
+                    sumsq += d[b].w;
+                }
+            };
+            // pairs of batches, every read unconditional (a read under a branch makes the
+            // compiler's wait at the join count it as outstanding on both paths)
+            const uint32_t np = nb / 2;
+            if (np) rd(ba, 0);
+            for (uint32_t i = 0; i < np; i++) {
+                rd(bb, 2 * i + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                add(ba);
+                __builtin_amdgcn_sched_barrier(0);
+                rd(ba, min(2 * i + 2, 2 * np - 1));
+                __builtin_amdgcn_sched_barrier(0);
+                add(bb);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (nb & 1) {
+                rd(ba, nb - 1);
+                add(ba);
+            }
+            for (uint32_t j = db; j < dim; j++) sumsq += row[j];
+    return sumsq;
+}
+
 // Rows of at most kSerialMaxDim elements: R = min(64, kNormTile / dim) rows per
 // block. The block loads its R rows (contiguous in memory) with every load
 // in flight, and stages each element's square (rounded on its own, as the
@@ -62,45 +106,7 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_rows_kernel(const float
     __syncthreads();
     if (threadIdx.x < nr) {
         const float* row = s_sq + threadIdx.x * stride;
-        float sumsq = 0.0f;
-        // 32 squares per batch in two alternating register sets: a batch's reads are
-        // issued before the previous batch's adds (the scheduling fences keep them
-        // there), so the dependent chain never waits for LDS
-        constexpr int B = 8;  // float4 per batch
-        const uint32_t nb = dim / (4 * B), db = nb * 4 * B;
-        float4 ba[B], bb[B];
-        auto rd = [&](float4(&d)[B], uint32_t batch) {
-#pragma unroll
-            for (int b = 0; b < B; b++) d[b] = *(const float4*)(row + 4 * B * batch + 4 * b);
-        };
-        auto add = [&](const float4(&d)[B]) {
-#pragma unroll
-            for (int b = 0; b < B; b++) {
-                sumsq += d[b].x;
-                sumsq += d[b].y;
-                sumsq += d[b].z;
-                sumsq += d[b].w;
-            }
-        };
-        // pairs of batches, every read unconditional (a read under a branch makes the
-        // compiler's wait at the join count it as outstanding on both paths)
-        const uint32_t np = nb / 2;
-        if (np) rd(ba, 0);
-        for (uint32_t i = 0; i < np; i++) {
-            rd(bb, 2 * i + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            add(ba);
-            __builtin_amdgcn_sched_barrier(0);
-            rd(ba, min(2 * i + 2, 2 * np - 1));
-            __builtin_amdgcn_sched_barrier(0);
-            add(bb);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (nb & 1) {
-            rd(ba, nb - 1);
-            add(ba);
-        }
-        for (uint32_t j = db; j < dim; j++) sumsq += row[j];
+        const float sumsq = staged_sumsq(row, dim);
         s_inv[threadIdx.x] = rms_inv(sumsq, (float)dim, eps);
     }
     __syncthreads();
@@ -220,6 +226,65 @@ __global__ __launch_bounds__(256) void kv_append_kernel(const float* __restrict_
     }
 }
 
+// The step's q and k norms, rotations and the append for shapes without a fused
+// attention kernel, in one launch instead of five (at one token each was 2-5 us of
+// latency): workgroup (token, block of rows_per_block rows), rows 0 .. n_q_heads - 1 the q
+// heads, then the kv heads. As in rms_norm_rows_kernel thread r adds row r's staged squares
+// in element order while the others wait; as in rope_kernel the token's cos / sin are made
+// once. A kv head's workgroup also appends its v row.
+constexpr uint32_t kPrepTile = 2048;  // floats of a block's rows
+constexpr uint32_t kPrepRows = 64;
+
+template <typename T>
+__global__ __launch_bounds__(kNormThreads) void step_prep_kernel(const StepPrepLaunch a, RopeTable table,
+                                                                 uint32_t rows_per_block) {
+    __shared__ __attribute__((aligned(16))) float s_sq[kPrepTile + 4 * kPrepRows];
+    __shared__ float s_x[kPrepTile], s_inv[kPrepRows], s_cos[kSerialMaxDim / 2], s_sin[kSerialMaxDim / 2];
+    const uint32_t dim = a.head_dim, half = dim / 2, t = blockIdx.x, row0 = blockIdx.y * rows_per_block;
+    const uint32_t nr = min(rows_per_block, a.n_q_heads + a.n_kv_heads - row0), n = nr * dim;
+    const float* q = a.q + (uint64_t)t * a.n_q_heads * dim;
+    const float* k = a.k + (uint64_t)t * a.n_kv_heads * dim;
+    const float* v = a.v + (uint64_t)t * a.n_kv_heads * dim;
+    const uint32_t nq = a.n_q_heads * dim;  // elements of the token's q
+    for (uint32_t i = threadIdx.x; i < n; i += kNormThreads) {
+        const uint32_t e = row0 * dim + i;
+        const float x = e < nq ? q[e] : k[e - nq];
+        s_x[i] = x;
+        s_sq[(i / dim) * (dim + 4) + i % dim] = x * x;
+        if (e >= nq) {
+            const uint32_t h = (e - nq) / dim;
+            ((T*)a.v_cache)[((uint64_t)h * a.max_ctx + a.pos + t) * dim + (e - nq) % dim] = to_cache<T>(v[e - nq]);
+        }
+    }
+    const float pos = (float)a.positions[t];
+    for (uint32_t i = threadIdx.x; i < half; i += kNormThreads) {
+        const float angle = pos * a.freq_scale * table.inv[i];
+        s_cos[i] = cosf(angle);
+        s_sin[i] = sinf(angle);
+    }
+    __syncthreads();
+    if (threadIdx.x < nr)
+        s_inv[threadIdx.x] = rms_inv(staged_sumsq(s_sq + threadIdx.x * (dim + 4), dim), (float)dim, a.eps);
+    __syncthreads();
+    for (uint32_t j = threadIdx.x; j < nr * half; j += kNormThreads) {
+        const uint32_t r = j / half, i = j % half, row = row0 + r;
+        const float* w = row < a.n_q_heads ? a.q_norm : a.k_norm;
+        const float inv = s_inv[r], c = s_cos[i], s = s_sin[i];
+        const float x0 = s_x[r * dim + i] * inv * w[i];
+        const float x1 = s_x[r * dim + i + half] * inv * w[i + half];
+        const float y0 = x0 * c - x1 * s, y1 = x0 * s + x1 * c;
+        if (row < a.n_q_heads) {
+            float* o = a.q + ((uint64_t)t * a.n_q_heads + row) * dim;
+            o[i] = y0;
+            o[i + half] = y1;
+        } else {
+            T* o = (T*)a.k_cache + ((uint64_t)(row - a.n_q_heads) * a.max_ctx + a.pos + t) * dim;
+            o[i] = to_cache<T>(y0);
+            o[i + half] = to_cache<T>(y1);
+        }
+    }
+}
+
 inline uint32_t grid_for(uint64_t total, uint32_t block) {
     const uint64_t g = (total + block - 1) / block;
     return (uint32_t)(g > 65535u * 16u ? 65535u * 16u : (g ? g : 1));
@@ -264,4 +329,19 @@ int launch_kv_append(ds5_hip_ctx* ctx, const KvAppendLaunch& a) {
                            a.max_ctx);
     }
     return ds5_after_launch(ctx, "kv_append_kernel");
+}
+
+int launch_step_prep(ds5_hip_ctx* ctx, const StepPrepLaunch& a) {
+    if (a.n_tokens == 0) return DS5_OK;
+    const uint32_t rows = a.n_q_heads + a.n_kv_heads;
+    const uint32_t most = std::max<uint32_t>(1, std::min<uint32_t>(kPrepRows, kPrepTile / a.head_dim));
+    const uint32_t blocks = (rows + most - 1) / most, rpb = (rows + blocks - 1) / blocks;
+    const dim3 grid(a.n_tokens, blocks);
+    if (a.kv_dtype == DS5_DTYPE_F16)
+        DS5_TIMED_LAUNCH(ctx, "step_prep_kernel", step_prep_kernel<f16>, grid, dim3(kNormThreads), 0, ctx->stream, a,
+                         *a.table, rpb);
+    else
+        DS5_TIMED_LAUNCH(ctx, "step_prep_kernel", step_prep_kernel<float>, grid, dim3(kNormThreads), 0, ctx->stream, a,
+                         *a.table, rpb);
+    return ds5_after_launch(ctx, "step_prep_kernel");
 }
