@@ -112,9 +112,10 @@ DS5_HD uint32_t plan_partial(uint32_t len, uint32_t chunk) { return (len == 0 ||
 // matmul_q8_mfma_kernel: block b's direct-to-LDS loads.
 // x: load i of wavefront `wave` fills stage bytes o = 1024 (wave + W i) + 16 lane;
 //    its plane byte offset (block 0) is row min(m0 + r, m - 1), swizzled chunk c.
-// raw q: dword d = min(64 i + lane, 9 * rows - 1) of the wavefront's area is dword
-//    d % 9 of local row d / 9 = tile row 16 wave + (threads / 4) (lr / 16) + lr % 16;
-//    the offsets from the block's scalar base (w + 34 b, or w + 34 b - 2 for odd b).
+// raw q: dword d % 9 of a row's block, counted from the dword boundary at or below it: the
+//    offsets from the block's scalar base (w + 34 b, or w + 34 b - 2 for odd b). The kernel
+//    loads dwords 0..3, 4..7 and 5..8 of each row; gemm_q_dword and gemm_q_row enumerate all
+//    nine of every row of a tile, as the host checks do.
 // ---------------------------------------------------------------------------
 DS5_HD uint32_t gemm_x_tile_row(uint32_t o, uint32_t BM) { return (o % (BM * 64)) / 64; }
 // the offset of tile row r's swizzled chunk in plane row `row`

@@ -16,6 +16,8 @@
 // as many bytes as the weights themselves. Q8_0 blocks are only 2-byte aligned:
 // a lane reads the nine dwords covering its block from the dword boundary below
 // it and realigns the bytes in registers.
+#include <type_traits>
+
 #include "ds5_common.hpp"
 
 namespace {
@@ -227,25 +229,34 @@ __global__ __launch_bounds__(kMmThreads) void matmul_rows_kernel(const float* __
 // matmul_x_split_kernel writes the two planes and the row exponents into the
 // context workspace; matmul_q8_mfma_kernel then only copies x tiles.
 //
-// GEMM workgroup: BM tokens x BN weight rows, WM x WN wavefronts, each with
-// TM x TN tiles of 16 x 16. Per block the workgroup stages x (hi and lo
-// planes), q (as f16) and the BN scales in LDS. The loop is bound by memory
-// latency, not by the matrix cores: every load is issued two blocks before the
-// block is multiplied. x goes HBM/L2 -> LDS with direct-to-LDS loads into a
-// ring of three stages; each thread's 8-byte q run and its row's scale go to
-// registers (three sets) and are converted to f16 into LDS one block ahead.
-// One workgroup barrier per block. The loads are inline asm with explicit
-// vmcnt waits (the compiler's waits would cover the later blocks' loads too).
-// LDS rows are 32 halves (four 16-byte chunks) with chunk c of row r stored at
-// c ^ ((r >> 2) & 3), so a 16-lane group reading one chunk of 16 rows hits 16
-// distinct bank groups.
+// GEMM workgroup: 32 TM tokens x 128 weight rows, four wavefronts, each all the tokens of
+// its own 32 weight rows (v_mfma_f32_32x32x16_f16: two products of 16 k per plane and
+// block), so a weight row is converted to f16 once, in the registers that multiply it.
+// What bounds it: the matrix cores (with random data the card's clock falls to about 1.7
+// GHz under them), then the memory pipe of the CU, which takes 64 B a cycle: a block's 22
+// KB (x planes and raw q) are 344 of its 512 matrix-core cycles. So every load is
+// direct-to-LDS (inline asm with explicit vmcnt waits: the compiler's would cover the later
+// blocks' loads too) and is issued between two products: issued together after the barrier
+// the six took 390 cycles in which no product ran. x comes two blocks ahead into a ring of
+// three stages, q three; one workgroup barrier per block. A 128-row tile takes 1160 cycles
+// per block alone on a CU and 1740 beside a second one. Against the previous kernel (16 x 16
+// tiles of 8 wavefronts, q converted through LDS by all of them, loads issued together):
+// m 203, n 9216, k 4096: 112 -> 72 us; m 500, n 5120, k 2048: 60 -> 43 us; 2048 tokens:
+// 138 -> 133 us, and 150 -> 128 us with the attention epilogue.
 //
-// MFMA operand layout (16x16x32): lane l supplies row / column l % 16 and the
-// eight k of chunk l / 16; result element (4 (l / 16) + i, l % 16) is in
-// register i of lane l.
+// LDS: x rows are 32 halves (four 16-byte chunks) with chunk c of row r stored at
+// c ^ ((r >> 2) & 3): the 32-row operand reads run at 220 of the 256 B a cycle (measured;
+// 16-row reads of the same layout reach half of it).
+//
+// MFMA operand layout (32x32x16): lane l supplies row / column l % 32 and eight k of half
+// l / 32; which k does not matter as long as x and q agree: half h takes elements
+// 16 h + 8 j + [0, 8) of the block in product j, so a lane's q are 16 consecutive bytes.
+// Result element (8 (i / 4) + 4 (l / 32) + i % 4, l % 32) is in register i of lane l.
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+
+constexpr int kGemmThreads = 256;  // 4 wavefronts, 32 weight rows each
+constexpr int kGemmCols = 128;
 
 constexpr int kSplitThreads = 256;
 constexpr int kXExpBias = 14;  // scaled rows have max |x'| in [2^14, 2^15)
@@ -501,13 +512,13 @@ struct MoeGemmTiles {
     const uint32_t* out_rows;
 };
 
-template <int BM, int BN, int WM, int WN, int EPI, bool GRP = false>
-__global__ __launch_bounds__(WM * WN * 64) void matmul_q8_mfma_kernel(const uint16_t* __restrict__ xhi,
-                                                                      const uint16_t* __restrict__ xlo,
-                                                                      const int* __restrict__ row_exp,
-                                                                      const WeightGroup g, uint32_t m, uint32_t k,
-                                                                      const AttnPrepEpi ep,
-                                                                      const MoeGemmTiles mt) {
+template <int TM, int EPI, bool GRP = false>
+__global__ __launch_bounds__(kGemmThreads, 2) void matmul_q8_mfma_kernel(const uint16_t* __restrict__ xhi,
+                                                                         const uint16_t* __restrict__ xlo,
+                                                                         const int* __restrict__ row_exp,
+                                                                         const WeightGroup g, uint32_t m, uint32_t k,
+                                                                         const AttnPrepEpi ep, const MoeGemmTiles mt) {
+    constexpr int BM = 32 * TM, BN = kGemmCols, W = kGemmThreads / 64;
     asm volatile("" ::DS5_GROUP_ARGS(g), "s"(xhi), "s"(xlo), "s"(row_exp), "s"(m), "s"(k));
     // this workgroup's entry and column tile (uniform); out may be the residual itself
     // Workgroup L = y * gridDim.x + x runs on XCD L % 8. With gridDim.y a multiple of 8
@@ -544,59 +555,34 @@ __global__ __launch_bounds__(WM * WN * 64) void matmul_q8_mfma_kernel(const uint
         m = te.y;
         w += (uint64_t)te.z * mt.w_stride;
     }
-    constexpr int kThreads = WM * WN * 64;
-    constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
-    static_assert(TM * WM * 16 == BM && TN * WN * 16 == BN, "tile split");
-    constexpr int kBPer = BN * 4 / kThreads;  // 8-byte q runs per thread and block
-    static_assert(kBPer >= 1, "at least one q run per thread");
 
-    // LDS: As [stage][hi, lo][row * 4 + swizzled chunk], raw q [stage][wavefront][rows of
-    // 9 dwords], Bs [buffer][row * 4 + swizzled chunk], Ss [buffer][row]; EPI 1 reuses
-    // the bytes for the f32 tile
-    constexpr int kRawBytes = 2 * WM * WN * ((16 * (BN * 4 / (WM * WN * 64)) * 9 + 63) / 64) * 256;
-    constexpr int kAsBytes = 3 * 2 * BM * 4 * 16, kBsBytes = 2 * BN * 4 * 16, kSsBytes = 2 * BN * 4;
-    constexpr int kMainBytes = kAsBytes + kRawBytes + kBsBytes + kSsBytes;
-    constexpr int kTileRow = BN + 4;  // EPI 1 tile row stride in floats (16-byte rows, rows 4 banks apart)
-    constexpr int kLdsBytes = EPI == 1 && BM * kTileRow * 4 > kMainBytes ? BM * kTileRow * 4 : kMainBytes;
+    // LDS: rings of three x stages [hi, lo][row * 4 + swizzled chunk] and three raw q stages
+    // of 2 KB per wavefront; EPI 1 reuses the bytes for a head's f32 tile
+    constexpr int kX = 2 * BM * 64, kStages = 3, kQ = 2048, kQ0 = kStages * kX;
+    constexpr int kMain = kQ0 + kStages * W * kQ;
+    constexpr int kTileRow = 128 + 4;  // EPI 1 tile row stride in floats (16-byte rows, rows 4 banks apart)
+    constexpr int kLdsBytes = EPI == 1 && BM * kTileRow * 4 > kMain ? BM * kTileRow * 4 : kMain;
     __shared__ __attribute__((aligned(16))) unsigned char smem[kLdsBytes];
-    auto& As = *reinterpret_cast<u32x4_t(*)[3][2][BM * 4]>(smem);
-    auto& Bs = *reinterpret_cast<u32x4_t(*)[2][BN * 4]>(smem + kAsBytes + kRawBytes);
-    auto& Ss = *reinterpret_cast<float(*)[2][BN]>(smem + kAsBytes + kRawBytes + kBsBytes);
+    // the tile rows' power-of-two shifts and (GRP) output rows, for the epilogue: read there
+    // from memory one by one they cost as much as the products (64 dependent loads a lane)
+    __shared__ __attribute__((aligned(16))) int s_sh[BM];
+    __shared__ __attribute__((aligned(16))) uint32_t s_orow[GRP ? BM : 4];
 
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const uint32_t n0 = tile * BN;
+    const int lane = threadIdx.x & 63, r32 = lane & 31, h = lane >> 5;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t n0 = tile * BN, col = 32 * wave + r32;
     const uint32_t nb = k / 32;
-    const uint64_t row_bytes = (uint64_t)nb * kQ8Bytes;
-
-    // ---- staging ------------------------------------------------------------------
-    // All global loads are direct-to-LDS, issued two blocks ahead and awaited
-    // explicitly. Iteration b issues x and the raw q of block b + 2 (one group of
-    // loads), multiplies block b, waits until only that group is outstanding
-    // (block b + 1 has landed), converts block b + 1's raw q to f16 and meets
-    // the barrier. Each wavefront loads the raw rows its own threads convert, so
-    // the conversion needs only the wavefront's own wait. Block j uses x stage
-    // j % 3, raw q stage j % 2 and f16 q buffer j % 2.
-    constexpr int kXStage = 2 * BM * 64;  // bytes: hi plane rows, then lo plane rows
-    constexpr int kRowDw = 9;             // raw q row: the 9 dwords covering a 34-byte block
-    constexpr int W = WM * WN;
-    constexpr int NX = kXStage / 1024 / W;  // x loads per wavefront and block
-    static_assert(NX >= 1 && NX * 1024 * W == kXStage, "whole 1 KB x loads per wavefront");
-    static_assert((BM * 64) % 1024 == 0, "an x load stays inside one plane");
-    constexpr int kWRows = 16 * kBPer;                   // tile rows whose runs a wavefront converts
-    constexpr int NQ = (kWRows * kRowDw + 63) / 64;      // raw q loads (256 bytes) per wavefront and block
-    constexpr int kQWave = NQ * 256;                     // a wavefront's raw q area in a stage
-    constexpr int kQStage = W * kQWave;
-    constexpr int kVmPerBlock = NX + NQ;
-    const uint32_t wave_u = (uint32_t)__builtin_amdgcn_readfirstlane(wave);
+    const uint32_t row_bytes = nb * kQ8Bytes;  // below 2^31: the launchers' 32-bit offsets
     const uint32_t smem_lds = gemm_lds_addr(smem);
 
-    // x: load i of this wavefront fills stage bytes [1024 (wave + W i), +1024), lane L
+    // x: load i of this wavefront fills bytes [1024 (wave + W i), +1024) of a stage, lane L
     // the 16 bytes at +16 L: plane, row r, slot L % 4 holding chunk (L % 4) ^ ((r >> 2) & 3).
+    constexpr int NX = kX / 1024 / W;
+    static_assert(NX >= 1 && NX * 1024 * W == kX && (BM * 64) % 1024 == 0, "whole 1 KB x loads inside one plane");
     uint32_t xoff[NX];  // byte offset in the plane: row min(m0 + r, m - 1), chunk c, block 0
 #pragma unroll
     for (int i = 0; i < NX; i++) {
-        const uint32_t o = 1024u * (wave_u + W * i) + 16u * lane;
+        const uint32_t o = 1024u * (wave + W * i) + 16u * lane;
         if (GRP && mt.x_rows) {  // uniform
             const uint32_t r = ds5idx::gemm_x_tile_row(o, BM);
             xoff[i] = ds5idx::gemm_x_off_row(r, (uint32_t)lane, mt.x_rows[min(m0 + r, m - 1)], k);
@@ -604,256 +590,322 @@ __global__ __launch_bounds__(WM * WN * 64) void matmul_q8_mfma_kernel(const uint
             xoff[i] = ds5idx::gemm_x_off(o, (uint32_t)lane, BM, m0, m, k);
         }
     }
-    auto issue_x = [&](uint32_t b, int stage) {
-#pragma unroll
-        for (int i = 0; i < NX; i++) {
-            const uint32_t blk = wave_u + W * i;  // uniform
-            const uint16_t* plane = blk * 1024 < BM * 64 ? xhi : xlo;
-            lds_dma<4>(xoff[i], uniform_u64((uint64_t)(uintptr_t)plane + 64ull * b),
-                       (uint32_t)__builtin_amdgcn_readfirstlane(smem_lds + stage * kXStage + 1024 * blk));
-        }
+    auto issue_x = [&](uint32_t b, uint32_t stage, int i) {
+        const uint32_t blk = wave + W * i;  // uniform
+        const uint16_t* plane = blk * 1024 < BM * 64 ? xhi : xlo;
+        lds_dma<4>(xoff[i], uniform_u64((uint64_t)(uintptr_t)plane + 64ull * b),
+                   (uint32_t)__builtin_amdgcn_readfirstlane(smem_lds + stage * kX + 1024 * blk));
     };
-
-    // raw q: the wavefront's local row lr < 16 kBPer is tile row 16 wave + (threads / 4)
-    // (lr / 16) + lr % 16 (the rows of its threads' runs). Dword d = 64 i + lane of its
-    // area (clamped to the last, d < 9 * 16 kBPer) is dword d % 9 of local row d / 9, from
-    // the dword boundary at or below the row's block: weight row wr = min(n0 + row,
-    // n - 1), rb = wr * row_bytes, block b at byte rb + 34 b of the weights. 34 b is
-    // 0 mod 4 for even b and 2 mod 4 for odd b, so the dwords start at 34 b + (rb & ~3)
-    // (even) or 34 b - 2 + ((rb + 2) & ~3) (odd): scalar base w + 34 b or w + 34 b - 2,
-    // lane offsets per parity (both sums of non-negative terms: no unsigned wrap).
-    uint32_t qoff_e[NQ], qoff_o[NQ];
+    // raw q: row r of the wavefront's 32 takes 48 bytes, three 16-byte lanes with dwords
+    // 0..3, 4..7 and 5..8 of the nine from the dword boundary at or below its block: 96
+    // lanes of two loads (the others repeat the last, into the area's padding). 34 b is 0 mod 4 for even b and 2 mod 4 for odd b:
+    // scalar base w + 34 b or w + 34 b - 2, lane offsets per parity.
+    uint32_t qe[2], qo[2];
 #pragma unroll
-    for (int i = 0; i < NQ; i++) {
-        const uint32_t d = ds5idx::gemm_q_dword(i, (uint32_t)lane, kWRows, kRowDw);
-        const uint32_t row = ds5idx::gemm_q_row(d, wave_u, kThreads, kRowDw);
-        ds5idx::gemm_q_off(d, row, n0, n, (uint32_t)row_bytes, kRowDw, qoff_e[i], qoff_o[i]);
+    for (int i = 0; i < 2; i++) {
+        const uint32_t u = min(64u * i + lane, 95u), part = u % 3;
+        ds5idx::gemm_q_off(part == 0 ? 0u : part + 3u, 32 * wave + u / 3, n0, n, row_bytes, 9, qe[i], qo[i]);
     }
-    const uint32_t q_lds = smem_lds + 3 * kXStage + wave_u * kQWave;
-    auto issue_q = [&](uint32_t b, int stage) {
+    auto issue_q = [&](uint32_t b, uint32_t slot, int i) {
         const bool odd = b & 1;
         const uint64_t base = uniform_u64((uint64_t)(uintptr_t)w + (uint64_t)kQ8Bytes * b - (odd ? 2u : 0u));
-#pragma unroll
-        for (int i = 0; i < NQ; i++)
-            lds_dma<1>(odd ? qoff_o[i] : qoff_e[i], base,
-                       (uint32_t)__builtin_amdgcn_readfirstlane(q_lds + stage * kQStage + 256 * i));
+        const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane(smem_lds + kQ0 + (slot * W + wave) * kQ);
+        lds_dma<4>(odd ? qo[i] : qe[i], base, at + 1024 * i);
     };
+    constexpr int kVmPerBlock = NX + 2;
 
-    // f16 q: thread c = tid + threads u takes tile row c / 4 (local row 16 u + lane / 4 of
-    // its wavefront), bytes 2 + 8 (c % 4) .. + 8 of its block: raw-row bytes (s & 3) + 2
-    // + 8 (c % 4) .. + 8, inside the three dwords 2 (c % 4) .. + 3 of the raw row (bytes
-    // 2..9 of them when s & 3 = 0, bytes 4..11 when it is 2). Part 0's first dword also
-    // holds the scale (bytes s & 3, + 1).
-    const unsigned char* qraw = smem + 3 * kXStage + wave_u * kQWave;
-    uint32_t rbp[kBPer], qrd[kBPer];  // (weight row * row_bytes) & 3; byte of the lane's dwords in the area
-#pragma unroll
-    for (int u = 0; u < kBPer; u++) {
-        const uint32_t c = threadIdx.x + kThreads * u;
-        rbp[u] = (min(n0 + (c >> 2), n - 1) * (uint32_t)row_bytes) & 3u;
-        qrd[u] = (16 * u + (lane >> 2)) * (kRowDw * 4) + 8 * (lane & 3);
-    }
-    auto convert_q = [&](uint32_t b, int stage, int buf) {
-#pragma unroll
-        for (int u = 0; u < kBPer; u++) {
-            const uint32_t c = threadIdx.x + kThreads * u;
-            const uint32_t row = c >> 2, part = c & 3;
-            const bool s2 = (rbp[u] + 2 * b) & 2u;  // s & 3 == 2
-            const uint32_t* rw = (const uint32_t*)(qraw + stage * kQStage + qrd[u]);
-            const uint32_t d0 = rw[0], d1 = rw[1], d2 = rw[2];
-            const uint32_t sel = s2 ? 0x07060504u : 0x05040302u;
-            const uint2 a = i8x4_to_f16x4(__builtin_amdgcn_perm(d1, d0, sel));
-            const uint2 bb = i8x4_to_f16x4(__builtin_amdgcn_perm(d2, d1, sel));
-            Bs[buf][row * 4 + (part ^ ((row >> 2) & 3))] = u32x4_t{a.x, a.y, bb.x, bb.y};
-            if (part == 0) Ss[buf][row] = f16_bits_to_f32(s2 ? d0 >> 16 : d0 & 0xffffu);
+    // q operand: lane (r32, h) takes bytes 16 h .. 16 h + 15 of its column's block (dwords
+    // 4 h .. 4 h + 4), converted to f16; the scale is in the h = 0 lanes' first dword.
+    const bool s2 = (min(n0 + col, n - 1) * row_bytes) & 2u;  // even blocks start 2 mod 4
+    struct QRaw {
+        u32x4_t d;
+        uint32_t d4;
+    };
+    auto q_raw = [&](uint32_t slot) {
+        const unsigned char* row = smem + kQ0 + (slot * W + wave) * kQ + 48 * r32;
+        return QRaw{*(const u32x4_t*)(row + 16 * h), *(const uint32_t*)(row + (h ? 44 : 16))};
+    };
+    // part p < 4: four elements; part 4: the scale, from the h = 0 half to both
+    auto q_part = [&](f16x8_t& q0, f16x8_t& q1, float& scale, const QRaw& r, bool at2, int p) {
+        if (p < 4) {
+            const uint2 v = i8x4_to_f16x4(__builtin_amdgcn_perm(p < 3 ? r.d[p < 3 ? p + 1 : 3] : r.d4, r.d[p],
+                                                                at2 ? 0x07060504u : 0x05040302u));
+            u32x4_t w4 = __builtin_bit_cast(u32x4_t, p < 2 ? q0 : q1);
+            w4[2 * (p & 1)] = v.x;
+            w4[2 * (p & 1) + 1] = v.y;
+            (p < 2 ? q0 : q1) = __builtin_bit_cast(f16x8_t, w4);
+        } else {
+            const uint32_t sb = at2 ? r.d[0] >> 16 : r.d[0] & 0xffffu;
+            scale = f16_bits_to_f32(__builtin_amdgcn_permlane32_swap(sb, sb, false, false)[0]);
         }
     };
 
-    // ---- per-wavefront tiles ---------------------------------------------------
-    const int wm0 = (wave / WN) * (BM / WM), wn0 = (wave % WN) * (BN / WN);
-    const int r16 = lane & 15, grp = lane >> 4;
-    f32x4_t acc[TM][TN];
+    if (threadIdx.x < BM) {
+        const uint32_t row = min(m0 + threadIdx.x, m - 1);
+        s_sh[threadIdx.x] = row_exp[GRP && mt.x_rows ? mt.x_rows[row] : row] - kXExpBias;
+        if constexpr (GRP) s_orow[threadIdx.x] = mt.out_rows ? mt.out_rows[row] : row;
+    }
+    static_assert(BM <= kGemmThreads, "a thread per tile row");
+
+    f32x16 acc[TM];
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int e = 0; e < 16; e++) acc[i][e] = 0.0f;
 
-    // GRP: the wavefront's 16-row tiles holding rows of the tile (uniform); the rest
-    // (an expert's last, partial tile) skip their products
-    int live = TM;
-    if constexpr (GRP) {
-        const int left = (int)m - (int)(m0 + wm0);
-        live = __builtin_amdgcn_readfirstlane(left <= 0 ? 0 : min(TM, (left + 15) / 16));
-    }
-    auto multiply = [&](int stage, int buf) {
-        f16x8_t bv[TN];
-        float sv[TN];
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int row = wn0 + 16 * j + r16;
-            bv[j] = __builtin_bit_cast(f16x8_t, Bs[buf][row * 4 + (grp ^ ((row >> 2) & 3))]);
-            sv[j] = Ss[buf][row];
-        }
-#pragma unroll
-        for (int i = 0; i < TM; i++) {
-            if (GRP && i >= live) break;
-            const int row = wm0 + 16 * i + r16;
-            const int slot = row * 4 + (grp ^ ((row >> 2) & 3));
-            const f16x8_t ah = __builtin_bit_cast(f16x8_t, As[stage][0][slot]);
-            const f16x8_t al = __builtin_bit_cast(f16x8_t, As[stage][1][slot]);
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                f32x4_t t = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bv[j], f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-                t = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bv[j], t, 0, 0, 0);
-#pragma unroll
-                for (int e = 0; e < 4; e++) acc[i][j][e] = __builtin_fmaf(sv[j], t[e], acc[i][j][e]);
-            }
-        }
+    // x operand of row subtile i, half j of the block: chunk 2 h + j of row 32 i + r32
+    const uint32_t swz = (r32 >> 2) & 3;
+    auto x_op = [&](const unsigned char* st, int plane, int i, int j) {
+        return *(const f16x8_t*)(st + plane * BM * 64 + i * 2048 + r32 * 64 + ((2 * h + j) ^ swz) * 16);
     };
-
-    // prologue: blocks 0 and 1 in flight; block 0's q converted once its loads have landed
-    issue_x(0, 0);
-    issue_q(0, 0);
-    if (nb > 1) {
-        issue_x(1, 1);
-        issue_q(1, 1);
-        wait_vm_only<kVmPerBlock>();
-    } else {
-        wait_vm_only<0>();
-    }
-    convert_q(0, 0, 0);
-    gemm_lds_sync();
-    // iteration b: x stage b % 3 (uniform)
-    uint32_t st = 0;
-    for (uint32_t b = 0; b < nb; b++) {
-        const uint32_t st1 = st == 2 ? 0 : st + 1, st2 = st == 0 ? 2 : st - 1;  // (b + 1) % 3, (b + 2) % 3
-        const bool ahead = b + 2 < nb;  // uniform
-        if (ahead) {
-            issue_x(b + 2, st2);  // the stage of block b - 1, read before the last barrier
-            issue_q(b + 2, b & 1);  // the raw stage of block b, converted before the last barrier
+    // Iteration b: wait until only what the last iteration asked for is outstanding (block
+    // b + 1's x, block b + 2's q), meet (block b's x is in LDS for everyone, and everyone is
+    // done with block b - 1, whose stage block b + 2's x takes), ask for block b + 2's x and
+    // block b + 3's q, multiply block b, convert block b + 1's q (the wavefront's own loads:
+    // its own wait covers them) beside it.
+    //
+    // Within the block the products run in pairs of subtiles, two chains of four (lo, lo,
+    // hi, hi) in turn. A slot is one product, the x operand read kAhead products early, and
+    // four of the previous pair's scale multiply-adds (across blocks too): a wavefront keeps
+    // the matrix core and the VALU busy by itself, the scheduling fences hold the order.
+    constexpr int kAhead = 6;
+    // Past the end the last block is asked for again, so that every iteration has the same
+    // loads outstanding; the loop ends on a full wait.
+    const uint32_t bl = nb - 1;
+    auto issue = [&](uint32_t b, uint32_t stage, uint32_t bq, uint32_t slot, int n) {
+        if (n < NX) issue_x(b, stage, n);
+        else if (n < NX + 2) issue_q(bq, slot, n - NX);
+    };
+#pragma unroll
+    for (int n = 0; n < NX + 2; n++) issue(0, 0, 0, 0, n);
+    issue_q(min(1u, bl), 1, 0);
+    issue_q(min(1u, bl), 1, 1);
+#pragma unroll
+    for (int n = 0; n < NX + 2; n++) issue(min(1u, bl), 1, min(2u, bl), 2, n);
+    auto loop = [&](auto pairs) {
+        constexpr int NP = decltype(pairs)::value, NS = 8 * NP;
+        f32x16 t[2][2];  // [parity of the pair][subtile]
+        float ps = 0.0f;
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) t[u / 2][u % 2][e] = 0.0f;
+        f16x8_t q0 = {}, q1 = {};
+        float sb = 0.0f;
+        {
+            wait_vm_only<kVmPerBlock>();
+            const QRaw r = q_raw(0);
+#pragma unroll
+            for (int p = 0; p < 5; p++) q_part(q0, q1, sb, r, s2, p);
         }
-        multiply(st, b & 1);
-        if (ahead) wait_vm_only<kVmPerBlock>();  // block b + 1 has landed
-        else wait_vm_only<0>();
-        if (b + 1 < nb) convert_q(b + 1, (b + 1) & 1, (b + 1) & 1);
-        gemm_lds_sync();
-        st = st1;
+        uint32_t st = 0;
+        auto block = [&](uint32_t b, auto par) {
+            constexpr int P0 = decltype(par)::value;
+            wait_vm_only<kVmPerBlock>();
+            gemm_lds_sync();
+            const unsigned char* at = smem + st * kX;
+            const uint32_t st0 = st, st2 = st == 0 ? 2 : st - 1;  // b % 3, (b + 2) % 3
+            st = st == 2 ? 0 : st + 1;
+            f16x8_t xr[NS];
+            auto read = [&](int n) {
+                const int p = n / 8, s = n % 8 / 2, u = n % 2;
+                xr[n] = x_op(at, s < 2 ? 1 : 0, 2 * p + u, s & 1);
+            };
+#pragma unroll
+            for (int n = 0; n < kAhead; n++) read(n);
+            const bool at2 = s2 != (bool)((b + 1) & 1);
+            const QRaw nx = q_raw(st);
+            f16x8_t n0q = q0, n1q = q1;
+            float ns = sb;
+            __builtin_amdgcn_sched_barrier(0);
+            static_assert(NS >= kVmPerBlock, "a slot for every load");
+#pragma unroll
+            for (int n = 0; n < NS; n++) {
+                const int p = n / 8, q = n % 8, s = q / 2, u = q % 2, cur = (P0 + p) & 1, pp = p == 0 ? NP - 1 : p - 1;
+                if (n + kAhead < NS) read(n + kAhead);
+                // one load per product or two: a load holds the wavefront's issue for as
+                // long as the memory pipe needs for it (64 B a cycle and CU), which only
+                // products in flight cover
+                if constexpr (NS >= 2 * kVmPerBlock) {
+                    if (n % 2 == 1) issue(min(b + 2, bl), st2, min(b + 3, bl), st0, n / 2);
+                } else {
+                    issue(min(b + 2, bl), st2, min(b + 3, bl), st0, n);
+                }
+                if (s == 0) {
+                    f32x16 z;
+#pragma unroll
+                    for (int e = 0; e < 16; e++) z[e] = 0.0f;
+                    t[cur][u] = mfma_32x32x16(xr[n], q0, z);
+                } else {
+                    t[cur][u] = mfma_32x32x16(xr[n], s & 1 ? q1 : q0, t[cur][u]);
+                }
+                const float sc = p == 0 ? ps : sb;
+#pragma unroll
+                for (int e = 4 * (q % 4); e < 4 * (q % 4) + 4; e++)
+{
+                    float v = __builtin_fmaf(sc, t[cur ^ 1][q / 4][e], acc[2 * pp + q / 4][e]);
+                    asm volatile("" : "+v"(v));  // here, not sunk into a later block
+                    acc[2 * pp + q / 4][e] = v;
+                }
+                if (p == NP - 1 && q < 5) q_part(n0q, n1q, ns, nx, at2, q);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            ps = sb;
+            q0 = n0q;
+            q1 = n1q;
+            sb = ns;
+        };
+        auto last = [&](auto par) {  // the last pair's sums
+            constexpr int C = decltype(par)::value;
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int e = 0; e < 16; e++)
+                    acc[2 * NP - 2 + u][e] = __builtin_fmaf(ps, t[C][u][e], acc[2 * NP - 2 + u][e]);
+        };
+        uint32_t b = 0;
+        for (; b + 2 <= nb; b += 2) {
+            block(b, std::integral_constant<int, 0>{});
+            block(b + 1, std::integral_constant<int, NP & 1>{});
+        }
+        if (b < nb) {
+            block(b, std::integral_constant<int, 0>{});
+            last(std::integral_constant<int, (NP - 1) & 1>{});
+        } else {
+            last(std::integral_constant<int, ((NP & 1) + NP - 1) & 1>{});
+        }
+        wait_vm_only<0>();  // the repeated loads, before their LDS is used or given up
+    };
+    // pairs of 32-row subtiles that hold rows (uniform); the others skip their products
+    const uint32_t live = (uint32_t)__builtin_amdgcn_readfirstlane((int)((m - m0 + 63) / 64));
+    if constexpr (TM > 2) {
+        if (live >= TM / 2) loop(std::integral_constant<int, TM / 2>{});
+        else loop(std::integral_constant<int, 1>{});
+        static_assert(TM <= 4, "one partial form");
+    } else {
+        loop(std::integral_constant<int, 1>{});
     }
 
     if constexpr (EPI == 1) {
-        // The whole 128 x 128 tile (one head of 128 tokens) goes through LDS once;
-        // then thread t takes rows t / 8 and t / 8 + 64, dims k8 + [0, 8) and
-        // 64 + k8 + [0, 8) (8 rope pairs), k8 = 8 (t % 8). Its norm weights and
-        // rope cos / sin are loaded before the tile is written, so their
-        // latency overlaps the tile's LDS round trip.
-        static_assert(BM == 128 && BN == 128 && WM == 4 && WN == 2, "one head of 128 dims per tile");
-        constexpr int D = 128, HALF = 64, TROW = kTileRow;
-        const uint32_t head = tile;  // BN = D: tile j of an entry is head j
+        // One head (128 columns, four wavefronts) at a time goes through LDS; then thread t
+        // takes row t / 8 (+ 64, ...), dims k8 + [0, 8) and 64 + k8 + [0, 8) (8 rope
+        // pairs), k8 = 8 (t % 8).
+        constexpr int D = 128, HALF = 64, TROW = kTileRow, kRowsPer = kGemmThreads / 8;
         const int r0 = threadIdx.x / 8, k8 = 8 * (threadIdx.x % 8);
         const float* nw = entry == 0 ? ep.q_norm : ep.k_norm;
-        float w0[8], w1[8], c[2][8], sn[2][8];
+        float w0[8], w1[8];
         if (entry != 2) {
             *(float4*)&w0[0] = *(const float4*)(nw + k8);
             *(float4*)&w0[4] = *(const float4*)(nw + k8 + 4);
             *(float4*)&w1[0] = *(const float4*)(nw + HALF + k8);
             *(float4*)&w1[4] = *(const float4*)(nw + HALF + k8 + 4);
-#pragma unroll
-            for (int rr = 0; rr < 2; rr++) {
-                const uint32_t tok = min(m0 + r0 + 64 * rr, m - 1);
-                const float* cs = ep.cs + (uint64_t)tok * D;
-                *(float4*)&c[rr][0] = *(const float4*)(cs + k8);
-                *(float4*)&c[rr][4] = *(const float4*)(cs + k8 + 4);
-                *(float4*)&sn[rr][0] = *(const float4*)(cs + HALF + k8);
-                *(float4*)&sn[rr][4] = *(const float4*)(cs + HALF + k8 + 4);
-            }
         }
-        // the main loop ended on a barrier after every wavefront's last LDS read
         float* tl = reinterpret_cast<float*>(smem);
+#pragma unroll 1
+        for (uint32_t hd = 0; hd < BN / D && n0 + D * hd < n; hd++) {  // uniform
+            const uint32_t head = tile * (BN / D) + hd;
+            __syncthreads();  // every wavefront's last read of the bytes
+            if (wave / 4 == hd) {
 #pragma unroll
-        for (int i = 0; i < TM; i++)
+                for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int lr = wm0 + 16 * i + 4 * grp + e;
-                const uint32_t row = m0 + lr;
-                const int sh = row < m ? row_exp[row] - kXExpBias : 0;
-#pragma unroll
-                for (int j = 0; j < TN; j++) tl[lr * TROW + wn0 + 16 * j + r16] = __builtin_ldexpf(acc[i][j][e], sh);
+                    for (int e = 0; e < 16; e++) {
+                        const int lr = 32 * i + 8 * (e / 4) + 4 * h + e % 4;
+                        tl[lr * TROW + (col & 127)] = __builtin_ldexpf(acc[i][e], s_sh[lr]);
+                    }
             }
-        __syncthreads();
-#pragma unroll
-        for (int rr = 0; rr < 2; rr++) {
-            const int r = r0 + 64 * rr;
-            const uint32_t tok = m0 + r;
-            const bool ok = tok < m;
-            const float* trow = tl + r * TROW;
-            float x0[8], x1[8];
-            *(float4*)&x0[0] = *(const float4*)(trow + k8);
-            *(float4*)&x0[4] = *(const float4*)(trow + k8 + 4);
-            *(float4*)&x1[0] = *(const float4*)(trow + HALF + k8);
-            *(float4*)&x1[4] = *(const float4*)(trow + HALF + k8 + 4);
-            f16x8_t y0v, y1v;
-            f16* dst;
-            if (entry == 2) {  // v: f16 append
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    y0v[j] = (f16)x0[j];
-                    y1v[j] = (f16)x1[j];
+            __syncthreads();
+#pragma unroll 1
+            for (int r = r0; r < BM; r += kRowsPer) {
+                const uint32_t tok = m0 + r;
+                if (m0 + (r - r0) >= m) break;  // uniform: no rows left
+                const bool ok = tok < m;
+                const float* trow = tl + r * TROW;
+                float x0[8], x1[8], c[8], sn[8];
+                if (entry != 2) {
+                    const float* cs = ep.cs + (uint64_t)min(tok, m - 1) * D;
+                    *(float4*)&c[0] = *(const float4*)(cs + k8);
+                    *(float4*)&c[4] = *(const float4*)(cs + k8 + 4);
+                    *(float4*)&sn[0] = *(const float4*)(cs + HALF + k8);
+                    *(float4*)&sn[4] = *(const float4*)(cs + HALF + k8 + 4);
                 }
-                dst = ep.v_cache + ((uint64_t)head * ep.max_ctx + ep.pos + tok) * D;
-            } else {
-                if (entry == 0) {
-                    // q: the thread's two quarters (pairs k8 .. k8 + 3 and k8 + 4 .. k8 + 7),
-                    // then the head's 8 threads in the balanced tree's order (xor 1, 2, 4)
-                    float ss = qk_quarter_sumsq(x0[0], x1[0], x0[1], x1[1], x0[2], x1[2], x0[3], x1[3]) +
-                               qk_quarter_sumsq(x0[4], x1[4], x0[5], x1[5], x0[6], x1[6], x0[7], x1[7]);
-#pragma unroll
-                    for (int mm = 1; mm < 8; mm <<= 1) ss += __shfl_xor(ss, mm, 64);
-                    const float r = rms_inv(ss, (float)D, ep.eps) * ep.q_scale;
+                *(float4*)&x0[0] = *(const float4*)(trow + k8);
+                *(float4*)&x0[4] = *(const float4*)(trow + k8 + 4);
+                *(float4*)&x1[0] = *(const float4*)(trow + HALF + k8);
+                *(float4*)&x1[4] = *(const float4*)(trow + HALF + k8 + 4);
+                f16x8_t y0v, y1v;
+                f16* dst;
+                if (entry == 2) {  // v: f16 append
 #pragma unroll
                     for (int j = 0; j < 8; j++) {
-                        _Float16 o0, o1;
-                        qk_q_pair(x0[j], x1[j], w0[j], w1[j], c[rr][j], sn[rr][j], r, o0, o1);
-                        y0v[j] = o0;
-                        y1v[j] = o1;
+                        y0v[j] = (f16)x0[j];
+                        y1v[j] = (f16)x1[j];
                     }
-                } else {  // k: the reference's serial sum of the row
-                    const float inv = rms_inv(qk_serial_sumsq(trow, D), (float)D, ep.eps);
+                    dst = ep.v_cache + ((uint64_t)head * ep.max_ctx + ep.pos + tok) * D;
+                } else {
+                    if (entry == 0) {
+                        // q: the thread's two quarters (pairs k8 .. k8 + 3 and k8 + 4 .. k8 + 7),
+                        // then the head's 8 threads in the balanced tree's order (xor 1, 2, 4)
+                        float ss = qk_quarter_sumsq(x0[0], x1[0], x0[1], x1[1], x0[2], x1[2], x0[3], x1[3]) +
+                                   qk_quarter_sumsq(x0[4], x1[4], x0[5], x1[5], x0[6], x1[6], x0[7], x1[7]);
 #pragma unroll
-                    for (int j = 0; j < 8; j++) {
-                        float y0, y1;
-                        qk_rotate(qk_norm_mul(x0[j], inv, w0[j]), qk_norm_mul(x1[j], inv, w1[j]), c[rr][j], sn[rr][j],
-                                  y0, y1);
-                        y0v[j] = (f16)y0;
-                        y1v[j] = (f16)y1;
+                        for (int mm = 1; mm < 8; mm <<= 1) ss += __shfl_xor(ss, mm, 64);
+                        const float r1 = rms_inv(ss, (float)D, ep.eps) * ep.q_scale;
+#pragma unroll
+                        for (int j = 0; j < 8; j++) {
+                            _Float16 o0, o1;
+                            qk_q_pair(x0[j], x1[j], w0[j], w1[j], c[j], sn[j], r1, o0, o1);
+                            y0v[j] = o0;
+                            y1v[j] = o1;
+                        }
+                    } else {  // k: the reference's serial sum of the row
+                        const float inv = rms_inv(qk_serial_sumsq(trow, D), (float)D, ep.eps);
+#pragma unroll
+                        for (int j = 0; j < 8; j++) {
+                            float y0, y1;
+                            qk_rotate(qk_norm_mul(x0[j], inv, w0[j]), qk_norm_mul(x1[j], inv, w1[j]), c[j], sn[j], y0,
+                                      y1);
+                            y0v[j] = (f16)y0;
+                            y1v[j] = (f16)y1;
+                        }
                     }
+                    dst = entry == 0 ? ep.q16 + ((uint64_t)tok * ep.n_q_heads + head) * D
+                                     : ep.k_cache + ((uint64_t)head * ep.max_ctx + ep.pos + tok) * D;
                 }
-                dst = entry == 0 ? ep.q16 + ((uint64_t)tok * ep.n_q_heads + head) * D
-                                 : ep.k_cache + ((uint64_t)head * ep.max_ctx + ep.pos + tok) * D;
-            }
-            if (ok) {
-                *(f16x8_t*)(dst + k8) = y0v;
-                *(f16x8_t*)(dst + HALF + k8) = y1v;
+                if (ok) {
+                    *(f16x8_t*)(dst + k8) = y0v;
+                    *(f16x8_t*)(dst + HALF + k8) = y1v;
+                }
             }
         }
         return;
     }
+    // rows 32 i + 8 v + 4 h + [0, 4) of the tile in acc[i][4 v ..]; every residual of a
+    // subtile is asked for before the first store
+    const uint32_t oc = n0 + col;
+    if (oc >= n) return;
 #pragma unroll
-    for (int i = 0; i < TM; i++)
+    for (int i = 0; i < TM; i++) {
+        uint64_t o[16];
+        float rv[16];
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const uint32_t row = m0 + wm0 + 16 * i + 4 * grp + e;
-            if (row >= m) continue;
-            const int sh = row_exp[GRP && mt.x_rows ? mt.x_rows[row] : row] - kXExpBias;
-            const uint32_t orow = GRP && mt.out_rows ? mt.out_rows[row] : row;
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                const uint32_t col = n0 + wn0 + 16 * j + r16;
-                if (col < n) {
-                    const uint64_t o = (uint64_t)orow * n + col;
-                    const float v = __builtin_ldexpf(acc[i][j][e], sh);
-                    out[o] = res ? res[o] + v : v;
-                }
-            }
+        for (int e = 0; e < 16; e++) {
+            const uint32_t lr = 32 * i + 8 * (e / 4) + 4 * h + e % 4;
+            const uint32_t orow = GRP ? s_orow[lr] : min(m0 + lr, m - 1);
+            o[e] = (uint64_t)orow * n + oc;
+            rv[e] = 0.0f;
         }
+        if (res) {  // uniform
+#pragma unroll
+            for (int e = 0; e < 16; e++) rv[e] = res[o[e]];
+        }
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            const uint32_t lr = 32 * i + 8 * (e / 4) + 4 * h + e % 4;
+            const float v = __builtin_ldexpf(acc[i][e], s_sh[lr]);
+            if (m0 + lr < m) out[o[e]] = res ? rv[e] + v : v;
+        }
+    }
 }
 
 // Any shape or alignment: one thread per output in the reference's serial order
@@ -957,8 +1009,18 @@ static uint32_t gemm_row_tiles(uint32_t m, uint32_t bm) {
     return t >= 8 ? (t + 7) / 8 * 8 : t;
 }
 
+// 64-row tiles while those fill the CUs at most about once: a tile of twice the rows then
+// only takes longer (m 100, n 2048, k 4096: 50 against 70 us; m 128, n 4096, k 2048: 26
+// against 38; m 203, n 9216, k 4096, 288 tiles: 72 against 75). Above, 128 rows convert each
+// weight half as often (m 500, n 5120, k 2048, 320 tiles: 42 against 46; 2048 tokens: 133
+// against 162).
+static bool gemm_half_tiles(const ds5_hip_ctx* ctx, uint32_t m, uint32_t cols) {
+    const uint64_t cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    return ((uint64_t)m + 63) / 64 * cols <= cu + cu / 8;
+}
+
 // The split x is made once and shared by the group's products.
-template <int BM, int BN, int WM, int WN>
+template <int TM>
 int launch_gemm(ds5_hip_ctx* ctx, const MatmulGroupLaunch& a) {
     void* ws = nullptr;
     if (int rc = ds5_workspace(ctx, x_split_bytes(a.m, a.k), &ws)) return rc;
@@ -976,13 +1038,13 @@ int launch_gemm(ds5_hip_ctx* ctx, const MatmulGroupLaunch& a) {
         g.res[g.count] = a.res[e];
         g.n[g.count] = a.n[e];
         g.wg0[g.count] = tiles;
-        tiles += (a.n[e] + BN - 1) / BN;
+        tiles += (a.n[e] + kGemmCols - 1) / kGemmCols;
         g.count += a.n[e] ? 1 : 0;  // entries without rows are dropped
     }
     if (tiles == 0) return DS5_OK;
-    DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<BM, BN, WM, WN, 0>),
-                     dim3(tiles, gemm_row_tiles(a.m, BM)), dim3(WM * WN * 64), 0, ctx->stream, hi, lo, row_exp, g, a.m, a.k,
-                     AttnPrepEpi{}, MoeGemmTiles{});
+    DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<TM, 0>),
+                     dim3(tiles, gemm_row_tiles(a.m, 32 * TM)), dim3(kGemmThreads), 0, ctx->stream, hi, lo, row_exp, g, a.m,
+                     a.k, AttnPrepEpi{}, MoeGemmTiles{});
     return ds5_after_launch(ctx, "matmul_q8_mfma_kernel");
 }
 
@@ -1015,7 +1077,7 @@ int launch_moe_h_split(ds5_hip_ctx* ctx, const float* g, const float* u, uint32_
     return ds5_after_launch(ctx, "moe_h_split_kernel");
 }
 
-template <int BM, int BN, int WM, int WN>
+template <int TM>
 static int launch_q8_gemm_grouped_t(ds5_hip_ctx* ctx, const uint16_t* hi, const uint16_t* lo, const int* row_exp,
                                     uint32_t k, const uint8_t* const* w, float* const* out, const uint32_t* n,
                                     uint32_t count, uint32_t max_tiles, const MoeGemmTiles& mt) {
@@ -1026,12 +1088,12 @@ static int launch_q8_gemm_grouped_t(ds5_hip_ctx* ctx, const uint16_t* hi, const 
         g.out[e] = out[e];
         g.n[e] = n[e];
         g.wg0[e] = nt;
-        nt += (n[e] + BN - 1) / BN;
+        nt += (n[e] + kGemmCols - 1) / kGemmCols;
     }
     g.count = count;
     if (nt == 0 || max_tiles == 0) return DS5_OK;
-    DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<BM, BN, WM, WN, 0, true>),
-                     dim3(nt, gemm_row_tiles(max_tiles, 1)), dim3(WM * WN * 64), 0, ctx->stream, hi, lo, row_exp, g, 0u, k,
+    DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<TM, 0, true>),
+                     dim3(nt, gemm_row_tiles(max_tiles, 1)), dim3(kGemmThreads), 0, ctx->stream, hi, lo, row_exp, g, 0u, k,
                      AttnPrepEpi{}, mt);
     return ds5_after_launch(ctx, "matmul_q8_mfma_kernel");
 }
@@ -1042,9 +1104,9 @@ int launch_q8_gemm_grouped(ds5_hip_ctx* ctx, const uint16_t* hi, const uint16_t*
                            uint64_t w_stride, const uint32_t* x_rows, const uint32_t* out_rows) {
     const MoeGemmTiles mt{tiles, n_tiles, w_stride, x_rows, out_rows};
     if (tile_rows == 64)
-        return launch_q8_gemm_grouped_t<64, 128, 2, 2>(ctx, hi, lo, row_exp, k, w, out, n, count, max_tiles, mt);
+        return launch_q8_gemm_grouped_t<2>(ctx, hi, lo, row_exp, k, w, out, n, count, max_tiles, mt);
     if (tile_rows == 128)
-        return launch_q8_gemm_grouped_t<128, 128, 4, 2>(ctx, hi, lo, row_exp, k, w, out, n, count, max_tiles, mt);
+        return launch_q8_gemm_grouped_t<4>(ctx, hi, lo, row_exp, k, w, out, n, count, max_tiles, mt);
     return ds5_fail(ctx, DS5_DEVICE_FAILURE, "moe: row tiles of %u rows", tile_rows);
 }
 
@@ -1057,7 +1119,6 @@ size_t qkv_prep_workspace_bytes(uint32_t m, uint32_t k, uint32_t head_dim) {
 }
 
 int launch_qkv_prep(ds5_hip_ctx* ctx, const QkvPrepLaunch& a) {
-    constexpr int BM = 128, BN = 128, WM = 4, WN = 2;
     uint16_t* hi = (uint16_t*)a.ws;
     uint16_t* lo = hi + (size_t)a.m * a.k;
     int* row_exp = (int*)(lo + (size_t)a.m * a.k);
@@ -1074,13 +1135,16 @@ int launch_qkv_prep(ds5_hip_ctx* ctx, const QkvPrepLaunch& a) {
         g.w[e] = ws[e];
         g.n[e] = ns[e];
         g.wg0[e] = tiles;
-        tiles += ns[e] / BN;
+        tiles += ns[e] / kGemmCols;
     }
     g.count = 3;
     AttnPrepEpi ep{a.q_norm, a.k_norm, cs, a.q16, a.k_cache, a.v_cache, a.pos, a.n_q_heads, a.max_ctx, a.eps, a.q_scale};
-    DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<BM, BN, WM, WN, 1>),
-                     dim3(tiles, gemm_row_tiles(a.m, BM)), dim3(WM * WN * 64), 0, ctx->stream, hi, lo, row_exp, g, a.m, a.k,
-                     ep, MoeGemmTiles{});
+    if (gemm_half_tiles(ctx, a.m, tiles))
+        DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<2, 1>), dim3(tiles, gemm_row_tiles(a.m, 64)),
+                         dim3(kGemmThreads), 0, ctx->stream, hi, lo, row_exp, g, a.m, a.k, ep, MoeGemmTiles{});
+    else
+        DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<4, 1>), dim3(tiles, gemm_row_tiles(a.m, 128)),
+                         dim3(kGemmThreads), 0, ctx->stream, hi, lo, row_exp, g, a.m, a.k, ep, MoeGemmTiles{});
     return ds5_after_launch(ctx, "matmul_q8_mfma_kernel");
 }
 
@@ -1129,8 +1193,11 @@ static int launch_same_path(ds5_hip_ctx* ctx, const MatmulGroupLaunch& a, Matmul
         return ds5_fail(ctx, DS5_DEVICE_FAILURE, "matmul: an in-kernel norm needs the row or GEMM path and k > %u",
                         kRmsSerialMaxDim);
     if (path == MatmulPath::Rows) return a.q8 ? launch_rows_q<true>(ctx, a) : launch_rows_q<false>(ctx, a);
-    if (path == MatmulPath::Gemm)
-        return a.m >= 128 ? launch_gemm<128, 128, 4, 2>(ctx, a) : launch_gemm<32, 64, 2, 2>(ctx, a);
+    if (path == MatmulPath::Gemm) {
+        uint32_t cols = 0;
+        for (uint32_t e = 0; e < a.count; e++) cols += (a.n[e] + kGemmCols - 1) / kGemmCols;
+        return gemm_half_tiles(ctx, a.m, cols) ? launch_gemm<2>(ctx, a) : launch_gemm<4>(ctx, a);
+    }
     for (uint32_t e = 0; e < a.count; e++)
         if (a.n[e])
             if (int rc = launch_generic(ctx, a.x, a.w[e], a.q8, a.out[e], a.res[e], a.m, a.n[e], a.k)) return rc;

@@ -1,0 +1,51 @@
+"""The Q8_0 matrix-core products at the edges of their tiles: rows around 32, 64 and 128, ragged
+columns, odd block counts, both tile heights (few and many workgroups), with and without a
+residual, against float64."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def q8_rows(g, n, k):
+    """Q8_0 rows [n, k / 32 * 34] with scales over two decades, and their exact f64 values."""
+    w = np.empty((n, k // 32, 34), np.uint8)
+    s = (10.0 ** g.uniform(-3, -1, (n, k // 32))).astype(np.float16)
+    q = g.integers(-127, 128, (n, k // 32, 32)).astype(np.int8)
+    w[:, :, :2] = s[..., None].view(np.uint8).reshape(n, k // 32, 2)
+    w[:, :, 2:] = q.view(np.uint8)
+    return w.reshape(n, -1), (s.astype(np.float64)[..., None] * q).reshape(n, k)
+
+
+def bound(x, w, extra=0.0):
+    """x as hi + lo f16 of the row's power of two (2^-22 of the row's largest element at worst,
+    2^-21 with both roundings), f32 sums of 32 exact products per block and of the blocks."""
+    k = x.shape[1]
+    xa = np.abs(x) + 2.0 ** -21 * np.abs(x).max(1, keepdims=True)
+    return (2.0 ** -21 + (32 + k // 32 + 8) * 2.0 ** -24) * (xa @ np.abs(w).T) + \
+        2.0 ** -21 * np.abs(x).max(1, keepdims=True) * np.abs(w).sum(1)[None] + extra
+
+
+CASES = [(16, 128, 64), (17, 1, 32), (31, 127, 96), (33, 300, 2048), (63, 512, 160), (64, 129, 4096), (65, 4096, 256),
+         (127, 40, 224), (128, 256, 32 * 65), (129, 130, 2048), (200, 20000, 64), (300, 12000, 96)]
+
+
+@pytest.mark.parametrize("m,n,k", CASES)
+@pytest.mark.parametrize("residual", [False, True], ids=["matmul", "matmul_add"])
+def test_gemm_tile_edges(ctx, hip, m, n, k, residual):
+    print(f"[gemm] m={m} n={n} k={k} residual={residual}", flush=True)
+    g = np.random.default_rng(m * 7 + n)
+    x = (g.standard_normal((m, k)) * 10.0 ** g.uniform(-4, 4, (m, 1))).astype(np.float32)
+    x[m // 2] = 0.0
+    wb, w = q8_rows(g, n, k)
+    pad = np.concatenate([wb.reshape(-1), np.zeros(4, np.uint8)])
+    res = g.standard_normal((m, n)).astype(np.float32)
+    xb, wbuf, out = ctx.from_numpy(x), ctx.from_numpy(pad), ctx.from_numpy(np.full((m, n), 7e30, np.float32))
+    if residual:
+        hip.matmulAdd(ctx, hip.MatmulAddArgs(xb, wbuf, hip.DTYPE_Q8_0, ctx.from_numpy(res), out, m, n, k))
+    else:
+        hip.matmul(ctx, hip.MatmulArgs(xb, wbuf, hip.DTYPE_Q8_0, out, m, n, k))
+    got = ctx.to_numpy(out, np.float32, (m, n)).astype(np.float64)
+    want = x.astype(np.float64) @ w.T + (res if residual else 0.0)
+    lim = bound(x.astype(np.float64), w, 2.0 ** -23 * np.abs(want) if residual else 0.0)
+    assert np.all(np.abs(got - want) <= lim + 1e-30), float(np.max(np.abs(got - want) / (lim + 1e-30)))
