@@ -139,9 +139,10 @@ struct MatmulLaunch {
     uint32_t m, n, k;
     const float* res = nullptr;  // out = res + x . W^T when set (res may be out itself)
 };
-// Which kernel runs: the row (GEMV) kernel, the Q8_0 matrix-core GEMM, or the
-// serial one-thread-per-output kernel that takes any shape and alignment.
-enum class MatmulPath { Generic, Rows, Gemm };
+// Which kernel runs: the row (GEMV) kernel, the Q8_0 matrix-core GEMM (GemmSplit: with a
+// tile's blocks split over groups of wavefronts), or the serial one-thread-per-output
+// kernel that takes any shape and alignment.
+enum class MatmulPath { Generic, Rows, Gemm, GemmSplit };
 MatmulPath matmul_path(const MatmulLaunch& a, uint64_t w_len);
 int launch_matmul(ds5_hip_ctx* ctx, const MatmulLaunch& a, MatmulPath path);
 // Up to kMatmulGroupMax products sharing x (and m, k, the weight dtype).
@@ -183,6 +184,7 @@ struct QkvPrepLaunch {
     void* ws;
     const float* norm_w;  // x normalised first, as MatmulGroupLaunch::norm_w (null: none)
     float norm_eps;
+    bool split;  // MatmulPath::GemmSplit for all three
 };
 size_t qkv_prep_workspace_bytes(uint32_t m, uint32_t k, uint32_t head_dim);
 int launch_qkv_prep(ds5_hip_ctx* ctx, const QkvPrepLaunch& a);
@@ -245,9 +247,9 @@ struct ExpertLaunch {
     uint32_t *perm, *xrow, *n_tiles;
     uint4* tiles;
 };
-// The grouped path's row tiles: at most P / rows + E of 64 or 128 rows (each expert's
+// The grouped path's row tiles: at most P / rows + E of 32, 64 or 128 rows (each expert's
 // last one partial).
-constexpr uint32_t kMoeMinTileRows = 64;
+constexpr uint32_t kMoeMinTileRows = 32;
 inline uint32_t moe_max_tiles(uint32_t n_pairs, uint32_t n_experts, uint32_t tile_rows = kMoeMinTileRows) {
     return n_pairs / tile_rows + n_experts + 1;
 }

@@ -283,10 +283,13 @@ static bool experts_fast(ds5_buf x, ds5_buf gate, ds5_buf up, ds5_buf down, uint
 }
 
 // The experts run grouped (sorted by expert, on the matrix cores) when their Q8_0
-// banks take the wavefront kernels and the pairs share experts: from two pairs per
-// expert on average, each expert's weights are read once instead of once per pair.
+// banks take the wavefront kernels and the pairs share experts: each expert's weights are
+// read once instead of once per pair. From 11 pairs per 8 experts on average where there are
+// enough pairs to pay for the four more launches (128 experts of 2048 x 768, the MoE call: 24
+// tokens x 8 pairs 271 us pair by pair, 234 grouped; 17 tokens 192 and 211), from two pairs
+// per expert in any case.
 static bool experts_grouped(bool fast, uint32_t dt, uint64_t P, uint64_t E, uint64_t dim, uint64_t ffn) {
-    return fast && dt == DS5_DTYPE_Q8_0 && E > 0 && E <= kMoeGroupedMaxExperts && P >= 2 * E &&
+    return fast && dt == DS5_DTYPE_Q8_0 && E > 0 && E <= kMoeGroupedMaxExperts && (P >= 2 * E || (8 * P >= 11 * E && P >= 32)) &&
            P * std::max(dim, ffn) * 2 < (1ull << 32) && row_bytes_of(dt, std::max(dim, ffn)) * std::max(dim, ffn) <
                                                                 (1ull << 31);
 }
@@ -365,10 +368,11 @@ static ExpertLaunch expert_launch(const ds5_buf& x, const ds5_buf& gate, const d
     l.grouped = s.tiles != nullptr && s.n_tiles != nullptr && experts_grouped(l.fast, dt, P, E, dim, ffn);
     if (l.grouped) {
         l.n_experts = E;
-        // 128-row tiles (8 wavefronts) from ~96 pairs per expert; below, 64-row tiles (4
-        // wavefronts) leave fewer rows of each expert's last tile empty (2048 tokens x 8
-        // over 128 experts: 1.01 ms with 128 rows, 1.12 with 64; 512 tokens: 0.53, 0.41)
-        l.tile_rows = P >= 96ull * E ? 128 : kMoeMinTileRows;
+        // 128-row tiles from ~96 pairs per expert; below, 64-row and then 32-row tiles leave
+        // fewer rows of each expert's last tile empty and more workgroups in flight (over 128
+        // experts, products of 256 tokens x 8: 236 us with 32 rows, 248 with 64; 512 tokens:
+        // 267 with 64, 312 with 32)
+        l.tile_rows = P >= 96ull * E ? 128 : P >= 24ull * E ? 64 : 32;
         l.max_tiles = moe_max_tiles(P, E, l.tile_rows);
         l.xhi = s.xhi;
         l.xlo = s.xlo;
@@ -852,7 +856,8 @@ int ds5_hip_attention_block(ds5_hip_ctx* ctx, const ds5_attention_block_args* a)
     // every projection takes one of them; otherwise rmsNorm writes h to the context's
     // second buffer first and the block runs on h.
     const bool all_rows = paths[0] == MatmulPath::Rows && paths[1] == MatmulPath::Rows && paths[2] == MatmulPath::Rows;
-    const bool all_gemm = paths[0] == MatmulPath::Gemm && paths[1] == MatmulPath::Gemm && paths[2] == MatmulPath::Gemm;
+    const bool all_gemm = paths[0] == paths[1] && paths[1] == paths[2] &&
+                          (paths[0] == MatmulPath::Gemm || paths[0] == MatmulPath::GemmSplit);
     const bool norm_inside = norm && a->hidden > kRmsSerialMaxDim && aligned16(a->x_norm) && (all_rows || all_gemm);
     if (norm && !norm_inside) {
         void* h = nullptr;
@@ -910,6 +915,7 @@ int ds5_hip_attention_block(ds5_hip_ctx* ctx, const ds5_attention_block_args* a)
     qp.ws = (char*)ws + q16_bytes;
     qp.norm_w = gl.norm_w;
     qp.norm_eps = gl.norm_eps;
+    qp.split = paths[0] == MatmulPath::GemmSplit;
     if (int rc = launch_qkv_prep(ctx, qp)) return rc;
     PrefillLaunch l{};
     l.q16 = (const f16*)ws;

@@ -255,8 +255,7 @@ __global__ __launch_bounds__(kMmThreads) void matmul_rows_kernel(const float* __
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kGemmThreads = 256;  // 4 wavefronts, 32 weight rows each
-constexpr int kGemmCols = 128;
+constexpr int kGemmCols = 128;  // columns of a tile of four wavefronts
 
 constexpr int kSplitThreads = 256;
 constexpr int kXExpBias = 14;  // scaled rows have max |x'| in [2^14, 2^15)
@@ -512,13 +511,17 @@ struct MoeGemmTiles {
     const uint32_t* out_rows;
 };
 
-template <int TM, int EPI, bool GRP = false>
-__global__ __launch_bounds__(kGemmThreads, 2) void matmul_q8_mfma_kernel(const uint16_t* __restrict__ xhi,
+// W wavefronts (32 columns each) make the tile. KS > 1: KS groups of W wavefronts share it,
+// each with its own rings over its own range of blocks; the groups' sums add in group order
+// at the end (W does not change the order).
+template <int TM, int W, int KS, int EPI, bool GRP = false>
+__global__ __launch_bounds__(64 * W * KS, W* KS <= 4 ? 2 : W * KS / 4) void matmul_q8_mfma_kernel(const uint16_t* __restrict__ xhi,
                                                                          const uint16_t* __restrict__ xlo,
                                                                          const int* __restrict__ row_exp,
                                                                          const WeightGroup g, uint32_t m, uint32_t k,
                                                                          const AttnPrepEpi ep, const MoeGemmTiles mt) {
-    constexpr int BM = 32 * TM, BN = kGemmCols, W = kGemmThreads / 64;
+    constexpr int BM = 32 * TM, BN = 32 * W, U = TM == 1 ? 1 : 2, kGroupThreads = 64 * W;
+    static_assert(EPI == 0 || BN == kGemmCols, "the epilogue takes a head of 128 columns");
     asm volatile("" ::DS5_GROUP_ARGS(g), "s"(xhi), "s"(xlo), "s"(row_exp), "s"(m), "s"(k));
     // this workgroup's entry and column tile (uniform); out may be the residual itself
     // Workgroup L = y * gridDim.x + x runs on XCD L % 8. With gridDim.y a multiple of 8
@@ -559,7 +562,8 @@ __global__ __launch_bounds__(kGemmThreads, 2) void matmul_q8_mfma_kernel(const u
     // LDS: rings of three x stages [hi, lo][row * 4 + swizzled chunk] and three raw q stages
     // of 2 KB per wavefront; EPI 1 reuses the bytes for a head's f32 tile
     constexpr int kX = 2 * BM * 64, kStages = 3, kQ = 2048, kQ0 = kStages * kX;
-    constexpr int kMain = kQ0 + kStages * W * kQ;
+    constexpr int kGroup = kQ0 + kStages * W * kQ, kMain = KS * kGroup;
+    static_assert((KS - 1) * TM * 16 * kGroupThreads * 4 <= kMain, "the groups' sums fit the rings");
     constexpr int kTileRow = 128 + 4;  // EPI 1 tile row stride in floats (16-byte rows, rows 4 banks apart)
     constexpr int kLdsBytes = EPI == 1 && BM * kTileRow * 4 > kMain ? BM * kTileRow * 4 : kMain;
     __shared__ __attribute__((aligned(16))) unsigned char smem[kLdsBytes];
@@ -569,11 +573,17 @@ __global__ __launch_bounds__(kGemmThreads, 2) void matmul_q8_mfma_kernel(const u
     __shared__ __attribute__((aligned(16))) uint32_t s_orow[GRP ? BM : 4];
 
     const int lane = threadIdx.x & 63, r32 = lane & 31, h = lane >> 5;
-    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wave_id = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wave = wave_id % W, group = wave_id / W;
     const uint32_t n0 = tile * BN, col = 32 * wave + r32;
     const uint32_t nb = k / 32;
     const uint32_t row_bytes = nb * kQ8Bytes;  // below 2^31: the launchers' 32-bit offsets
-    const uint32_t smem_lds = gemm_lds_addr(smem);
+    unsigned char* const ring = smem + group * kGroup;
+    const uint32_t smem_lds = gemm_lds_addr(ring);
+    // this group's blocks [first, first + iters) below nb: every group runs iters iterations
+    // (the barriers), those past its blocks without loads or products
+    const uint32_t iters = (nb + KS - 1) / KS, first = min(group * iters, nb - 1);
+    const uint32_t blocks = min(iters, nb - min(group * iters, nb));
 
     // x: load i of this wavefront fills bytes [1024 (wave + W i), +1024) of a stage, lane L
     // the 16 bytes at +16 L: plane, row r, slot L % 4 holding chunk (L % 4) ^ ((r >> 2) & 3).
@@ -622,7 +632,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void matmul_q8_mfma_kernel(const u
         uint32_t d4;
     };
     auto q_raw = [&](uint32_t slot) {
-        const unsigned char* row = smem + kQ0 + (slot * W + wave) * kQ + 48 * r32;
+        const unsigned char* row = ring + kQ0 + (slot * W + wave) * kQ + 48 * r32;
         return QRaw{*(const u32x4_t*)(row + 16 * h), *(const uint32_t*)(row + (h ? 44 : 16))};
     };
     // part p < 4: four elements; part 4: the scale, from the h = 0 half to both
@@ -645,7 +655,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void matmul_q8_mfma_kernel(const u
         s_sh[threadIdx.x] = row_exp[GRP && mt.x_rows ? mt.x_rows[row] : row] - kXExpBias;
         if constexpr (GRP) s_orow[threadIdx.x] = mt.out_rows ? mt.out_rows[row] : row;
     }
-    static_assert(BM <= kGemmThreads, "a thread per tile row");
+    static_assert(BM <= kGroupThreads * KS, "a thread per tile row");
 
     f32x16 acc[TM];
 #pragma unroll
@@ -671,19 +681,19 @@ __global__ __launch_bounds__(kGemmThreads, 2) void matmul_q8_mfma_kernel(const u
     constexpr int kAhead = 6;
     // Past the end the last block is asked for again, so that every iteration has the same
     // loads outstanding; the loop ends on a full wait.
-    const uint32_t bl = nb - 1;
+    const uint32_t bl = first + max(blocks, 1u) - 1;
     auto issue = [&](uint32_t b, uint32_t stage, uint32_t bq, uint32_t slot, int n) {
         if (n < NX) issue_x(b, stage, n);
         else if (n < NX + 2) issue_q(bq, slot, n - NX);
     };
 #pragma unroll
-    for (int n = 0; n < NX + 2; n++) issue(0, 0, 0, 0, n);
-    issue_q(min(1u, bl), 1, 0);
-    issue_q(min(1u, bl), 1, 1);
+    for (int n = 0; n < NX + 2; n++) issue(first, 0, first, 0, n);
+    issue_q(min(first + 1, bl), 1, 0);
+    issue_q(min(first + 1, bl), 1, 1);
 #pragma unroll
-    for (int n = 0; n < NX + 2; n++) issue(min(1u, bl), 1, min(2u, bl), 2, n);
+    for (int n = 0; n < NX + 2; n++) issue(min(first + 1, bl), 1, min(first + 2, bl), 2, n);
     auto loop = [&](auto pairs) {
-        constexpr int NP = decltype(pairs)::value, NS = 8 * NP;
+        constexpr int NP = decltype(pairs)::value, PS = 4 * U, NS = PS * NP;
         f32x16 t[2][2];  // [parity of the pair][subtile]
         float ps = 0.0f;
 #pragma unroll
@@ -696,32 +706,33 @@ __global__ __launch_bounds__(kGemmThreads, 2) void matmul_q8_mfma_kernel(const u
             wait_vm_only<kVmPerBlock>();
             const QRaw r = q_raw(0);
 #pragma unroll
-            for (int p = 0; p < 5; p++) q_part(q0, q1, sb, r, s2, p);
+            for (int p = 0; p < 5; p++) q_part(q0, q1, sb, r, s2 != (bool)(first & 1), p);
         }
         uint32_t st = 0;
-        auto block = [&](uint32_t b, auto par) {
+        auto block = [&](uint32_t i, auto par) {
             constexpr int P0 = decltype(par)::value;
             wait_vm_only<kVmPerBlock>();
             gemm_lds_sync();
-            const unsigned char* at = smem + st * kX;
+            if (KS > 1 && i >= blocks) return;  // wavefront-uniform
+            const uint32_t b = first + i;
+            const unsigned char* at = ring + st * kX;
             const uint32_t st0 = st, st2 = st == 0 ? 2 : st - 1;  // b % 3, (b + 2) % 3
             st = st == 2 ? 0 : st + 1;
             f16x8_t xr[NS];
             auto read = [&](int n) {
-                const int p = n / 8, s = n % 8 / 2, u = n % 2;
-                xr[n] = x_op(at, s < 2 ? 1 : 0, 2 * p + u, s & 1);
+                const int p = n / PS, s = n % PS / U, u = n % U;
+                xr[n] = x_op(at, s < 2 ? 1 : 0, U * p + u, s & 1);
             };
 #pragma unroll
-            for (int n = 0; n < kAhead; n++) read(n);
+            for (int n = 0; n < min(kAhead, NS); n++) read(n);
             const bool at2 = s2 != (bool)((b + 1) & 1);
             const QRaw nx = q_raw(st);
             f16x8_t n0q = q0, n1q = q1;
             float ns = sb;
             __builtin_amdgcn_sched_barrier(0);
-            static_assert(NS >= kVmPerBlock, "a slot for every load");
 #pragma unroll
             for (int n = 0; n < NS; n++) {
-                const int p = n / 8, q = n % 8, s = q / 2, u = q % 2, cur = (P0 + p) & 1, pp = p == 0 ? NP - 1 : p - 1;
+                const int p = n / PS, q = n % PS, s = q / U, u = q % U, cur = (P0 + p) & 1, pp = p == 0 ? NP - 1 : p - 1;
                 if (n + kAhead < NS) read(n + kAhead);
                 // one load per product or two: a load holds the wavefront's issue for as
                 // long as the memory pipe needs for it (64 B a cycle and CU), which only
@@ -729,7 +740,9 @@ __global__ __launch_bounds__(kGemmThreads, 2) void matmul_q8_mfma_kernel(const u
                 if constexpr (NS >= 2 * kVmPerBlock) {
                     if (n % 2 == 1) issue(min(b + 2, bl), st2, min(b + 3, bl), st0, n / 2);
                 } else {
-                    issue(min(b + 2, bl), st2, min(b + 3, bl), st0, n);
+#pragma unroll
+                    for (int v = n * kVmPerBlock / NS; v < (n + 1) * kVmPerBlock / NS; v++)
+                        issue(min(b + 2, bl), st2, min(b + 3, bl), st0, v);
                 }
                 if (s == 0) {
                     f32x16 z;
@@ -743,11 +756,12 @@ __global__ __launch_bounds__(kGemmThreads, 2) void matmul_q8_mfma_kernel(const u
 #pragma unroll
                 for (int e = 4 * (q % 4); e < 4 * (q % 4) + 4; e++)
 {
-                    float v = __builtin_fmaf(sc, t[cur ^ 1][q / 4][e], acc[2 * pp + q / 4][e]);
+                    float v = __builtin_fmaf(sc, t[cur ^ 1][q / 4][e], acc[U * pp + q / 4][e]);
                     asm volatile("" : "+v"(v));  // here, not sunk into a later block
-                    acc[2 * pp + q / 4][e] = v;
+                    acc[U * pp + q / 4][e] = v;
                 }
                 if (p == NP - 1 && q < 5) q_part(n0q, n1q, ns, nx, at2, q);
+                if (PS < 5 && n == NS - 1) q_part(n0q, n1q, ns, nx, at2, 4);
                 __builtin_amdgcn_sched_barrier(0);
             }
             ps = sb;
@@ -758,39 +772,55 @@ __global__ __launch_bounds__(kGemmThreads, 2) void matmul_q8_mfma_kernel(const u
         auto last = [&](auto par) {  // the last pair's sums
             constexpr int C = decltype(par)::value;
 #pragma unroll
-            for (int u = 0; u < 2; u++)
+            for (int u = 0; u < U; u++)
 #pragma unroll
                 for (int e = 0; e < 16; e++)
-                    acc[2 * NP - 2 + u][e] = __builtin_fmaf(ps, t[C][u][e], acc[2 * NP - 2 + u][e]);
+                    acc[U * (NP - 1) + u][e] = __builtin_fmaf(ps, t[C][u][e], acc[U * (NP - 1) + u][e]);
         };
-        uint32_t b = 0;
-        for (; b + 2 <= nb; b += 2) {
-            block(b, std::integral_constant<int, 0>{});
-            block(b + 1, std::integral_constant<int, NP & 1>{});
+        for (uint32_t i = 0; i < iters; i += 2) {
+            block(i, std::integral_constant<int, 0>{});
+            if (i + 1 < iters) block(i + 1, std::integral_constant<int, NP & 1>{});
         }
-        if (b < nb) {
-            block(b, std::integral_constant<int, 0>{});
-            last(std::integral_constant<int, (NP - 1) & 1>{});
-        } else {
-            last(std::integral_constant<int, ((NP & 1) + NP - 1) & 1>{});
-        }
+        if (NP & 1 && blocks % 2 == 0) last(std::integral_constant<int, NP & 1>{});  // uniform
+        else last(std::integral_constant<int, (NP - 1) & 1>{});
         wait_vm_only<0>();  // the repeated loads, before their LDS is used or given up
     };
     // pairs of 32-row subtiles that hold rows (uniform); the others skip their products
     const uint32_t live = (uint32_t)__builtin_amdgcn_readfirstlane((int)((m - m0 + 63) / 64));
+    static_assert(TM == 1 || TM == 2 || TM == 4, "tiles");
     if constexpr (TM > 2) {
         if (live >= TM / 2) loop(std::integral_constant<int, TM / 2>{});
         else loop(std::integral_constant<int, 1>{});
-        static_assert(TM <= 4, "one partial form");
     } else {
         loop(std::integral_constant<int, 1>{});
+    }
+
+    if constexpr (KS > 1) {
+        // the groups' sums to group 0, in group order
+        float* part = reinterpret_cast<float*>(smem);
+        __syncthreads();  // every group's last ring reads
+        if (group > 0)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int e = 0; e < 16; e++)
+                    part[(((group - 1) * TM + i) * 16 + e) * kGroupThreads + (threadIdx.x % kGroupThreads)] = acc[i][e];
+        __syncthreads();
+        if (group == 0)
+#pragma unroll
+            for (int q = 1; q < KS; q++)
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) acc[i][e] += part[(((q - 1) * TM + i) * 16 + e) * kGroupThreads + threadIdx.x];
+        if (EPI == 0 && group > 0) return;
     }
 
     if constexpr (EPI == 1) {
         // One head (128 columns, four wavefronts) at a time goes through LDS; then thread t
         // takes row t / 8 (+ 64, ...), dims k8 + [0, 8) and 64 + k8 + [0, 8) (8 rope
         // pairs), k8 = 8 (t % 8).
-        constexpr int D = 128, HALF = 64, TROW = kTileRow, kRowsPer = kGemmThreads / 8;
+        constexpr int D = 128, HALF = 64, TROW = kTileRow, kRowsPer = kGroupThreads * KS / 8;
         const int r0 = threadIdx.x / 8, k8 = 8 * (threadIdx.x % 8);
         const float* nw = entry == 0 ? ep.q_norm : ep.k_norm;
         float w0[8], w1[8];
@@ -805,7 +835,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void matmul_q8_mfma_kernel(const u
         for (uint32_t hd = 0; hd < BN / D && n0 + D * hd < n; hd++) {  // uniform
             const uint32_t head = tile * (BN / D) + hd;
             __syncthreads();  // every wavefront's last read of the bytes
-            if (wave / 4 == hd) {
+            if (wave / 4 == hd && group == 0) {
 #pragma unroll
                 for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -1019,8 +1049,15 @@ static bool gemm_half_tiles(const ds5_hip_ctx* ctx, uint32_t m, uint32_t cols) {
     return ((uint64_t)m + 63) / 64 * cols <= cu + cu / 8;
 }
 
+// Split products: 32 columns a workgroup until 128 fill the CUs (m 17, n 2048, k 4096: 14
+// against 28 us; above, x would be read four times as often: n 65536, 805 MB of it).
+static bool gemm_narrow_tiles(const ds5_hip_ctx* ctx, uint32_t m, uint32_t cols) {
+    const uint64_t cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    return ((uint64_t)m + 31) / 32 * cols <= cu;
+}
+
 // The split x is made once and shared by the group's products.
-template <int TM>
+template <int TM, int W, int KS>
 int launch_gemm(ds5_hip_ctx* ctx, const MatmulGroupLaunch& a) {
     void* ws = nullptr;
     if (int rc = ds5_workspace(ctx, x_split_bytes(a.m, a.k), &ws)) return rc;
@@ -1038,12 +1075,12 @@ int launch_gemm(ds5_hip_ctx* ctx, const MatmulGroupLaunch& a) {
         g.res[g.count] = a.res[e];
         g.n[g.count] = a.n[e];
         g.wg0[g.count] = tiles;
-        tiles += (a.n[e] + kGemmCols - 1) / kGemmCols;
+        tiles += (a.n[e] + 32 * W - 1) / (32 * W);
         g.count += a.n[e] ? 1 : 0;  // entries without rows are dropped
     }
     if (tiles == 0) return DS5_OK;
-    DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<TM, 0>),
-                     dim3(tiles, gemm_row_tiles(a.m, 32 * TM)), dim3(kGemmThreads), 0, ctx->stream, hi, lo, row_exp, g, a.m,
+    DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<TM, W, KS, 0>),
+                     dim3(tiles, gemm_row_tiles(a.m, 32 * TM)), dim3(64 * W * KS), 0, ctx->stream, hi, lo, row_exp, g, a.m,
                      a.k, AttnPrepEpi{}, MoeGemmTiles{});
     return ds5_after_launch(ctx, "matmul_q8_mfma_kernel");
 }
@@ -1077,7 +1114,7 @@ int launch_moe_h_split(ds5_hip_ctx* ctx, const float* g, const float* u, uint32_
     return ds5_after_launch(ctx, "moe_h_split_kernel");
 }
 
-template <int TM>
+template <int TM, int W, int KS>
 static int launch_q8_gemm_grouped_t(ds5_hip_ctx* ctx, const uint16_t* hi, const uint16_t* lo, const int* row_exp,
                                     uint32_t k, const uint8_t* const* w, float* const* out, const uint32_t* n,
                                     uint32_t count, uint32_t max_tiles, const MoeGemmTiles& mt) {
@@ -1088,12 +1125,12 @@ static int launch_q8_gemm_grouped_t(ds5_hip_ctx* ctx, const uint16_t* hi, const 
         g.out[e] = out[e];
         g.n[e] = n[e];
         g.wg0[e] = nt;
-        nt += (n[e] + kGemmCols - 1) / kGemmCols;
+        nt += (n[e] + 32 * W - 1) / (32 * W);
     }
     g.count = count;
     if (nt == 0 || max_tiles == 0) return DS5_OK;
-    DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<TM, 0, true>),
-                     dim3(nt, gemm_row_tiles(max_tiles, 1)), dim3(kGemmThreads), 0, ctx->stream, hi, lo, row_exp, g, 0u, k,
+    DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<TM, W, KS, 0, true>),
+                     dim3(nt, gemm_row_tiles(max_tiles, 1)), dim3(64 * W * KS), 0, ctx->stream, hi, lo, row_exp, g, 0u, k,
                      AttnPrepEpi{}, mt);
     return ds5_after_launch(ctx, "matmul_q8_mfma_kernel");
 }
@@ -1103,10 +1140,12 @@ int launch_q8_gemm_grouped(ds5_hip_ctx* ctx, const uint16_t* hi, const uint16_t*
                            const uint4* tiles, const uint32_t* n_tiles, uint32_t max_tiles, uint32_t tile_rows,
                            uint64_t w_stride, const uint32_t* x_rows, const uint32_t* out_rows) {
     const MoeGemmTiles mt{tiles, n_tiles, w_stride, x_rows, out_rows};
+    if (tile_rows == 32)
+        return launch_q8_gemm_grouped_t<1, 4, 1>(ctx, hi, lo, row_exp, k, w, out, n, count, max_tiles, mt);
     if (tile_rows == 64)
-        return launch_q8_gemm_grouped_t<2>(ctx, hi, lo, row_exp, k, w, out, n, count, max_tiles, mt);
+        return launch_q8_gemm_grouped_t<2, 4, 1>(ctx, hi, lo, row_exp, k, w, out, n, count, max_tiles, mt);
     if (tile_rows == 128)
-        return launch_q8_gemm_grouped_t<4>(ctx, hi, lo, row_exp, k, w, out, n, count, max_tiles, mt);
+        return launch_q8_gemm_grouped_t<4, 4, 1>(ctx, hi, lo, row_exp, k, w, out, n, count, max_tiles, mt);
     return ds5_fail(ctx, DS5_DEVICE_FAILURE, "moe: row tiles of %u rows", tile_rows);
 }
 
@@ -1139,12 +1178,16 @@ int launch_qkv_prep(ds5_hip_ctx* ctx, const QkvPrepLaunch& a) {
     }
     g.count = 3;
     AttnPrepEpi ep{a.q_norm, a.k_norm, cs, a.q16, a.k_cache, a.v_cache, a.pos, a.n_q_heads, a.max_ctx, a.eps, a.q_scale};
-    if (gemm_half_tiles(ctx, a.m, tiles))
-        DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<2, 1>), dim3(tiles, gemm_row_tiles(a.m, 64)),
-                         dim3(kGemmThreads), 0, ctx->stream, hi, lo, row_exp, g, a.m, a.k, ep, MoeGemmTiles{});
-    else
-        DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<4, 1>), dim3(tiles, gemm_row_tiles(a.m, 128)),
-                         dim3(kGemmThreads), 0, ctx->stream, hi, lo, row_exp, g, a.m, a.k, ep, MoeGemmTiles{});
+    auto launch = [&](auto tm, auto ks) {
+        constexpr int TM = decltype(tm)::value, KS = decltype(ks)::value;
+        DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<TM, 4, KS, 1>),
+                         dim3(tiles, gemm_row_tiles(a.m, 32 * TM)), dim3(256 * KS), 0, ctx->stream, hi, lo, row_exp, g, a.m,
+                         a.k, ep, MoeGemmTiles{});
+    };
+    using std::integral_constant;
+    if (a.split) launch(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+    else if (gemm_half_tiles(ctx, a.m, tiles)) launch(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+    else launch(integral_constant<int, 4>{}, integral_constant<int, 1>{});
     return ds5_after_launch(ctx, "matmul_q8_mfma_kernel");
 }
 
@@ -1166,6 +1209,16 @@ static bool gemm_offsets_fit(uint32_t m, uint32_t k, uint64_t w_end) {
     return (uint64_t)m * k * 2 < (1ull << 32) && w_end + 2 < (1ull << 32);
 }
 
+// Few tokens on a matrix that is not huge: four groups of wavefronts split a tile's blocks,
+// as otherwise most CUs have no tile and the others wait for one block after the other
+// (m 32, n 2048, k 4096: 41 us unsplit, 15 split; m 64, n 5120, k 2048: 26 and 17; m 128, n
+// 2048, k 4096: 50 and 20). From 16384 columns there are tiles enough, and 32-row tiles would
+// only read the weights once more. Chosen from the product's own shape: in a group or in the
+// attention block it adds in the same order.
+static bool gemm_split(uint32_t m, uint32_t n, uint32_t k) {
+    return k >= 32 * 8 && (m <= 32 || (m <= 128 && n < 16384));
+}
+
 MatmulPath matmul_path(const MatmulLaunch& a, uint64_t w_len) {
     const uintptr_t x_addr = (uintptr_t)a.x, out_addr = (uintptr_t)a.out, w_addr = (uintptr_t)a.w;
     if (a.k % 32 != 0 || (x_addr & 15u)) return MatmulPath::Generic;
@@ -1174,9 +1227,10 @@ MatmulPath matmul_path(const MatmulLaunch& a, uint64_t w_len) {
     const uint64_t end = (uint64_t)a.n * (a.k / 32) * kQ8Bytes;
     if ((w_addr & 3u) || !((w_addr + end) % 4 == 0 || w_len >= end + 2)) return MatmulPath::Generic;
     const bool gemm = (out_addr & 3u) == 0 && gemm_offsets_fit(a.m, a.k, end);
-    if (a.m >= kGemmMinM && gemm) return MatmulPath::Gemm;
+    const MatmulPath gemm_path = gemm_split(a.m, a.n, a.k) ? MatmulPath::GemmSplit : MatmulPath::Gemm;
+    if (a.m >= kGemmMinM && gemm) return gemm_path;
     if (a.k / 32 <= 256 && (out_addr & 15u) == 0) return MatmulPath::Rows;
-    return gemm ? MatmulPath::Gemm : MatmulPath::Generic;
+    return gemm ? gemm_path : MatmulPath::Generic;
 }
 
 static int launch_generic(ds5_hip_ctx* ctx, const float* x, const uint8_t* w, bool q8, float* out, const float* res,
@@ -1193,10 +1247,12 @@ static int launch_same_path(ds5_hip_ctx* ctx, const MatmulGroupLaunch& a, Matmul
         return ds5_fail(ctx, DS5_DEVICE_FAILURE, "matmul: an in-kernel norm needs the row or GEMM path and k > %u",
                         kRmsSerialMaxDim);
     if (path == MatmulPath::Rows) return a.q8 ? launch_rows_q<true>(ctx, a) : launch_rows_q<false>(ctx, a);
-    if (path == MatmulPath::Gemm) {
+    if (path == MatmulPath::Gemm || path == MatmulPath::GemmSplit) {
         uint32_t cols = 0;
         for (uint32_t e = 0; e < a.count; e++) cols += (a.n[e] + kGemmCols - 1) / kGemmCols;
-        return gemm_half_tiles(ctx, a.m, cols) ? launch_gemm<2>(ctx, a) : launch_gemm<4>(ctx, a);
+        if (path == MatmulPath::Gemm)
+            return gemm_half_tiles(ctx, a.m, cols) ? launch_gemm<2, 4, 1>(ctx, a) : launch_gemm<4, 4, 1>(ctx, a);
+        return gemm_narrow_tiles(ctx, a.m, cols) ? launch_gemm<1, 1, 4>(ctx, a) : launch_gemm<1, 4, 4>(ctx, a);
     }
     for (uint32_t e = 0; e < a.count; e++)
         if (a.n[e])

@@ -49,3 +49,37 @@ def test_gemm_tile_edges(ctx, hip, m, n, k, residual):
     want = x.astype(np.float64) @ w.T + (res if residual else 0.0)
     lim = bound(x.astype(np.float64), w, 2.0 ** -23 * np.abs(want) if residual else 0.0)
     assert np.all(np.abs(got - want) <= lim + 1e-30), float(np.max(np.abs(got - want) / (lim + 1e-30)))
+
+
+@pytest.mark.parametrize("T,E,K,dim,ffn", [(22, 16, 1, 256, 96), (44, 16, 1, 512, 64), (60, 24, 4, 2048, 768)])
+def test_grouped_experts_few_pairs(ctx, hip, T, E, K, dim, ffn):
+    """Few pairs per expert (below, at and above the grouped threshold of 11 per 8 experts) against
+    float64, twice: rows of one expert land in any order."""
+    print(f"[moe] few pairs T={T} E={E} K={K}", flush=True)
+    g = np.random.default_rng(T)
+    (G, Gf), (U, Uf), (D, Df) = (q8_rows(g, E * a, b) for a, b in ((ffn, dim), (ffn, dim), (dim, ffn)))
+    x = (0.05 * g.standard_normal((T, dim))).astype(np.float32)
+    pairs = np.zeros(T * K, hip.PAIR_DTYPE)
+    pairs["token"] = np.repeat(np.arange(T), K)
+    pairs["expert"] = g.integers(0, E, T * K)
+    pairs["weight"] = g.random(T * K).astype(np.float32)
+    want, lim = np.zeros((T, dim)), np.zeros((T, dim))
+    for t, e, w in pairs:
+        Ge, Ue, De = (v.reshape(E, -1, v.shape[1])[e] for v in (Gf, Uf, Df))
+        xd = x[t:t + 1].astype(np.float64)
+        a, u = xd @ Ge.T, xd @ Ue.T
+        da, du = bound(xd, Ge), bound(xd, Ue)
+        h = a / (1 + np.exp(-a)) * u
+        # |silu'| <= 1.1; the exponential and the division within 4 ulp
+        dh = 1.1 * da * np.abs(u) + np.abs(a) * du + 1.1 * da * du + 4 * 2.0 ** -23 * np.abs(h)
+        want[t] += w * (h @ De.T)[0]
+        lim[t] += w * (bound(h, De) + (dh + 2.0 ** -21 * dh.max()) @ np.abs(De).T)[0] + 2.0 ** -22 * np.abs(w * (h @ De.T)[0])
+    lim += (K + 2) * 2.0 ** -23 * np.abs(want)
+    bufs = [ctx.from_numpy(np.concatenate([v.reshape(-1), np.zeros(4, np.uint8)])) for v in (G, U, D)]
+    runs = []
+    for _ in range(2):
+        out = ctx.createBuffer(T * dim * 4)
+        hip.expertMlpSwiglu(ctx, ctx.from_numpy(x), *bufs, hip.DTYPE_Q8_0, pairs, out, T, dim, ffn, E)
+        runs.append(ctx.to_numpy(out, np.float32, (T, dim)))
+    assert np.all(np.abs(runs[0] - want) <= lim), float(np.max(np.abs(runs[0] - want) / lim))
+    assert np.array_equal(runs[0], runs[1])
