@@ -459,9 +459,10 @@ int ds5_hip_attention_block(ds5_hip_ctx* ctx, const ds5_attention_block_args* ar
 /* No reference counterpart. For callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc): ds5_hip_attention_step with the same kernels, arguments,
- * preconditions and results, but the split-K partials (decode) or the f16 q
- * operand (prefill) live in the library's static device scratch array of
- * DS5_NOALLOC_SCRATCH_BYTES per GPU instead of the context's workspace, and
+ * preconditions and results, but the split-K partials (decode) or the rope table
+ * (prefill) live in the library's static device scratch array of
+ * DS5_NOALLOC_SCRATCH_BYTES per GPU instead of the context's workspace (partials of
+ * a prefill split over its keys in a second array of 32 MiB, their upper limit), and
  * the call allocates nothing. A call that would need more scratch than that
  * (e.g. a long prefill) fails with ShapeMismatch before any device work.
  * Every call on one GPU shares that GPU's array: calls that overlap on one

@@ -64,6 +64,7 @@ struct ds5_hip_ctx {
     // comes from there and nothing is allocated.
     void* scratch = nullptr;
     size_t scratch_bytes = 0;
+    void* split_scratch = nullptr;  // kSplitBytesMax bytes, for the same calls' partial results
     bool use_scratch = false;
     // Decode tuning: positions per split-K workgroup (0 = heuristic); paged
     // plan: workgroups per launch the plan aims at (0 = two per CU).
@@ -97,9 +98,18 @@ int ds5_fail(ds5_hip_ctx* ctx, int code, const char* fmt, ...) __attribute__((fo
 int ds5_hip_status(ds5_hip_ctx* ctx, hipError_t err, const char* what);
 int ds5_after_launch(ds5_hip_ctx* ctx, const char* what);
 int ds5_workspace(ds5_hip_ctx* ctx, size_t bytes, void** out);
-// The workspace if `bytes` of it can be had: false, with no error left behind, where a
-// stream capture would have to allocate, the static scratch is smaller, or memory is out.
-bool ds5_workspace_if(ds5_hip_ctx* ctx, size_t bytes, void** out);
+// Workspace for a launch that splits its work: `base` bytes that it needs anyway and `part`
+// (at most kSplitBytesMax) for partial results. False, with no error left behind, where a
+// stream capture would have to allocate or memory is out: the launch then runs unsplit. The
+// allocation-free entry point has a static array for the partials beside its scratch, so
+// that it splits as the allocating one does.
+constexpr size_t kSplitBytesMax = 32u << 20;
+bool ds5_split_workspace(ds5_hip_ctx* ctx, size_t base, size_t part, void** base_out, void** part_out);
+// The most splits of `rows` rows of partials that kSplitBytesMax holds.
+inline uint32_t ds5_max_splits(uint64_t rows, uint32_t head_dim) {
+    const uint64_t row = rows * (head_dim + 2) * sizeof(float);
+    return row ? (uint32_t)std::min<uint64_t>(64, kSplitBytesMax / row) : 64u;
+}
 int ds5_aux_workspace(ds5_hip_ctx* ctx, size_t bytes, void** out);
 // Looks up (once per device) the address of the static scratch array on the
 // context's device, which must be current, and records it in the context.
@@ -345,14 +355,14 @@ struct GenericAttnLaunch {
 };
 int launch_generic_attention(ds5_hip_ctx* ctx, const GenericAttnLaunch& a);
 // The same over f32 caches with head_dim 64 or 128, q, caches and out 16-byte aligned, on
-// the f32 matrix cores (k_attn_f32.hip). chunk positions per split, at most kAttnF32MaxSplits
+// the f32 matrix cores (k_attn_f32.hip). chunk positions per split, at most ds5_max_splits
 // splits; wave_rows: a wavefront per 16-row tile instead of a workgroup.
-constexpr uint32_t kAttnF32MaxSplits = 64;
 struct AttnF32Plan {
     uint32_t row_tiles, chunk, n_splits;
     bool wave_rows;
 };
-AttnF32Plan attn_f32_plan(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads);
+AttnF32Plan attn_f32_plan(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads,
+                          uint32_t head_dim);
 size_t attn_f32_workspace_bytes(uint32_t n_tokens, uint32_t n_q_heads, uint32_t head_dim, uint32_t n_splits);
 int launch_attn_f32(ds5_hip_ctx* ctx, const GenericAttnLaunch& a);
 
@@ -406,8 +416,15 @@ struct PrefillLaunch {
     const f16* v_cache;
     float* out;
     uint32_t pos, n_tokens, n_q_heads, n_kv_heads, head_dim, max_ctx;
+    // the keys split over n_splits workgroups (prefill_splits; 0 or 1: not split), with
+    // prefill_part_bytes of partial results
+    uint32_t n_splits;
+    float* part;
 };
 int launch_prefill(ds5_hip_ctx* ctx, const PrefillLaunch& a);
+uint32_t prefill_splits(const ds5_hip_ctx* ctx, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads,
+                        uint32_t head_dim);
+size_t prefill_part_bytes(uint32_t n_tokens, uint32_t n_q_heads, uint32_t head_dim, uint32_t n_splits);
 
 int launch_fill_normal_f16(ds5_hip_ctx* ctx, f16* out, uint64_t n, uint64_t seed);
 int launch_stream_read(ds5_hip_ctx* ctx, const void* src, uint64_t len, uint32_t* sink);

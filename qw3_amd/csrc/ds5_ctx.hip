@@ -76,11 +76,13 @@ int ds5_workspace(ds5_hip_ctx* ctx, size_t bytes, void** out) {
     return DS5_OK;
 }
 
-bool ds5_workspace_if(ds5_hip_ctx* ctx, size_t bytes, void** out) {
+bool ds5_split_workspace(ds5_hip_ctx* ctx, size_t base, size_t part, void** base_out, void** part_out) {
     if (ctx->use_scratch) {
-        *out = ctx->scratch;
-        return bytes <= ctx->scratch_bytes;
+        *base_out = ctx->scratch;
+        *part_out = ctx->split_scratch;
+        return base <= ctx->scratch_bytes && part <= kSplitBytesMax;
     }
+    const size_t at = (base + 255) & ~(size_t)255, bytes = at + part;
     if (bytes > ctx->workspace_bytes) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return false;
@@ -92,7 +94,8 @@ bool ds5_workspace_if(ds5_hip_ctx* ctx, size_t bytes, void** out) {
             return false;
         }
     }
-    *out = ctx->workspace;
+    *base_out = ctx->workspace;
+    *part_out = (char*)ctx->workspace + at;
     return true;
 }
 

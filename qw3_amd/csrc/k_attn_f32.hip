@@ -332,7 +332,8 @@ int launch_d(ds5_hip_ctx* ctx, const AttnF32Params& p, const AttnF32Plan& plan, 
 
 }  // namespace
 
-AttnF32Plan attn_f32_plan(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads) {
+AttnF32Plan attn_f32_plan(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads,
+                          uint32_t head_dim) {
     const uint32_t group = n_q_heads / n_kv_heads, cu = cu_count ? cu_count : 256;
     const uint64_t L = (uint64_t)pos + n_tokens;
     AttnF32Plan pl{};
@@ -345,7 +346,9 @@ AttnF32Plan attn_f32_plan(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, ui
     const uint64_t least = pl.wave_rows ? 128 : step;  // a split's partials cost about a 100-position tile row
     uint64_t chunk = (L + want - 1) / want;
     chunk = std::max<uint64_t>(least, (chunk + step - 1) / step * step);
-    chunk = std::max<uint64_t>(chunk, (L + kAttnF32MaxSplits * step - 1) / (kAttnF32MaxSplits * step) * step);
+    const uint64_t most = ds5_max_splits((uint64_t)n_tokens * n_q_heads, head_dim);
+    if (most < 2) chunk = L;
+    else chunk = std::max<uint64_t>(chunk, (L + most * step - 1) / (most * step) * step);
     pl.chunk = (uint32_t)std::min<uint64_t>(chunk, 0xfffffff0u);
     pl.n_splits = (uint32_t)((L + pl.chunk - 1) / pl.chunk);
     return pl;
@@ -357,11 +360,12 @@ size_t attn_f32_workspace_bytes(uint32_t n_tokens, uint32_t n_q_heads, uint32_t 
 
 int launch_attn_f32(ds5_hip_ctx* ctx, const GenericAttnLaunch& a) {
     if (a.n_tokens == 0) return DS5_OK;
-    AttnF32Plan plan = attn_f32_plan(ctx->cu_count, a.pos, a.n_tokens, a.n_q_heads, a.n_kv_heads);
-    void* ws = nullptr;
+    AttnF32Plan plan = attn_f32_plan(ctx->cu_count, a.pos, a.n_tokens, a.n_q_heads, a.n_kv_heads, a.head_dim);
+    void *ws = nullptr, *base = nullptr;
     if (plan.n_splits > 1 &&
-        !ds5_workspace_if(ctx, attn_f32_workspace_bytes(a.n_tokens, a.n_q_heads, a.head_dim, plan.n_splits), &ws)) {
-        // no room (a capture that may not allocate, the static scratch): one split needs none
+        !ds5_split_workspace(ctx, 0, attn_f32_workspace_bytes(a.n_tokens, a.n_q_heads, a.head_dim, plan.n_splits), &base,
+                             &ws)) {
+        // no room (a capture that may not allocate): one split needs none
         plan.n_splits = 1;
         plan.chunk = 0xffffffffu;
     }

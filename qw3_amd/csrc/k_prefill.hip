@@ -187,7 +187,15 @@ struct PrefillParams {
     float* out;
     uint32_t pos, n_tokens, n_q_heads, group, max_ctx;
     uint32_t n_qtiles, n_pairs, n_hgroups, n_items, items_per_xcd;
+    // n_splits > 1: workgroup (x, s) takes part s of each of its q tiles' key tiles and leaves
+    // O, unnormalised, in part_o [token, q head, split, D] and (reference, row sum) in part_ml
+    uint32_t n_splits;
+    float* part_o;
+    float2* part_ml;
 };
+
+// Key tiles [lo, hi) of part s of a q tile's n.
+__device__ __forceinline__ uint32_t split_first(uint32_t n, uint32_t s, uint32_t n_splits) { return n * s / n_splits; }
 
 template <int D>
 struct PGeo {
@@ -340,15 +348,21 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(PrefillPara
 
     // Items: the heavy tile's key tiles 0 .. H-1, then the light tile's 0 .. L-1.
     const uint32_t heavy = p.n_qtiles - 1 - pair;
-    const bool has_light = pair < heavy;  // the middle tile of an odd count is processed once
     auto kv_end_of = [&](uint32_t qtile) -> uint32_t {  // keys the q tile needs (exclusive)
         return p.pos + min(p.n_tokens, qtile * kQRows + kQRows);
     };
-    const uint32_t H = (kv_end_of(heavy) + kKTile - 1) / kKTile;
-    const uint32_t L = has_light ? (kv_end_of(pair) + kKTile - 1) / kKTile : 0;
+    // (split: this part's of them, from hk0 and lk0; a heavy tile has at least half of the
+    // keys' tiles and n_splits is at most that half, so H > 0)
+    const uint32_t Hn = (kv_end_of(heavy) + kKTile - 1) / kKTile, Ln = (kv_end_of(pair) + kKTile - 1) / kKTile;
+    const uint32_t split = blockIdx.y;
+    const uint32_t hk0 = split_first(Hn, split, p.n_splits), lk0 = split_first(Ln, split, p.n_splits);
+    const uint32_t H = split_first(Hn, split + 1, p.n_splits) - hk0;
+    // (the middle tile of an odd count is processed once)
+    const uint32_t L = pair < heavy ? split_first(Ln, split + 1, p.n_splits) - lk0 : 0;
+    const bool has_light = L > 0;
     const uint32_t n_items = H + L;
     auto item_qt = [&](uint32_t i) -> uint32_t { return i < H ? heavy : pair; };
-    auto item_kt = [&](uint32_t i) -> uint32_t { return i < H ? i : i - H; };
+    auto item_kt = [&](uint32_t i) -> uint32_t { return i < H ? hk0 + i : lk0 + (i - H); };
     auto k_stage = [&](uint32_t i) -> uint32_t { return (i % kStages) * G::STAGE; };
 
     if (hw == kHeads) {
@@ -711,8 +725,14 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(PrefillPara
     constexpr int OBLK = (G::STAGE / 4) / (32 * OSTR) < DT ? (G::STAGE / 4) / (32 * OSTR) : DT;
     static_assert(OBLK >= 1 && DT % OBLK == 0, "whole passes");
     auto write_rows = [&](uint32_t qtile, char* area) {
-        const float inv_l = 1.0f / Lsum[0];
+        const bool whole = p.n_splits == 1;  // uniform
+        const float inv_l = whole ? 1.0f / Lsum[0] : 1.0f;
         const uint32_t q0 = qtile * kQRows, lane = lane_here();
+        float* const dst = whole ? p.out : p.part_o + (uint64_t)split * D;
+        const uint64_t row_stride = whole ? D : (uint64_t)p.n_splits * D;
+        if (!whole && lane < 32 && live && q0 + lane < p.n_tokens)  // (a row without a key here: weight 0)
+            p.part_ml[((uint64_t)(q0 + lane) * p.n_q_heads + hq) * p.n_splits + split] =
+                float2{Lsum[0] > 0.0f ? m_sh : -INFINITY, Lsum[0]};
 #pragma unroll
         for (int d0 = 0; d0 < DT; d0 += OBLK) {
 #pragma unroll
@@ -729,7 +749,7 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(PrefillPara
                     const uint32_t row = 8 * it + lane / 8, c4 = lane % 8;
                     const float4 v = *(const float4*)(area + (32 * u + row) * OSTR + 16 * c4);
                     if (live && q0 + row < p.n_tokens)
-                        *(float4*)(p.out + ((uint64_t)(q0 + row) * p.n_q_heads + hq) * D + 32 * (d0 + u) + 4 * c4) = v;
+                        *(float4*)(dst + ((uint64_t)(q0 + row) * p.n_q_heads + hq) * row_stride + 32 * (d0 + u) + 4 * c4) = v;
                 }
         }
     };
@@ -820,7 +840,8 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(PrefillPara
     // crosses a q tile's first row (key tile kt of q tile qt with 64 kt + 63 > pos +
     // 32 qt, i.e. kt >= first_masked).
     auto first_masked = [&](uint32_t qtile) -> uint32_t { return (p.pos + qtile * kQRows + 1) / kKTile; };
-    const uint32_t mh = min(first_masked(heavy), H), ml = H + first_masked(pair);
+    auto from = [](uint32_t a, uint32_t b) -> uint32_t { return a > b ? a - b : 0; };
+    const uint32_t mh = min(from(first_masked(heavy), hk0), H), ml = H + from(first_masked(pair), lk0);
     auto next_special = [&](uint32_t r) -> uint32_t {  // the first special round >= r
         uint32_t ns = n_items;
         if (has_light) {
@@ -847,7 +868,55 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(PrefillPara
     }
     write_rows(has_light ? pair : heavy, area_of(k_stage(n_items + kStages - 2)));
 }
+
+// The parts of a split launch: 256 threads take 1024 / D rows, a float4 column each, and fold
+// the row's parts in order.
+template <int D>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
+    constexpr int COLS = D / 4, ROWS = 256 / COLS;
+    const uint64_t row = (uint64_t)blockIdx.x * ROWS + threadIdx.x / COLS;
+    const uint32_t c4 = 4 * (threadIdx.x % COLS);
+    if (row >= (uint64_t)p.n_tokens * p.n_q_heads) return;
+    const uint32_t qt = (uint32_t)(row / p.n_q_heads) / kQRows;
+    const uint32_t n = (p.pos + min(p.n_tokens, qt * kQRows + kQRows) + kKTile - 1) / kKTile;
+    const float2* ml = p.part_ml + row * p.n_splits;
+    const float* o = p.part_o + row * p.n_splits * D + c4;
+    auto used = [&](uint32_t s) { return split_first(n, s, p.n_splits) < split_first(n, s + 1, p.n_splits); };
+    float M = -INFINITY;
+    for (uint32_t s = 0; s < p.n_splits; s++)
+        if (used(s)) M = fmaxf(M, ml[s].x);
+    float l = 0.0f;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t s = 0; s < p.n_splits; s++)
+        if (used(s)) {
+            const float2 v = ml[s];
+            const float w = fast_exp2(v.x - M);
+            l += v.y * w;
+            acc += *(const f32x4*)(o + (uint64_t)s * D) * w;
+        }
+    *(f32x4*)(p.out + row * D + c4) = acc / l;
+}
 }  // namespace
+
+// Parts of a launch's key tiles. A workgroup's rounds are ~1800 cycles each and its prologue
+// and end ~20,000: parts of at least 12 rounds, and as many as CUs have no workgroup
+// otherwise (203 tokens at 6000, 64 q / 4 kv heads: 64 workgroups of 193 rounds, 140 us).
+constexpr uint32_t kSplitMinRounds = 12;
+uint32_t prefill_splits(const ds5_hip_ctx* ctx, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads,
+                        uint32_t head_dim) {
+    const uint32_t qtiles = (n_tokens + kQRows - 1) / kQRows, pairs = (qtiles + 1) / 2;
+    const uint32_t hgroups = (n_q_heads / n_kv_heads + kHeads - 1) / kHeads;
+    const uint64_t wgs = (uint64_t)n_kv_heads * hgroups * pairs, cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    const uint64_t tiles = ((uint64_t)pos + n_tokens + kKTile - 1) / kKTile;
+    const uint64_t rounds = qtiles > 1 ? tiles + (pos + kQRows + kKTile - 1) / kKTile : tiles;
+    const uint64_t s = std::min<uint64_t>({cu / std::max<uint64_t>(wgs, 1), rounds / kSplitMinRounds, tiles / 2,
+                                           (uint64_t)ds5_max_splits((uint64_t)n_tokens * n_q_heads, head_dim)});
+    return (uint32_t)std::max<uint64_t>(s, 1);
+}
+
+size_t prefill_part_bytes(uint32_t n_tokens, uint32_t n_q_heads, uint32_t head_dim, uint32_t n_splits) {
+    return n_splits > 1 ? (size_t)n_tokens * n_q_heads * n_splits * (head_dim + 2) * sizeof(float) : 0;
+}
 
 bool prefill_prep_supported(uint32_t n_kv_heads, uint32_t head_dim) {
     return (uint64_t)n_kv_heads * head_dim <= kPrepMaxRow && (head_dim == 64 || head_dim == 128);
@@ -866,7 +935,8 @@ int launch_kv_prep(ds5_hip_ctx* ctx, const KvPrepLaunch& a) {
 
 template <int D, int QM>
 static void launch_prefill_k(ds5_hip_ctx* ctx, const PrefillParams& p) {
-    DS5_TIMED_LAUNCH(ctx, "prefill_attention_kernel", (prefill_attention_kernel<D, QM>), dim3(p.n_items), dim3(kThreads),
+    DS5_TIMED_LAUNCH(ctx, "prefill_attention_kernel", (prefill_attention_kernel<D, QM>), dim3(p.n_items, p.n_splits),
+                     dim3(kThreads),
                      0, ctx->stream, p);
 }
 
@@ -892,6 +962,10 @@ int launch_prefill(ds5_hip_ctx* ctx, const PrefillLaunch& a) {
     p.n_hgroups = (p.group + kHeads - 1) / kHeads;
     p.n_items = a.n_kv_heads * p.n_hgroups * p.n_pairs;
     p.items_per_xcd = p.n_items % 8 == 0 ? p.n_items / 8 : 0;
+    p.n_splits = std::max(a.n_splits, 1u);
+    const uint64_t rows = (uint64_t)a.n_tokens * a.n_q_heads;
+    p.part_o = a.part;
+    p.part_ml = p.n_splits > 1 ? (float2*)(a.part + rows * p.n_splits * a.head_dim) : nullptr;
     const int qm = a.q16 ? kQOperand : a.cs ? kQRaw : kQRotated;
     if (a.head_dim == 128) {
         if (qm == kQOperand) launch_prefill_k<128, kQOperand>(ctx, p);
@@ -902,5 +976,13 @@ int launch_prefill(ds5_hip_ctx* ctx, const PrefillLaunch& a) {
         else if (qm == kQRaw) launch_prefill_k<64, kQRaw>(ctx, p);
         else launch_prefill_k<64, kQRotated>(ctx, p);
     }
-    return ds5_after_launch(ctx, "prefill_attention_kernel");
+    if (int rc = ds5_after_launch(ctx, "prefill_attention_kernel")) return rc;
+    if (p.n_splits == 1) return DS5_OK;
+    const uint32_t per = 1024 / a.head_dim;
+    const dim3 grid((unsigned)((rows + per - 1) / per));
+    if (a.head_dim == 128)
+        DS5_TIMED_LAUNCH(ctx, "prefill_merge_kernel", prefill_merge_kernel<128>, grid, dim3(256), 0, ctx->stream, p);
+    else
+        DS5_TIMED_LAUNCH(ctx, "prefill_merge_kernel", prefill_merge_kernel<64>, grid, dim3(256), 0, ctx->stream, p);
+    return ds5_after_launch(ctx, "prefill_merge_kernel");
 }

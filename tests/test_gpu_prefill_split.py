@@ -1,0 +1,79 @@
+"""Prefill attention whose key tiles are split over workgroups: short chunks over long
+contexts, where the launch would leave compute units idle. Against float64 at the attention
+gate of the f16 paths (max-abs 2e-3, cosine 0.99999), at parts that start inside a tile
+pair's masked rounds, odd tile counts, part-filled q tiles and the smallest split; and the
+allocation-free step against the step, whose partials live in different memory."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # T, pos, hq, hkv, d
+    (2, 1600, 64, 4, 128),    # one part-filled q tile, the smallest context that splits in two
+    (17, 3001, 32, 4, 128),
+    (33, 2047, 16, 2, 64),    # two q tiles, the light one full
+    (65, 5000, 5, 1, 128),    # an odd count of q tiles, a head group of one
+    (203, 6000, 64, 4, 128),
+    (100, 700, 4, 2, 64),
+    (1600, 0, 4, 1, 128),     # diagonal tiles in every part
+    (1000, 400, 2, 1, 64),
+]
+
+
+def _f64(q, kc, vc, pos, scale):
+    T, hq, d = q.shape
+    group = hq // kc.shape[0]
+    out = np.empty((T, hq, d))
+    L = pos + T
+    mask = np.arange(L)[None, :] > pos + np.arange(T)[:, None]
+    for h in range(hq):
+        k, v = (c[h // group, :L].astype(np.float64) for c in (kc, vc))
+        s = q[:, h].astype(np.float64) @ k.T * scale
+        s[mask] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        out[:, h] = p @ v / p.sum(1, keepdims=True)
+    return out
+
+
+@pytest.mark.parametrize("T,pos,hq,hkv,d", SHAPES)
+def test_prefill_split(ctx, hip, T, pos, hq, hkv, d):
+    print(f"[prefill_split] T={T} pos={pos} hq={hq} hkv={hkv} d={d}", flush=True)
+    g = np.random.default_rng(T + pos)
+    cap = pos + T + 5
+    q = g.standard_normal((T, hq, d)).astype(np.float16).astype(np.float32) * 2
+    kc, vc = (g.standard_normal((hkv, cap, d)).astype(np.float16) for _ in range(2))
+    kc[:, pos + T:] = np.nan
+    vc[:, pos + T:] = np.nan
+    scale = float(np.float32(1.0) / np.sqrt(np.float32(d)))
+    want = _f64(q, kc, vc, pos, scale)
+    out = ctx.createBuffer(T * hq * d * 4)
+    args = hip.AttnArgs(ctx.from_numpy(q), ctx.from_numpy(kc), ctx.from_numpy(vc), hip.DTYPE_F16, out, pos, T, hq, hkv, d,
+                        cap, scale)
+    ctx.set_kernel_timing(True)
+    hip.gqaAttention(ctx, args)
+    assert ctx.kernel_time("prefill_merge_kernel")[0] == 1  # split, one merge
+    ctx.set_kernel_timing(False)
+    got = ctx.to_numpy(out, np.float32, (T, hq, d)).astype(np.float64)
+    err = np.abs(got - want).max()
+    cos = (got * want).sum() / np.sqrt((got ** 2).sum() * (want ** 2).sum())
+    print(f"  max-abs {err:.2e}, 1 - cosine {1 - cos:.2e}", flush=True)
+    assert err <= 2e-3 and cos >= 0.99999
+
+
+@pytest.mark.parametrize("kv", ["f16", "f32"])
+def test_split_noalloc_is_the_step(ctx, hip, kv):
+    T, pos, hq, hkv, d = 150, 3000, 64, 4, 128
+    cap = pos + T
+    g = np.random.default_rng(5)
+    q, k, v = (g.standard_normal((T, h, d)).astype(np.float32) for h in (hq, hkv, hkv))
+    dt = np.float16 if kv == "f16" else np.float32
+    kc, vc = (g.standard_normal((hkv, cap, d)).astype(dt) for _ in range(2))
+    qn, kn = (np.ones(d, np.float32) for _ in range(2))
+    outs = []
+    for fn in (hip.attentionStep, hip.attentionStepNoAlloc, hip.attentionStep):
+        bufs = [ctx.from_numpy(a) for a in (q, k, v, qn, kn, np.arange(pos, cap, dtype=np.int32), kc, vc)]
+        out = ctx.createBuffer(T * hq * d * 4)
+        fn(ctx, hip.AttentionStepArgs(*bufs, out, hip.DTYPE_F16 if kv == "f16" else hip.DTYPE_F32, pos, T, hq, hkv, d, cap,
+                                      1e-6, 1e6, 1.0, float(np.float32(d) ** np.float32(-0.5))))
+        outs.append(ctx.to_numpy(out, np.uint32, (T, hq, d)))
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
