@@ -871,7 +871,7 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(PrefillPara
 
 // The parts of a split launch: 256 threads take 1024 / D rows, a float4 column each, and fold
 // the row's parts in order.
-template <int D>
+template <int D, int B>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     constexpr int COLS = D / 4, ROWS = 256 / COLS;
     const uint64_t row = (uint64_t)blockIdx.x * ROWS + threadIdx.x / COLS;
@@ -881,27 +881,56 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     const uint32_t n = (p.pos + min(p.n_tokens, qt * kQRows + kQRows) + kKTile - 1) / kKTile;
     const float2* ml = p.part_ml + row * p.n_splits;
     const float* o = p.part_o + row * p.n_splits * D + c4;
-    auto used = [&](uint32_t s) { return split_first(n, s, p.n_splits) < split_first(n, s + 1, p.n_splits); };
+    // B parts' loads at a time: the fold waits on memory, not on bandwidth, when the rows are
+    // few (2 tokens at 8000, 10 parts: 7.1 us one by one, 5.4 by eights; 1000 tokens in 2
+    // parts: 9.5 by twos, 13 by eights). A part without a key tile of this row's q tile holds
+    // nothing; it is read and dropped.
+    auto part = [&](uint32_t s) { return min(s, p.n_splits - 1); };
+    auto used = [&](uint32_t s) {
+        return s < p.n_splits && split_first(n, s, p.n_splits) < split_first(n, s + 1, p.n_splits);
+    };
     float M = -INFINITY;
-    for (uint32_t s = 0; s < p.n_splits; s++)
-        if (used(s)) M = fmaxf(M, ml[s].x);
+    for (uint32_t s0 = 0; s0 < p.n_splits; s0 += B) {
+        float m[B];
+#pragma unroll
+        for (int u = 0; u < B; u++) m[u] = ml[part(s0 + u)].x;
+#pragma unroll
+        for (int u = 0; u < B; u++) M = used(s0 + u) ? fmaxf(M, m[u]) : M;
+    }
     float l = 0.0f;
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t s = 0; s < p.n_splits; s++)
-        if (used(s)) {
-            const float2 v = ml[s];
-            const float w = fast_exp2(v.x - M);
-            l += v.y * w;
-            acc += *(const f32x4*)(o + (uint64_t)s * D) * w;
+    for (uint32_t s0 = 0; s0 < p.n_splits; s0 += B) {
+        float2 v[B];
+        f32x4 ov[B];
+#pragma unroll
+        for (int u = 0; u < B; u++) {
+            v[u] = ml[part(s0 + u)];
+            ov[u] = *(const f32x4*)(o + (uint64_t)part(s0 + u) * D);
         }
+#pragma unroll
+        for (int u = 0; u < B; u++)
+            if (used(s0 + u)) {  // uniform over a row
+                const float w = fast_exp2(v[u].x - M);
+                l += v[u].y * w;
+                acc += ov[u] * w;
+            }
+    }
     *(f32x4*)(p.out + row * D + c4) = acc / l;
 }
 }  // namespace
 
-// Parts of a launch's key tiles. A workgroup's rounds are ~1800 cycles each and its prologue
-// and end ~20,000: parts of at least 12 rounds, and as many as CUs have no workgroup
-// otherwise (203 tokens at 6000, 64 q / 4 kv heads: 64 workgroups of 193 rounds, 140 us).
-constexpr uint32_t kSplitMinRounds = 12;
+// Parts of a launch's key tiles: as many as give each compute unit one workgroup (one fits a
+// unit), of at least 8 rounds (64 keys of a q tile, 0.72 us each; a workgroup's ends and the
+// merge cost ~7 us). Attention and merge, us,
+// unsplit and at the rule (q heads / kv heads 32 / 4, D 128 unless stated):
+//   203 tokens at 6000, 64 / 4   147 -> 57 + 7 (4 parts; 2 parts 84 + 5)
+//   203 tokens at 6000           142 -> 35 + 9 (8; 10 parts, more than units, 51 + 10)
+//   500 tokens at 1500            51 -> 27 + 8 (4)
+//   300 tokens at 3000, 16 / 2, D 64   59 -> 19 + 6 (8)
+//   700 tokens at 6000           172 -> 98 + 7 (2)
+// Splits of a launch that already has a workgroup per unit gain nothing (700 tokens at 2000,
+// 64 / 4: 81 unsplit, 74 to 84 at 2 to 16 parts without their merge).
+constexpr uint32_t kSplitMinRounds = 8;
 uint32_t prefill_splits(const ds5_hip_ctx* ctx, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads,
                         uint32_t head_dim) {
     const uint32_t qtiles = (n_tokens + kQRows - 1) / kQRows, pairs = (qtiles + 1) / 2;
@@ -936,8 +965,20 @@ int launch_kv_prep(ds5_hip_ctx* ctx, const KvPrepLaunch& a) {
 template <int D, int QM>
 static void launch_prefill_k(ds5_hip_ctx* ctx, const PrefillParams& p) {
     DS5_TIMED_LAUNCH(ctx, "prefill_attention_kernel", (prefill_attention_kernel<D, QM>), dim3(p.n_items, p.n_splits),
-                     dim3(kThreads),
-                     0, ctx->stream, p);
+                     dim3(kThreads), 0, ctx->stream, p);
+}
+
+template <int D>
+static void launch_merge(ds5_hip_ctx* ctx, const PrefillParams& p) {
+    const uint64_t per = 1024 / D, rows = (uint64_t)p.n_tokens * p.n_q_heads;
+    const dim3 grid((unsigned)((rows + per - 1) / per));
+    const char* name = "prefill_merge_kernel";
+    if (p.n_splits <= 2)
+        DS5_TIMED_LAUNCH(ctx, name, (prefill_merge_kernel<D, 2>), grid, dim3(256), 0, ctx->stream, p);
+    else if (p.n_splits <= 4)
+        DS5_TIMED_LAUNCH(ctx, name, (prefill_merge_kernel<D, 4>), grid, dim3(256), 0, ctx->stream, p);
+    else
+        DS5_TIMED_LAUNCH(ctx, name, (prefill_merge_kernel<D, 8>), grid, dim3(256), 0, ctx->stream, p);
 }
 
 int launch_prefill(ds5_hip_ctx* ctx, const PrefillLaunch& a) {
@@ -978,11 +1019,7 @@ int launch_prefill(ds5_hip_ctx* ctx, const PrefillLaunch& a) {
     }
     if (int rc = ds5_after_launch(ctx, "prefill_attention_kernel")) return rc;
     if (p.n_splits == 1) return DS5_OK;
-    const uint32_t per = 1024 / a.head_dim;
-    const dim3 grid((unsigned)((rows + per - 1) / per));
-    if (a.head_dim == 128)
-        DS5_TIMED_LAUNCH(ctx, "prefill_merge_kernel", prefill_merge_kernel<128>, grid, dim3(256), 0, ctx->stream, p);
-    else
-        DS5_TIMED_LAUNCH(ctx, "prefill_merge_kernel", prefill_merge_kernel<64>, grid, dim3(256), 0, ctx->stream, p);
+    if (a.head_dim == 128) launch_merge<128>(ctx, p);
+    else launch_merge<64>(ctx, p);
     return ds5_after_launch(ctx, "prefill_merge_kernel");
 }
