@@ -257,12 +257,18 @@ __global__ __launch_bounds__(kRouterThreads) void router_logits_kernel(const flo
 
 // Logits for many tokens (router_logits_tile_kernel): workgroup (16 RT tokens, 16 RT
 // experts) stages chunks of kRtK elements of x and of the expert rows (f16 widened
-// to f32 exactly) in LDS, transposed, two chunks in turn; thread (tx, ty) keeps the
-// RT x RT logits of tokens RT ty + a and experts RT tx + b, each dotRow's serial sum
-// (kernels_c.zig:40-68): the product rounded, then added, in element order. The
-// chains of the thread's logits interleave, so the adds' latency is covered; RT 2
-// shares each LDS read among more products, RT 1 gives four times the workgroups.
-constexpr uint32_t kRtK = 64;
+// to f32 exactly) in LDS, two chunks in turn; thread (tx, ty) keeps the RT x RT logits of
+// tokens ty + 16 a and experts tx + 16 b, each dotRow's serial sum (kernels_c.zig:40-68):
+// the product rounded, then added, in element order. A multiply and an add per product, 4
+// cycles each, are the work (27 us for 2048 tokens x 128 experts x 2048 on 256 CUs); a
+// SIMD has one wavefront, which therefore reads LDS a group of elements ahead, 16 bytes a
+// read, forms that group's products between the adds of the group before (one after the
+// other a product and its add wait 16 cycles, the chain alone 8), and loads the next chunk
+// while it sums one. 128 experts x 2048: 32 tokens 30.7 -> 17.8 us (the chain of adds alone
+// 7.5), 512 tokens 31 -> 19, 2048 tokens 66 -> 51; chunks of 64 elements waited for memory
+// in each one of them.
+// RT 2 shares each LDS read among more products, RT 1 gives four times the workgroups.
+constexpr uint32_t kRtK = 256;
 
 template <uint32_t DT>
 __device__ __forceinline__ f32x4 router_tile_w4(const uint8_t* row, uint32_t i) {
@@ -281,59 +287,73 @@ __global__ __launch_bounds__(256) void router_logits_tile_kernel(const float* __
                                                                  uint32_t dim, uint32_t n_tokens, uint32_t n_experts,
                                                                  float* __restrict__ logits) {
 #pragma clang fp contract(off)
-    constexpr uint32_t TR = 16 * RT, S = TR + 1;  // tile rows; LDS row stride (conflict-free transposed stores)
-    static_assert(kRtK == 64, "staging: 16 threads of float4s per row and chunk");
-    __shared__ float xs[2][kRtK * S], ws[2][kRtK * S];
+    // LDS row stride: 16 rows' reads of one 16-byte column meet all 64 banks once
+    constexpr uint32_t TR = 16 * RT, S = kRtK + 4;
+    constexpr int U = kRtK / 16 * RT / 4;  // staged rows per thread: a wavefront takes a row at a time
+    static_assert(kRtK == 256, "staging: 64 threads of float4s per row and chunk");
+    __shared__ __align__(16) float xs[2][TR * S], ws[2][TR * S];
     const uint32_t t0 = blockIdx.x * TR, e0 = blockIdx.y * TR;
     const uint32_t tid = threadIdx.x, tx = tid % 16, ty = tid / 16;
-    // staging unit s: tile row tid / 16 + 16 s, elements 4 (tid % 16) .. + 3 of the chunk
-    const uint32_t c4 = tid % 16;
-    const float* xr[RT];
-    const uint8_t* wr[RT];
-    f32x4 xv[RT], wv[RT];
+    // staging unit s: tile row tid / 64 + 4 s, elements 4 (tid % 64) .. + 3 of the chunk
+    const uint32_t c4 = tid % 64, r0 = tid / 64;
+    f32x4 xv[U], wv[U];
 #pragma unroll
-    for (int s = 0; s < RT; s++) {
-        const uint32_t r = tid / 16 + 16 * s;
-        xr[s] = x + (uint64_t)min(t0 + r, n_tokens - 1) * dim;
-        wr[s] = w + (uint64_t)min(e0 + r, n_experts - 1) * row_bytes;
-        xv[s] = wv[s] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
+    for (int s = 0; s < U; s++) xv[s] = wv[s] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     auto load = [&](uint32_t k0) {
         const uint32_t i = k0 + 4 * c4;
         if (i < dim) {  // dim % 4 == 0: the four elements are all inside
 #pragma unroll
-            for (int s = 0; s < RT; s++) {
-                xv[s] = *(const f32x4*)(xr[s] + i);
-                wv[s] = router_tile_w4<DT>(wr[s], i);
+            for (int s = 0; s < U; s++) {
+                xv[s] = *(const f32x4*)(x + (uint64_t)min(t0 + r0 + 4 * s, n_tokens - 1) * dim + i);
+                wv[s] = router_tile_w4<DT>(w + (uint64_t)min(e0 + r0 + 4 * s, n_experts - 1) * row_bytes, i);
             }
         }
     };
     auto store = [&](int b) {
 #pragma unroll
-        for (int s = 0; s < RT; s++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                xs[b][(4 * c4 + j) * S + tid / 16 + 16 * s] = xv[s][j];
-                ws[b][(4 * c4 + j) * S + tid / 16 + 16 * s] = wv[s][j];
-            }
+        for (int s = 0; s < U; s++) {
+            *(f32x4*)(xs[b] + (r0 + 4 * s) * S + 4 * c4) = xv[s];
+            *(f32x4*)(ws[b] + (r0 + 4 * s) * S + 4 * c4) = wv[s];
+        }
     };
     float acc[RT][RT];
 #pragma unroll
     for (int a = 0; a < RT; a++)
 #pragma unroll
         for (int b = 0; b < RT; b++) acc[a][b] = 0.0f;
-    auto step = [&](const float* xb, const float* wb) {
-        float xa[RT], wb_[RT];
-#pragma unroll
-        for (int a = 0; a < RT; a++) {
-            xa[a] = xb[a];
-            wb_[a] = wb[a];
-        }
-#pragma unroll
-        for (int a = 0; a < RT; a++)
-#pragma unroll
-            for (int b = 0; b < RT; b++) acc[a][b] += xa[a] * wb_[b];
+    constexpr int G = RT == 1 ? 8 : 2;  // float4 columns of a group
+    struct Cols {
+        f32x4 x[G][RT], w[G][RT];
     };
+    auto read = [&](Cols& v, const float* xb, const float* wb, uint32_t group) {
+        const uint32_t at = 4 * G * group;
+#pragma unroll
+        for (int g = 0; g < G; g++)
+#pragma unroll
+            for (int a = 0; a < RT; a++) {
+                v.x[g][a] = *(const f32x4*)(xb + 16 * a * S + at + 4 * g);
+                v.w[g][a] = *(const f32x4*)(wb + 16 * a * S + at + 4 * g);
+            }
+        __builtin_amdgcn_sched_barrier(0);  // the reads stay ahead of the sums
+    };
+    // A group's products are formed while the group before is added: an add waits for the
+    // add before it, and the multiply issues meanwhile.
+    float prod[4 * G][RT][RT];
+    auto each = [&](const Cols& v, auto add, auto mul) {
+#pragma unroll
+        for (int i = 0; i < 4 * G; i++) {
+#pragma unroll
+            for (int a = 0; a < RT; a++)
+#pragma unroll
+                for (int b = 0; b < RT; b++) {
+                    if constexpr (decltype(add)::value) acc[a][b] += prod[i][a][b];
+                    if constexpr (decltype(mul)::value) prod[i][a][b] = v.x[i / 4][a][i % 4] * v.w[i / 4][b][i % 4];
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
     load(0);
     store(0);
     __syncthreads();
@@ -341,14 +361,31 @@ __global__ __launch_bounds__(256) void router_logits_tile_kernel(const float* __
     for (uint32_t c = 0; c < nch; c++) {
         const int b = c & 1;
         if (c + 1 < nch) load((c + 1) * kRtK);
-        const float* xb = xs[b] + RT * ty;
-        const float* wb = ws[b] + RT * tx;
-        const uint32_t kc = min(kRtK, dim - c * kRtK);  // uniform
-        if (kc == kRtK) {
-#pragma unroll 16
-            for (uint32_t i = 0; i < kRtK; i++) step(xb + i * S, wb + i * S);
+        const float* xb = xs[b] + ty * S;
+        const float* wb = ws[b] + tx * S;
+        const uint32_t n4 = min(kRtK, dim - c * kRtK) / 4;  // uniform
+        if (n4 == kRtK / 4) {
+            constexpr uint32_t NG = kRtK / 4 / G;
+            static_assert(NG % 2 == 0, "groups in turn");
+            Cols v0, v1;
+            read(v0, xb, wb, 0);
+            each(v0, no, yes);
+            read(v0, xb, wb, 1);
+#pragma unroll 1
+            for (uint32_t g = 1; g < NG - 1; g += 2) {
+                read(v1, xb, wb, g + 1);
+                each(v0, yes, yes);
+                read(v0, xb, wb, g + 2);
+                each(v1, yes, yes);
+            }
+            each(v0, yes, yes);
+            each(v0, yes, no);
         } else {
-            for (uint32_t i = 0; i < kc; i++) step(xb + i * S, wb + i * S);
+            for (uint32_t i = 0; i < 4 * n4; i++)
+#pragma unroll
+                for (int a = 0; a < RT; a++)
+#pragma unroll
+                    for (int b2 = 0; b2 < RT; b2++) acc[a][b2] += xb[16 * a * S + i] * wb[16 * b2 * S + i];
         }
         if (c + 1 < nch) store(b ^ 1);  // the buffer read in chunk c - 1, before the last barrier
         __syncthreads();
@@ -357,7 +394,7 @@ __global__ __launch_bounds__(256) void router_logits_tile_kernel(const float* __
     for (int a = 0; a < RT; a++)
 #pragma unroll
         for (int b = 0; b < RT; b++) {
-            const uint32_t t = t0 + RT * ty + a, e = e0 + RT * tx + b;
+            const uint32_t t = t0 + ty + 16 * a, e = e0 + tx + 16 * b;
             if (t < n_tokens && e < n_experts) logits[(uint64_t)t * n_experts + e] = acc[a][b];
         }
 }
