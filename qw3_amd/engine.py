@@ -140,13 +140,16 @@ class Engine:
 
     def embed_row(self, tok: int) -> np.ndarray:
         """forward.zig:503-516: dequantise the token's Q8_0 (or f32) embedding row."""
-        hidden = self.cfg["hidden_dim"]
-        e = self.w.token_embd
+        return self.embed_rows([tok])[0]
+
+    def embed_rows(self, toks) -> np.ndarray:
+        """The tokens' embedding rows [n, hidden], each as embed_row gives it."""
+        e, n = self.w.token_embd, len(toks)
         if e.dtype != np.uint8:
-            return np.asarray(e[tok], np.float32)
-        blk = e[tok].reshape(hidden // 32, 34)
-        scale = blk[:, 0:2].copy().view(np.float16).astype(np.float32)
-        return (scale * blk[:, 2:].copy().view(np.int8).astype(np.float32)).reshape(hidden)
+            return np.asarray(e[toks], np.float32)
+        blk = e[toks].reshape(n, self.cfg["hidden_dim"] // 32, 34)
+        scale = blk[:, :, 0:2].copy().view(np.float16).astype(np.float32)
+        return (scale * blk[:, :, 2:].view(np.int8).astype(np.float32)).reshape(n, -1)
 
     def forward(self, tokens, want_logits: bool = True):
         """Runs tokens at positions pos..pos+n-1 through every layer; returns the logits
@@ -160,10 +163,11 @@ class Engine:
         if n > self.capacity or self.pos > self.capacity - n:
             raise ValueError("ContextOverflow")
         scale = float(np.float32(1.0) / np.sqrt(np.float32(hd)))
-        for i, tok in enumerate(tokens):
-            if tok >= vocab:
-                raise ValueError("TokenOutOfRange")
-            ctx.upload(self.x, i * hidden * 4, self.embed_row(int(tok)))
+        if any(tok >= vocab for tok in tokens):
+            raise ValueError("TokenOutOfRange")
+        # one copy for all rows: an upload waits for its copy (61 tokens of 1024, with the rows taken from the
+        # table one by one: 1.0 ms of 1.7)
+        ctx.upload(self.x, 0, self.embed_rows([int(tok) for tok in tokens]))
         self._trace(-1, "embed", self.x, n * hidden)
         ctx.upload(self.positions, 0, np.arange(self.pos, self.pos + n, dtype=np.int32))
 

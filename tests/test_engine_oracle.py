@@ -149,3 +149,26 @@ def test_trace_points_and_first_divergence(oracle, model):
     assert OE.first_divergence(clean, clean, cfg["n_layers"], 2e-3, 1e-2) is None
     layer, op, r = OE.first_divergence(clean, bad, cfg["n_layers"], 2e-3, 1e-2)
     assert (layer, op) == (1, "attn_resid") and not r.passed
+
+
+@pytest.mark.parametrize("kind", ["q8_0", "f32", "f16"])
+def test_embedding_rows_of_a_prompt(model, kind):
+    """The engine's rows of a whole prompt (one upload) equal the oracle's token by token, repeats and
+    the table's ends among them."""
+    from types import SimpleNamespace
+    from oracle import engine as O
+    from qw3_amd import engine as E
+    cfg, w, _ = model
+    eng = E.Engine.__new__(E.Engine)
+    table = w["token_embd.weight"]
+    if kind != "q8_0":
+        g = np.random.default_rng(1)
+        table = g.standard_normal((512, 256)).astype(np.float32 if kind == "f32" else np.float16)
+    eng.cfg, eng.w = cfg, SimpleNamespace(token_embd=table)
+    ref = O.Engine({**w, "token_embd.weight": table}, cfg, context_capacity=8)
+    for toks in ([0], [511, 0, 7, 7], list(range(100, 161))):
+        rows = eng.embed_rows(toks)
+        assert rows.dtype == np.float32 and rows.shape == (len(toks), 256)
+        for row, tok in zip(rows, toks):
+            assert np.array_equal(row, np.asarray(ref.embed_row(tok), np.float32))
+            assert np.array_equal(row, eng.embed_row(tok))
