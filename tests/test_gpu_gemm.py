@@ -83,3 +83,38 @@ def test_grouped_experts_few_pairs(ctx, hip, T, E, K, dim, ffn):
         runs.append(ctx.to_numpy(out, np.float32, (T, dim)))
     assert np.all(np.abs(runs[0] - want) <= lim), float(np.max(np.abs(runs[0] - want) / lim))
     assert np.array_equal(runs[0], runs[1])
+
+
+@pytest.mark.parametrize("T,E", [(1024, 16), (1025, 16), (3001, 24), (66000, 40)])
+def test_grouped_experts_sort_slices(ctx, hip, T, E):
+    """Pair counts at the edges of the sort's slices (1024 pairs each, then 64 of equal size), one
+    pair a token, half of them on one expert: every token's row against float64, twice."""
+    print(f"[moe] sort slices T={T} E={E}", flush=True)
+    dim, ffn = 256, 64
+    g = np.random.default_rng(T)
+    (G, Gf), (U, Uf), (D, Df) = (q8_rows(g, E * a, b) for a, b in ((ffn, dim), (ffn, dim), (dim, ffn)))
+    x = (0.05 * g.standard_normal((T, dim))).astype(np.float32)
+    pairs = np.zeros(T, hip.PAIR_DTYPE)
+    pairs["token"] = g.permutation(T)
+    pairs["expert"] = np.where(g.random(T) < 0.5, 3, g.integers(0, E, T))
+    pairs["weight"] = g.random(T).astype(np.float32)
+    bufs = [ctx.from_numpy(np.concatenate([v.reshape(-1), np.zeros(4, np.uint8)])) for v in (G, U, D)]
+    xb, runs = ctx.from_numpy(x), []
+    for _ in range(2):
+        out = ctx.from_numpy(np.zeros((T, dim), np.float32))
+        hip.expertMlpSwiglu(ctx, xb, *bufs, hip.DTYPE_Q8_0, pairs, out, T, dim, ffn, E)
+        runs.append(ctx.to_numpy(out, np.float32, (T, dim)))
+    assert np.array_equal(runs[0], runs[1])
+    for e in range(E):
+        p = pairs[pairs["expert"] == e]
+        tok, w = p["token"], p["weight"][:, None].astype(np.float64)
+        Ge, Ue, De = (v.reshape(E, -1, v.shape[1])[e] for v in (Gf, Uf, Df))
+        xd = x[tok].astype(np.float64)
+        a, u = xd @ Ge.T, xd @ Ue.T
+        da, du = bound(xd, Ge), bound(xd, Ue)
+        h = a / (1 + np.exp(-a)) * u
+        # the bound of test_grouped_experts_few_pairs
+        dh = 1.1 * da * np.abs(u) + np.abs(a) * du + 1.1 * da * du + 4 * 2.0 ** -23 * np.abs(h)
+        want = w * (h @ De.T)
+        lim = w * (bound(h, De) + (dh + 2.0 ** -21 * dh.max(1, keepdims=True)) @ np.abs(De).T) + 2.0 ** -20 * np.abs(want)
+        assert np.all(np.abs(runs[0][tok] - want) <= lim), float(np.max(np.abs(runs[0][tok] - want) / lim))
