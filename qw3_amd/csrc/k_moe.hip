@@ -1016,8 +1016,8 @@ int launch_router(ds5_hip_ctx* ctx, const RouterLaunch& a) {
 // What bounds it is the scatter, a cache line a lane: one workgroup took 27.6 us for 16384
 // pairs over 128 experts (5.2 for 192). So workgroup s of S scatters only its slice of the
 // pairs. Each counts all of them itself, those before its slice apart, where its rows of an
-// expert begin: S reads of the pairs from L2 and no meeting of workgroups: 9.6 us (192 pairs 5.2, as before),
-// the MoE call of 2048 tokens 722 -> 707.
+// expert begin: S reads of the pairs from L2 and no meeting of workgroups: 9.6 us (192 pairs
+// 5.2, as before), the MoE call of 2048 tokens 722 -> 707.
 constexpr int kSortThreads = 1024;
 constexpr int kSortBatch = 16;       // pairs per thread whose loads are in flight together
 constexpr uint32_t kSortSlice = 1024;  // pairs of a slice, while there are at most 64
