@@ -56,6 +56,16 @@ void ds5_index_gemm_q(uint32_t wave, uint32_t threads, uint32_t nq, uint32_t w_r
 uint32_t ds5_index_prefill_tile(uint32_t head_dim, int v, uint32_t key0, uint32_t kv_end, uint32_t* off);
 uint32_t ds5_index_pf_q_token(uint32_t q0, uint32_t row, uint32_t n_tokens);
 
+/* attn_f32_kernel: a launch's plan, out = [row tiles, positions per split, splits, 1 if a
+ * wavefront takes a row tile]; the first query row of a wavefront; a load's position; what a
+ * split writes of a row (0 nothing, 1 the output, 2 a partial result); a row's splits. */
+void ds5_index_attn_f32_plan(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads,
+                             uint32_t head_dim, uint32_t* out);
+uint32_t ds5_index_af_row0(uint32_t bx, uint32_t wave, int wave_rows);
+uint32_t ds5_index_af_load_pos(uint32_t p, uint32_t end);
+uint32_t ds5_index_af_store(uint32_t lim, uint32_t start, uint32_t chunk);
+uint32_t ds5_index_af_row_splits(uint32_t lim, uint32_t chunk);
+
 #ifdef __cplusplus
 }
 #endif

@@ -3,7 +3,7 @@
 // No reference counterpart; nothing here touches the device.
 #include <stdint.h>
 
-#include "ds5_index.hpp"
+#include "ds5_common.hpp"
 #include "ds5_index.h"
 
 extern "C" {
@@ -123,5 +123,22 @@ uint32_t ds5_index_prefill_tile(uint32_t head_dim, int v, uint32_t key0, uint32_
 uint32_t ds5_index_pf_q_token(uint32_t q0, uint32_t row, uint32_t n_tokens) {
     return ds5idx::pf_q_token(q0, row, n_tokens);
 }
+
+
+// The f32 attention: its plan, and the rows, positions and stores of a split.
+void ds5_index_attn_f32_plan(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads,
+                             uint32_t head_dim, uint32_t* out) {
+    const AttnF32Plan p = attn_f32_plan(cu_count, pos, n_tokens, n_q_heads, n_kv_heads, head_dim);
+    out[0] = p.row_tiles;
+    out[1] = p.chunk;
+    out[2] = p.n_splits;
+    out[3] = p.wave_rows;
+}
+uint32_t ds5_index_af_row0(uint32_t bx, uint32_t wave, int wave_rows) { return ds5idx::af_row0(bx, wave, wave_rows != 0); }
+uint32_t ds5_index_af_load_pos(uint32_t p, uint32_t end) { return ds5idx::af_load_pos(p, end); }
+uint32_t ds5_index_af_store(uint32_t lim, uint32_t start, uint32_t chunk) {
+    return (uint32_t)ds5idx::af_store(lim, start, chunk);
+}
+uint32_t ds5_index_af_row_splits(uint32_t lim, uint32_t chunk) { return ds5idx::af_row_splits(lim, chunk); }
 
 }  // extern "C"

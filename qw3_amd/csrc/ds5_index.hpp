@@ -9,7 +9,9 @@
 //   matmul_q8_mfma_kernel (k_matmul.hip): the lane offsets of the direct-to-LDS
 //     x-plane and raw Q8_0 row loads;
 //   prefill_attention_kernel (k_prefill.hip): the lane offsets of a K/V tile's
-//     direct-to-LDS loads and their clamp, and the staged q and output rows.
+//     direct-to-LDS loads and their clamp, and the staged q and output rows;
+//   attn_f32_kernel (k_attn_f32.hip): a wavefront's query rows, the clamped positions of
+//     its loads, and which split writes a row where.
 #pragma once
 
 #include <stdint.h>
@@ -40,6 +42,9 @@ constexpr uint32_t kDecMaxSplits = 64;
 constexpr int kPfHeads = 4, kPfQRows = 32, kPfKTile = 64;
 DS5_HDC int pf_rsk(int D) { return 2 * D + 16; }
 DS5_HDC int pf_rsv(int D) { return 2 * D + 64; }
+
+// attn_f32_kernel's shape: 16 query rows and 16 positions a tile, four wavefronts.
+constexpr int kAfRows = 16, kAfPos = 16, kAfWaves = 4;
 
 // Split-K geometry of a contiguous decode launch: positions per split (a multiple
 // of 128, at least max_len / 64; about four workgroups per CU unless decode_chunk
@@ -159,5 +164,24 @@ DS5_HD uint32_t pf_clamped_off(uint32_t off, uint32_t key0, uint32_t kv_end, int
 }
 // A q tile's row `row` (< 32) reads token min(q0 + row, n_tokens - 1).
 DS5_HD uint32_t pf_q_token(uint32_t q0, uint32_t row, uint32_t n_tokens) { return umin(q0 + row, n_tokens - 1); }
+
+// ---------------------------------------------------------------------------
+// attn_f32_kernel. Query rows R = t * group + head in the group; a wavefront (wave_rows) or
+// a workgroup takes the kAfRows rows from af_row0. Positions at or past a split's end re-read
+// the one before it.
+// ---------------------------------------------------------------------------
+DS5_HD uint32_t af_row0(uint32_t bx, uint32_t wave, bool wave_rows) {
+    return (wave_rows ? bx * kAfWaves + wave : bx) * kAfRows;
+}
+DS5_HD uint32_t af_load_pos(uint32_t p, uint32_t end) { return umin(p, end - 1); }
+// What the split of positions from `start` leaves of a row whose last position is lim: nothing
+// where the row ends before the split (tiles hold rows of several tokens, and the other rows
+// may go on), the output itself where the row has no other split, or a partial result.
+enum AfStore : int { kAfNone = 0, kAfOut = 1, kAfPart = 2 };
+DS5_HD int af_store(uint32_t lim, uint32_t start, uint32_t chunk) {
+    return lim < start ? kAfNone : lim < chunk ? kAfOut : kAfPart;
+}
+// The splits that hold a partial result of the row (1: its only split wrote the output).
+DS5_HD uint32_t af_row_splits(uint32_t lim, uint32_t chunk) { return lim / chunk + 1; }
 
 }  // namespace ds5idx

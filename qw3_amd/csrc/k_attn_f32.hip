@@ -30,8 +30,8 @@
 
 namespace {
 
-constexpr int kRows = 16, kPos = 16;  // query rows and positions of a tile
-constexpr int kWaves = 4;
+constexpr int kRows = ds5idx::kAfRows, kPos = ds5idx::kAfPos;  // query rows and positions of a tile
+constexpr int kWaves = ds5idx::kAfWaves;
 constexpr int kThreads = kWaves * 64;
 
 struct AttnF32Params {
@@ -59,12 +59,12 @@ struct Tile {
 // Rows at or past `end` re-read row end - 1: their scores are masked.
 template <int D>
 DS5_DEVICE_INLINE void load_tile(Tile<D>& t, const float* kb, const float* vb, uint32_t p0, uint32_t end, int c, int g) {
-    const float* kr = kb + (uint64_t)min(p0 + c, end - 1) * D + 4 * g;
+    const float* kr = kb + (uint64_t)ds5idx::af_load_pos(p0 + c, end) * D + 4 * g;
 #pragma unroll
     for (int j = 0; j < D / 16; j++) t.k[j] = *(const f32x4*)(kr + 16 * j);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const float* vr = vb + (uint64_t)min(p0 + 4 * g + i, end - 1) * D + 4 * c;
+        const float* vr = vb + (uint64_t)ds5idx::af_load_pos(p0 + 4 * g + i, end) * D + 4 * c;
 #pragma unroll
         for (int u = 0; u < D / 64; u++) t.v[i][u] = *(const f32x4*)(vr + 64 * u);
     }
@@ -78,7 +78,7 @@ __global__ __launch_bounds__(kThreads) void attn_f32_kernel(const AttnF32Params 
     const uint32_t n_rows = p.n_tokens * p.group, kvh = blockIdx.y;
     // the last row tiles (the longest contexts) first
     const uint32_t bx = gridDim.x - 1 - blockIdx.x;
-    const uint32_t R0 = (WS == 1 ? bx * kWaves + wave : bx) * kRows;
+    const uint32_t R0 = ds5idx::af_row0(bx, wave, WS == 1);
     if (R0 >= n_rows) return;  // WS 1: wave-uniform, no barrier follows; WS 4: never
     const uint32_t R = min(R0 + c, n_rows - 1), t = R / p.group;
     const uint64_t row = (uint64_t)t * p.n_q_heads + kvh * p.group + R % p.group;
@@ -205,9 +205,10 @@ __global__ __launch_bounds__(kThreads) void attn_f32_kernel(const AttnF32Params 
     // O[u][e][k] of lane (c, g): row c, dim 64 u + 16 g + 4 k + e
     if constexpr (WS == 1) {
         if (R0 + c < n_rows) {
-            const bool single = lim < p.chunk;  // the row's only split: the output itself
+            const int to = ds5idx::af_store(lim, start, p.chunk);
+            const bool single = to == ds5idx::kAfOut;
             float* dst = single ? p.out + row * D : p.part_o + (row * p.n_splits + blockIdx.z) * D;
-            if (single || lim >= start) {
+            if (to != ds5idx::kAfNone) {
                 const float den = single ? l : 1.0f;
 #pragma unroll
                 for (int u = 0; u < NU; u++)
@@ -237,7 +238,8 @@ __global__ __launch_bounds__(kThreads) void attn_f32_kernel(const AttnF32Params 
             if (Rr >= n_rows) break;
             const uint32_t tr = Rr / p.group;
             const uint64_t orow = (uint64_t)tr * p.n_q_heads + kvh * p.group + Rr % p.group;
-            if (p.pos + tr < start) continue;  // the row ends before this split
+            const int to = ds5idx::af_store(p.pos + tr, start, p.chunk);
+            if (to == ds5idx::kAfNone) continue;
             float M = s_m[0][r];
 #pragma unroll
             for (int w = 1; w < kWaves; w++) M = fmaxf(M, s_m[w][r]);
@@ -251,7 +253,7 @@ __global__ __launch_bounds__(kThreads) void attn_f32_kernel(const AttnF32Params 
                 acc += *(const f32x4*)&s_o[w][r * OROW + d0] * f;
                 lt += s_l[w][r] * f;
             }
-            if (p.pos + tr < p.chunk) {
+            if (to == ds5idx::kAfOut) {
                 *(f32x4*)(p.out + orow * D + d0) = acc / lt;
             } else {
                 *(f32x4*)(p.part_o + (orow * p.n_splits + blockIdx.z) * D + d0) = acc;
@@ -270,7 +272,7 @@ __global__ __launch_bounds__(256) void attn_f32_merge_kernel(const AttnF32Params
     __shared__ float2 s_ml[SLOTS];
     const uint64_t row = blockIdx.x;
     const uint32_t t = (uint32_t)(row / p.n_q_heads);
-    const uint32_t ns = (p.pos + t) / p.chunk + 1;
+    const uint32_t ns = ds5idx::af_row_splits(p.pos + t, p.chunk);
     if (ns <= 1) return;  // written by its split
     const int col = threadIdx.x % COLS, slot = threadIdx.x / COLS;
     const float2* ml_row = (const float2*)p.part_ml + row * p.n_splits;

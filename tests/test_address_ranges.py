@@ -43,6 +43,9 @@ def ix(hip):
         "ds5_index_gemm_x": ([u32] * 7 + [P], None), "ds5_index_gemm_q": ([u32] * 8 + [P] * 4, None),
         "ds5_index_gemm_x_rows": ([u32] * 7 + [P, P], None),
         "ds5_index_prefill_tile": ([u32, C.c_int, u32, u32, P], u32), "ds5_index_pf_q_token": ([u32] * 3, u32),
+        "ds5_index_attn_f32_plan": ([u32] * 6 + [P], None), "ds5_index_af_row0": ([u32, u32, C.c_int], u32),
+        "ds5_index_af_load_pos": ([u32] * 2, u32), "ds5_index_af_store": ([u32] * 3, u32),
+        "ds5_index_af_row_splits": ([u32] * 2, u32),
     }
     for name, (a, r) in sig.items():
         f = getattr(lib, name)
@@ -62,7 +65,7 @@ def test_index_header_symbols_exported(hip):
     """Every function include/ds5_index.h declares is exported by the library."""
     text = open(os.path.join(ROOT, "include", "ds5_index.h")).read()
     names = set(re.findall(r"^\s*(?:void|uint32_t|uint64_t)\s+(ds5_index_\w+)\(", text, re.M))
-    assert len(names) == 17
+    assert len(names) == 22
     for n in names:
         assert getattr(hip.LIB, n) is not None
 
@@ -485,3 +488,54 @@ def check_prefill(ix, pos, T, hq, hkv, D, max_ctx):
 def test_prefill_dma_addresses(ix, pos, T, hq, hkv, D, cap):
     """C2 and the GPU parity suite's prefill shapes (chunked continuations, odd q-tile counts)."""
     assert check_prefill(ix, pos, T, hq, hkv, D, cap) > 0
+
+
+# ---------------------------------------------------------------------------
+# attn_f32_kernel (k_attn_f32.hip)
+# ---------------------------------------------------------------------------
+ROWS, TILE, WAVES = 16, 16, 4
+NONE, OUT, PART = 0, 1, 2
+
+
+@pytest.mark.parametrize("pos,T,hq,hkv,D", [
+    (0, 1, 32, 4, 128), (2999, 1, 32, 4, 128), (9000, 1, 16, 1, 64), (127, 2, 32, 4, 128), (1000, 5, 6, 2, 64),
+    (0, 500, 32, 4, 128), (7, 300, 32, 4, 128), (1, 290, 32, 4, 64), (5, 700, 12, 4, 128), (63, 400, 24, 8, 64),
+    (130, 260, 48, 2, 128), (3, 2100, 4, 2, 64), (0, 33, 32, 4, 128), (8000, 250, 64, 4, 128),
+])
+@pytest.mark.parametrize("planned", [True, False])
+def test_attn_f32_positions_and_stores(ix, pos, T, hq, hkv, D, planned):
+    """Every workgroup, wavefront and split of a launch: loads stay inside the positions the
+    rows attend, each row is written to the output once, by its only split, or leaves one
+    partial result in each of the splits that the merge folds. planned False: the one split
+    of a launch without room for partial results."""
+    plan = _u32s(4)
+    ix.ds5_index_attn_f32_plan(256, pos, T, hq, hkv, D, _ptr(plan))
+    row_tiles, chunk, n_splits, wave_rows = (int(v) for v in plan)
+    if not planned:
+        chunk, n_splits = U32 - 1, 1
+    group, L = hq // hkv, pos + T
+    n_rows = T * group
+    assert row_tiles * ROWS >= n_rows and chunk * n_splits >= L and n_splits <= 64
+    out, part = np.zeros(n_rows, int), np.zeros((n_rows, n_splits), int)
+    waves = range(WAVES) if wave_rows else [0]
+    for z in range(n_splits):
+        start = z * chunk
+        for bx in range(-(-row_tiles // WAVES) if wave_rows else row_tiles):
+            for w in waves:
+                R0 = ix.ds5_index_af_row0(bx, w, wave_rows)
+                if R0 >= n_rows:
+                    continue
+                last_lim = pos + (min(R0 + ROWS, n_rows) - 1) // group
+                if start > last_lim:
+                    continue
+                end = min(start + chunk, last_lim + 1)
+                for p0 in (start, start + (end - start - 1) // TILE * TILE):  # the first and the last tile
+                    seen = [ix.ds5_index_af_load_pos(p, end) for p in range(p0, p0 + TILE)]
+                    assert min(seen) >= start and max(seen) < min(end, L)
+                for R in range(R0, min(R0 + ROWS, n_rows)):
+                    to = ix.ds5_index_af_store(pos + R // group, start, chunk)
+                    out[R] += to == OUT
+                    part[R, z] += to == PART
+    splits = np.array([ix.ds5_index_af_row_splits(pos + R // group, chunk) for R in range(n_rows)])
+    assert np.array_equal(out, (splits == 1).astype(int))
+    assert np.array_equal(part, ((np.arange(n_splits)[None] < splits[:, None]) & (splits[:, None] > 1)).astype(int))

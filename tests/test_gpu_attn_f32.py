@@ -43,6 +43,8 @@ SHAPES = [  # T, pos, hq, hkv, d
     (1, 0, 32, 4, 128), (1, 15, 32, 4, 128), (1, 16, 4, 2, 64), (1, 63, 64, 4, 128), (1, 64, 32, 4, 128),
     (1, 65, 8, 8, 64), (1, 2999, 32, 4, 128), (1, 9000, 16, 1, 64), (2, 127, 32, 4, 128), (5, 1000, 6, 2, 64),
     (17, 0, 4, 2, 64), (16, 48, 48, 2, 128), (33, 7, 32, 4, 128), (260, 0, 32, 4, 64), (150, 300, 64, 4, 128),
+    # a wavefront per row tile, the tiles' tokens on both sides of a split's first position
+    (300, 7, 32, 4, 128), (290, 1, 32, 4, 64), (700, 5, 12, 4, 128), (400, 63, 24, 8, 64),
 ]
 
 
