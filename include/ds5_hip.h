@@ -58,8 +58,8 @@ typedef struct ds5_hip_ctx ds5_hip_ctx;
  * ======================================================================== */
 
 /* Ctx.init (metal.zig:131, ctx.zig:20): picks device `device_index`
- * (0 for the first visible GPU) and creates the context's stream and
- * timing events. */
+ * (0 for the first visible GPU) and creates the context's stream, timing
+ * events and the 32 MiB that attention launches split over their keys use. */
 int ds5_hip_init(int device_index, ds5_hip_ctx** out);
 
 /* Ctx.deinit (ctx.zig:26-30): waits for the stream, frees every buffer the
@@ -194,9 +194,11 @@ int ds5_hip_kv_append(ds5_hip_ctx* ctx, const ds5_kv_append_args* args);
  * kernels/gpu/kernels.zig:254-286). n_tokens == 1 runs the split-K
  * flash-decoding kernels, n_tokens > 1 the causal MFMA prefill kernel
  * (f16 cache, head_dim 64 or 128), f32 caches of head_dim 64 or 128 the f32
- * matrix-core kernel (one or many tokens; split over positions, and merged, where
- * the context workspace has or may get room for the partials, else one split);
- * other shapes run a generic streaming kernel. All paths are device code. */
+ * matrix-core kernel (one or many tokens); other shapes run a generic streaming
+ * kernel. All paths are device code. Prefill and f32 launches that would leave
+ * compute units idle split their positions and merge the parts: by the shape alone,
+ * so a captured call gives the eager call's bits (the parts lie in the context's own
+ * 32 MiB, allocated at init; a context without it runs them unsplit). */
 typedef struct ds5_attn_args {
     ds5_buf q;       /* f32 [n_tokens, n_q_heads, head_dim], post-norm post-rope */
     ds5_buf k_cache; /* kv_dtype [n_kv_heads, max_ctx, head_dim] */
@@ -461,8 +463,7 @@ int ds5_hip_attention_block(ds5_hip_ctx* ctx, const ds5_attention_block_args* ar
  * hipMalloc): ds5_hip_attention_step with the same kernels, arguments,
  * preconditions and results, but the split-K partials (decode) or the rope table
  * (prefill) live in the library's static device scratch array of
- * DS5_NOALLOC_SCRATCH_BYTES per GPU instead of the context's workspace (partials of
- * a prefill split over its keys in a second array of 32 MiB, their upper limit), and
+ * DS5_NOALLOC_SCRATCH_BYTES per GPU instead of the context's workspace, and
  * the call allocates nothing. A call that would need more scratch than that
  * (e.g. a long prefill) fails with ShapeMismatch before any device work.
  * Every call on one GPU shares that GPU's array: calls that overlap on one

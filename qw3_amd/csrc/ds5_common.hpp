@@ -64,8 +64,12 @@ struct ds5_hip_ctx {
     // comes from there and nothing is allocated.
     void* scratch = nullptr;
     size_t scratch_bytes = 0;
-    void* split_scratch = nullptr;  // kSplitBytesMax bytes, for the same calls' partial results
     bool use_scratch = false;
+    // kSplitBytesMax bytes for the partial results of an attention launch split over its keys
+    // (prefill, f32 caches), allocated at init: whether a call splits then depends on its shape
+    // alone, captured or not, whatever ran before it. Null if there was no memory for it: such
+    // a context runs those launches unsplit.
+    void* split_buf = nullptr;
     // Decode tuning: positions per split-K workgroup (0 = heuristic); paged
     // plan: workgroups per launch the plan aims at (0 = two per CU).
     uint32_t decode_chunk = 0;
@@ -98,13 +102,7 @@ int ds5_fail(ds5_hip_ctx* ctx, int code, const char* fmt, ...) __attribute__((fo
 int ds5_hip_status(ds5_hip_ctx* ctx, hipError_t err, const char* what);
 int ds5_after_launch(ds5_hip_ctx* ctx, const char* what);
 int ds5_workspace(ds5_hip_ctx* ctx, size_t bytes, void** out);
-// Workspace for a launch that splits its work: `base` bytes that it needs anyway and `part`
-// (at most kSplitBytesMax) for partial results. False, with no error left behind, where a
-// stream capture would have to allocate or memory is out: the launch then runs unsplit. The
-// allocation-free entry point has a static array for the partials beside its scratch, so
-// that it splits as the allocating one does.
 constexpr size_t kSplitBytesMax = 32u << 20;
-bool ds5_split_workspace(ds5_hip_ctx* ctx, size_t base, size_t part, void** base_out, void** part_out);
 // The most splits of `rows` rows of partials that kSplitBytesMax holds.
 inline uint32_t ds5_max_splits(uint64_t rows, uint32_t head_dim) {
     const uint64_t row = rows * (head_dim + 2) * sizeof(float);
@@ -364,7 +362,6 @@ struct AttnF32Plan {
 };
 AttnF32Plan attn_f32_plan(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads,
                           uint32_t head_dim);
-size_t attn_f32_workspace_bytes(uint32_t n_tokens, uint32_t n_q_heads, uint32_t head_dim, uint32_t n_splits);
 int launch_attn_f32(ds5_hip_ctx* ctx, const GenericAttnLaunch& a);
 
 // Split-K MFMA decode (one query token per sequence), f16 cache, head_dim 64
@@ -417,15 +414,12 @@ struct PrefillLaunch {
     const f16* v_cache;
     float* out;
     uint32_t pos, n_tokens, n_q_heads, n_kv_heads, head_dim, max_ctx;
-    // the keys split over n_splits workgroups (prefill_splits; 0 or 1: not split), with
-    // prefill_part_bytes of partial results
-    uint32_t n_splits;
-    float* part;
 };
 int launch_prefill(ds5_hip_ctx* ctx, const PrefillLaunch& a);
-uint32_t prefill_splits(const ds5_hip_ctx* ctx, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads,
+// The parts that a launch's keys are split into, their partial results in the context's split
+// buffer (1: not split).
+uint32_t prefill_splits(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads,
                         uint32_t head_dim);
-size_t prefill_part_bytes(uint32_t n_tokens, uint32_t n_q_heads, uint32_t head_dim, uint32_t n_splits);
 
 int launch_fill_normal_f16(ds5_hip_ctx* ctx, f16* out, uint64_t n, uint64_t seed);
 int launch_stream_read(ds5_hip_ctx* ctx, const void* src, uint64_t len, uint32_t* sink);

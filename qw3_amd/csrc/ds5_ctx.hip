@@ -76,29 +76,6 @@ int ds5_workspace(ds5_hip_ctx* ctx, size_t bytes, void** out) {
     return DS5_OK;
 }
 
-bool ds5_split_workspace(ds5_hip_ctx* ctx, size_t base, size_t part, void** base_out, void** part_out) {
-    if (ctx->use_scratch) {
-        *base_out = ctx->scratch;
-        *part_out = ctx->split_scratch;
-        return base <= ctx->scratch_bytes && part <= kSplitBytesMax;
-    }
-    const size_t at = (base + 255) & ~(size_t)255, bytes = at + part;
-    if (bytes > ctx->workspace_bytes) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return false;
-        const std::string before = ctx->last_error;
-        void* ws = nullptr;
-        if (ds5_workspace(ctx, bytes, &ws)) {
-            (void)hipGetLastError();
-            ctx->last_error = before;
-            return false;
-        }
-    }
-    *base_out = ctx->workspace;
-    *part_out = (char*)ctx->workspace + at;
-    return true;
-}
-
 int ds5_aux_workspace(ds5_hip_ctx* ctx, size_t bytes, void** out) {
     if (int rc = grow_buffer(ctx, bytes, ctx->aux, ctx->aux_bytes, "workspace")) return rc;
     *out = ctx->aux;
@@ -153,6 +130,10 @@ int ds5_hip_init(int device_index, ds5_hip_ctx** out) {
     if (!rc) rc = ds5_hip_status(ctx, hipEventCreate(&ctx->ev_begin), "hipEventCreate");
     if (!rc) rc = ds5_hip_status(ctx, hipEventCreate(&ctx->ev_end), "hipEventCreate");
     if (!rc) rc = ds5_scratch_init(ctx);
+    if (!rc && hipMalloc(&ctx->split_buf, kSplitBytesMax) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->split_buf = nullptr;
+    }
     if (rc) {
         ds5_hip_deinit(ctx);
         return rc;
@@ -173,6 +154,7 @@ void ds5_hip_deinit(ds5_hip_ctx* ctx) {
     for (hipEvent_t e : ctx->marks) (void)hipEventDestroy(e);
     if (ctx->workspace) (void)hipFree(ctx->workspace);
     if (ctx->aux) (void)hipFree(ctx->aux);
+    if (ctx->split_buf) (void)hipFree(ctx->split_buf);
     if (ctx->ev_begin) (void)hipEventDestroy(ctx->ev_begin);
     if (ctx->ev_end) (void)hipEventDestroy(ctx->ev_end);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);

@@ -24,26 +24,23 @@
 // address.
 // ---------------------------------------------------------------------------
 static __device__ __align__(256) unsigned char scratch[DS5_NOALLOC_SCRATCH_BYTES];
-static __device__ __align__(256) unsigned char split_scratch[kSplitBytesMax];
 
 int ds5_scratch_init(ds5_hip_ctx* ctx) {
     static std::mutex mu;
-    static std::map<int, std::pair<void*, void*>> per_device;  // device index -> the two arrays' addresses there
+    static std::map<int, void*> per_device;  // device index -> address of `scratch` there
     std::lock_guard<std::mutex> lock(mu);
     auto it = per_device.find(ctx->device);
     if (it == per_device.end()) {
-        void *ptr = nullptr, *split = nullptr;
-        hipError_t err = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-        if (err == hipSuccess) err = hipGetSymbolAddress(&split, HIP_SYMBOL(split_scratch));
-        if (err != hipSuccess || !ptr || !split) {
+        void* ptr = nullptr;
+        const hipError_t err = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
+        if (err != hipSuccess || !ptr) {
             (void)hipGetLastError();  // do not leave the error for a later launch check
             return ds5_fail(ctx, DS5_DEVICE_FAILURE, "hipGetSymbolAddress(scratch) on device %d: %s", ctx->device,
                             hipGetErrorString(err));
         }
-        it = per_device.emplace(ctx->device, std::make_pair(ptr, split)).first;
+        it = per_device.emplace(ctx->device, ptr).first;
     }
-    ctx->scratch = it->second.first;
-    ctx->split_scratch = it->second.second;
+    ctx->scratch = it->second;
     ctx->scratch_bytes = DS5_NOALLOC_SCRATCH_BYTES;
     return DS5_OK;
 }
@@ -650,13 +647,6 @@ int ds5_hip_gqa_attention(ds5_hip_ctx* ctx, const ds5_attn_args* a) {
         l.n_kv_heads = a->n_kv_heads;
         l.head_dim = a->head_dim;
         l.max_ctx = a->max_ctx;
-        l.n_splits = prefill_splits(ctx, l.pos, l.n_tokens, l.n_q_heads, l.n_kv_heads, l.head_dim);
-        void *ws = nullptr, *part = nullptr;
-        if (l.n_splits > 1 && ds5_split_workspace(ctx, 0, prefill_part_bytes(l.n_tokens, l.n_q_heads, l.head_dim, l.n_splits),
-                                                  &ws, &part))
-            l.part = (float*)part;
-        else
-            l.n_splits = 1;
         return launch_prefill(ctx, l);
     }
     GenericAttnLaunch g{(const float*)ds5_ptr(a->q), ds5_ptr(a->k_cache), ds5_ptr(a->v_cache), (float*)ds5_ptr(a->out),
@@ -738,14 +728,8 @@ int ds5_hip_attention_step(ds5_hip_ctx* ctx, const ds5_attention_step_args* a) {
         if (prefill_step_fused(a)) {
             // the pre-pass's rope cos/sin table [n_tokens, head_dim] in the workspace;
             // the attention kernel normalises, rotates and scales q itself
-            void *ws = nullptr, *part = nullptr;
-            uint32_t splits = prefill_splits(ctx, a->pos, a->n_tokens, a->n_q_heads, a->n_kv_heads, a->head_dim);
-            const size_t base = prefill_step_workspace_bytes(T, hd);
-            if (splits < 2 || !ds5_split_workspace(ctx, base, prefill_part_bytes(a->n_tokens, a->n_q_heads, a->head_dim, splits),
-                                                   &ws, &part)) {
-                splits = 1;
-                if (int rc = ds5_workspace(ctx, base, &ws)) return rc;
-            }
+            void* ws = nullptr;
+            if (int rc = ds5_workspace(ctx, prefill_step_workspace_bytes(T, hd), &ws)) return rc;
             KvPrepLaunch kp{};
             kp.k = (const float*)ds5_ptr(a->k);
             kp.v = (const float*)ds5_ptr(a->v);
@@ -778,8 +762,6 @@ int ds5_hip_attention_step(ds5_hip_ctx* ctx, const ds5_attention_step_args* a) {
             l.n_kv_heads = a->n_kv_heads;
             l.head_dim = a->head_dim;
             l.max_ctx = a->max_ctx;
-            l.n_splits = splits;
-            l.part = (float*)part;
             return launch_prefill(ctx, l);
         }
     }
@@ -906,13 +888,8 @@ int ds5_hip_attention_block(ds5_hip_ctx* ctx, const ds5_attention_block_args* a)
     const uint64_t T = s.n_tokens;
     const size_t q16_bytes = (size_t)T * s.n_q_heads * hd * sizeof(uint16_t);
     const size_t prep_bytes = qkv_prep_workspace_bytes(s.n_tokens, a->hidden, hd);
-    void *ws = nullptr, *part = nullptr;
-    uint32_t splits = prefill_splits(ctx, s.pos, s.n_tokens, s.n_q_heads, s.n_kv_heads, hd);
-    if (splits < 2 || !ds5_split_workspace(ctx, q16_bytes + prep_bytes, prefill_part_bytes(s.n_tokens, s.n_q_heads, hd, splits),
-                                           &ws, &part)) {
-        splits = 1;
-        if (int rc = ds5_workspace(ctx, q16_bytes + prep_bytes, &ws)) return rc;
-    }
+    void* ws = nullptr;
+    if (int rc = ds5_workspace(ctx, q16_bytes + prep_bytes, &ws)) return rc;
     QkvPrepLaunch qp{};
     qp.x = (const float*)ds5_ptr(a->x);
     qp.wq = (const uint8_t*)ds5_ptr(a->wq);
@@ -951,8 +928,6 @@ int ds5_hip_attention_block(ds5_hip_ctx* ctx, const ds5_attention_block_args* a)
     l.n_kv_heads = s.n_kv_heads;
     l.head_dim = hd;
     l.max_ctx = s.max_ctx;
-    l.n_splits = splits;
-    l.part = (float*)part;
     return launch_prefill(ctx, l);
 }
 

@@ -356,18 +356,10 @@ AttnF32Plan attn_f32_plan(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, ui
     return pl;
 }
 
-size_t attn_f32_workspace_bytes(uint32_t n_tokens, uint32_t n_q_heads, uint32_t head_dim, uint32_t n_splits) {
-    return n_splits > 1 ? (size_t)n_tokens * n_q_heads * n_splits * (head_dim + 2) * sizeof(float) : 0;
-}
-
 int launch_attn_f32(ds5_hip_ctx* ctx, const GenericAttnLaunch& a) {
     if (a.n_tokens == 0) return DS5_OK;
     AttnF32Plan plan = attn_f32_plan(ctx->cu_count, a.pos, a.n_tokens, a.n_q_heads, a.n_kv_heads, a.head_dim);
-    void *ws = nullptr, *base = nullptr;
-    if (plan.n_splits > 1 &&
-        !ds5_split_workspace(ctx, 0, attn_f32_workspace_bytes(a.n_tokens, a.n_q_heads, a.head_dim, plan.n_splits), &base,
-                             &ws)) {
-        // no room (a capture that may not allocate): one split needs none
+    if (plan.n_splits > 1 && !ctx->split_buf) {  // one split needs no partials
         plan.n_splits = 1;
         plan.chunk = 0xffffffffu;
     }
@@ -376,8 +368,10 @@ int launch_attn_f32(ds5_hip_ctx* ctx, const GenericAttnLaunch& a) {
     p.k_cache = (const float*)a.k_cache;
     p.v_cache = (const float*)a.v_cache;
     p.out = a.out;
-    p.part_o = (float*)ws;
-    p.part_ml = p.part_o ? p.part_o + (size_t)a.n_tokens * a.n_q_heads * plan.n_splits * a.head_dim : nullptr;
+    if (plan.n_splits > 1) {
+        p.part_o = (float*)ctx->split_buf;
+        p.part_ml = p.part_o + (size_t)a.n_tokens * a.n_q_heads * plan.n_splits * a.head_dim;
+    }
     p.pos = a.pos;
     p.n_tokens = a.n_tokens;
     p.n_q_heads = a.n_q_heads;

@@ -931,20 +931,16 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
 // Splits of a launch that already has a workgroup per unit gain nothing (700 tokens at 2000,
 // 64 / 4: 81 unsplit, 74 to 84 at 2 to 16 parts without their merge).
 constexpr uint32_t kSplitMinRounds = 8;
-uint32_t prefill_splits(const ds5_hip_ctx* ctx, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads,
+uint32_t prefill_splits(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads,
                         uint32_t head_dim) {
     const uint32_t qtiles = (n_tokens + kQRows - 1) / kQRows, pairs = (qtiles + 1) / 2;
     const uint32_t hgroups = (n_q_heads / n_kv_heads + kHeads - 1) / kHeads;
-    const uint64_t wgs = (uint64_t)n_kv_heads * hgroups * pairs, cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    const uint64_t wgs = (uint64_t)n_kv_heads * hgroups * pairs, cu = cu_count ? cu_count : 256;
     const uint64_t tiles = ((uint64_t)pos + n_tokens + kKTile - 1) / kKTile;
     const uint64_t rounds = qtiles > 1 ? tiles + (pos + kQRows + kKTile - 1) / kKTile : tiles;
     const uint64_t s = std::min<uint64_t>({cu / std::max<uint64_t>(wgs, 1), rounds / kSplitMinRounds, tiles / 2,
                                            (uint64_t)ds5_max_splits((uint64_t)n_tokens * n_q_heads, head_dim)});
     return (uint32_t)std::max<uint64_t>(s, 1);
-}
-
-size_t prefill_part_bytes(uint32_t n_tokens, uint32_t n_q_heads, uint32_t head_dim, uint32_t n_splits) {
-    return n_splits > 1 ? (size_t)n_tokens * n_q_heads * n_splits * (head_dim + 2) * sizeof(float) : 0;
 }
 
 bool prefill_prep_supported(uint32_t n_kv_heads, uint32_t head_dim) {
@@ -1003,10 +999,11 @@ int launch_prefill(ds5_hip_ctx* ctx, const PrefillLaunch& a) {
     p.n_hgroups = (p.group + kHeads - 1) / kHeads;
     p.n_items = a.n_kv_heads * p.n_hgroups * p.n_pairs;
     p.items_per_xcd = p.n_items % 8 == 0 ? p.n_items / 8 : 0;
-    p.n_splits = std::max(a.n_splits, 1u);
-    const uint64_t rows = (uint64_t)a.n_tokens * a.n_q_heads;
-    p.part_o = a.part;
-    p.part_ml = p.n_splits > 1 ? (float2*)(a.part + rows * p.n_splits * a.head_dim) : nullptr;
+    p.n_splits = ctx->split_buf ? prefill_splits(ctx->cu_count, a.pos, a.n_tokens, a.n_q_heads, a.n_kv_heads, a.head_dim) : 1;
+    if (p.n_splits > 1) {
+        p.part_o = (float*)ctx->split_buf;
+        p.part_ml = (float2*)(p.part_o + (uint64_t)a.n_tokens * a.n_q_heads * p.n_splits * a.head_dim);
+    }
     const int qm = a.q16 ? kQOperand : a.cs ? kQRaw : kQRotated;
     if (a.head_dim == 128) {
         if (qm == kQOperand) launch_prefill_k<128, kQOperand>(ctx, p);

@@ -129,24 +129,27 @@ def test_step_equals_its_ops(ctx, hip, kv, T, pos, hq, hkv, d):
         assert np.array_equal(a, c)
 
 
-def test_f32_capture_before_any_call_needs_no_workspace(hip):
-    """A split launch captured on a fresh context (no workspace yet) runs as one split, and
-    the graph's replays equal each other and float64."""
+def test_f32_capture_before_any_call(hip):
+    """A split launch captured on a fresh context: the graph's replays give float64's outputs
+    and the eager call's bits."""
     print("[attn_f32] capture on a fresh context", flush=True)
     T, pos, hq, hkv, d = 1, 700, 32, 4, 128
     q, kc, vc = _inputs(T, pos, hq, hkv, d, pos + T)
     scale = float(np.float32(1.0) / np.sqrt(np.float32(d)))
     c = hip.Ctx.init(0)
     try:
-        out = c.createBuffer(T * hq * d * 4)
-        args = hip.AttnArgs(c.from_numpy(q), c.from_numpy(kc), c.from_numpy(vc), hip.DTYPE_F32, out, pos, T, hq, hkv, d,
-                            pos + T, scale)
+        out, eager = (c.createBuffer(T * hq * d * 4) for _ in range(2))
+        bufs = [c.from_numpy(a) for a in (q, kc, vc)]
+        args, eager_args = (hip.AttnArgs(*bufs, hip.DTYPE_F32, o, pos, T, hq, hkv, d, pos + T, scale) for o in (out, eager))
         graph = c.capture(lambda: hip.gqaAttention(c, args))
         want, bound = _f64(q, kc, vc, pos, scale)
         for _ in range(3):
             c.zero(out, T * hq * d * 4)
             graph.launch()
-            assert np.all(np.abs(c.to_numpy(out, np.float32, (T, hq, d)) - want) <= bound)
+            got = c.to_numpy(out, np.float32, (T, hq, d))
+            assert np.all(np.abs(got - want) <= bound)
+            hip.gqaAttention(c, eager_args)
+            assert np.array_equal(got.view(np.uint32), c.to_numpy(eager, np.uint32, (T, hq, d)))
         graph.destroy()
     finally:
         c.deinit()

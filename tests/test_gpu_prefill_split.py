@@ -77,3 +77,64 @@ def test_split_noalloc_is_the_step(ctx, hip, kv):
                                       1e-6, 1e6, 1.0, float(np.float32(d) ** np.float32(-0.5))))
         outs.append(ctx.to_numpy(out, np.uint32, (T, hq, d)))
     assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
+
+
+def _block_inputs(oracle, T, pos, hq, hkv, hidden):
+    g = np.random.default_rng(9)
+    d, cap = 128, pos + T
+    x = g.standard_normal((T, hidden)).astype(np.float32)
+    w = [oracle.q8_0_quantize(g.standard_normal((h * d, hidden)).astype(np.float32) * np.float32(0.05))
+         for h in (hq, hkv, hkv)]
+    kc, vc = (g.standard_normal((hkv, cap, d)).astype(np.float16) for _ in range(2))
+    return x, w, kc, vc
+
+
+@pytest.mark.parametrize("T,pos,hq,hkv,merges", [(100, 3000, 32, 4, 1), (17, 1500, 8, 2, 1), (40, 64, 8, 2, 0)])
+def test_split_block_is_the_two_calls_also_captured(hip, oracle, T, pos, hq, hkv, merges):
+    """attentionBlock on a launch split over its keys equals matmulGroup and attentionStep, bit
+    for bit, eagerly and captured: the two calls on a context of their own, the block captured
+    where only the same block at position 0 (nothing split there) ran before it."""
+    print(f"[split_block] T={T} pos={pos} hq={hq} hkv={hkv}", flush=True)
+    d, hidden = 128, 512
+    x, w, kc, vc = _block_inputs(oracle, T, pos, hq, hkv, hidden)
+    scale = float(np.float32(1.0) / np.sqrt(np.float32(d)))
+
+    def args(c, at):
+        bufs = [c.createBuffer(T * h * d * 4) for h in (hq, hkv, hkv)]
+        bufs += [c.from_numpy(a) for a in (np.ones(d, np.float32), np.ones(d, np.float32),
+                                           np.arange(at, at + T, dtype=np.int32), kc, vc)]
+        return hip.AttentionStepArgs(*bufs, c.createBuffer(T * hq * d * 4), hip.DTYPE_F16, at, T, hq, hkv, d, pos + T, 1e-6,
+                                     1e6, 1.0, scale)
+
+    def results(c, a):
+        return [c.to_numpy(b, np.uint8, None) for b in (a.out, a.k_cache, a.v_cache)]
+
+    c = hip.Ctx.init(0)
+    try:  # the two calls
+        xb, wb, a = c.from_numpy(x), [c.from_numpy(v) for v in w], args(c, pos)
+        hip.matmulGroup(c, hip.MatmulGroupArgs.of(xb, hip.DTYPE_Q8_0, T, hidden, [(wb[0], a.q, hq * d), (wb[1], a.k, hkv * d),
+                                                                                 (wb[2], a.v, hkv * d)]))
+        c.set_kernel_timing(True)
+        hip.attentionStep(c, a)
+        assert c.kernel_time("prefill_merge_kernel")[0] == merges
+        c.set_kernel_timing(False)
+        want = results(c, a)
+    finally:
+        c.deinit()
+    c = hip.Ctx.init(0)
+    try:
+        xb, wb = c.from_numpy(x), [c.from_numpy(v) for v in w]
+        block = lambda a: hip.attentionBlock(c, hip.AttentionBlockArgs(xb, *wb, hip.DTYPE_Q8_0, hidden, a))  # noqa: E731
+        block(args(c, 0))
+        a, eager = args(c, pos), args(c, pos)
+        graph = c.capture(lambda: block(a))
+        for _ in range(3):
+            c.zero(a.out, T * hq * d * 4)
+            graph.launch()
+            c.submit()
+            assert all(np.array_equal(p, q) for p, q in zip(results(c, a), want))
+            block(eager)
+            assert all(np.array_equal(p, q) for p, q in zip(results(c, eager), want))
+        graph.destroy()
+    finally:
+        c.deinit()

@@ -1,6 +1,6 @@
 """The allocation-free attention step (ds5_hip_attention_step_noalloc) against
 ds5_hip_attention_step, through the C ABI: the same kernels run, only the
-split-K partials / f16 q operand live in the library's static per-GPU scratch,
+decode partials or the prefill rope table live in the library's static per-GPU scratch,
 so outputs and cache rows must be bit-identical. Two calls in a row, the second
 smaller, check that the array keeps nothing that matters between calls; a call
 needing more scratch than the array holds is rejected before any device work;
