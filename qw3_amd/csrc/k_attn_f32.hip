@@ -43,8 +43,12 @@ struct AttnF32Params {
     float* part_ml;  // [n_tokens * n_q_heads, n_splits, 2]
     uint32_t pos, n_tokens, n_q_heads, group, max_ctx;
     uint32_t chunk, n_splits;  // positions per split
-    float scale_log2;
+    float scale;
 };
+
+// exp(d) of a score less its reference. The scores stay as they are (not in units of log2,
+// where a finite score above 2.4e38 would overflow): only the difference is scaled.
+DS5_DEVICE_INLINE float weight_of(float d) { return fast_exp2(d * kLog2e); }
 
 DS5_DEVICE_INLINE f32x4 mfma_f32_16x16x4(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -114,7 +118,7 @@ __global__ __launch_bounds__(kThreads) void attn_f32_kernel(const AttnF32Params 
         const bool edge = p0 + kPos - 1 > first_lim || p0 + kPos > end;
         float s[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) s[i] = (s0[i] + s1[i]) * p.scale_log2;
+        for (int i = 0; i < 4; i++) s[i] = (s0[i] + s1[i]) * p.scale;
         if (edge) {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -127,10 +131,10 @@ __global__ __launch_bounds__(kThreads) void attn_f32_kernel(const AttnF32Params 
         const float m_new = fmaxf(m, mx);
         // a row without a score yet keeps weights of 0 (-inf - -inf would be NaN)
         const float ref = m_new == -INFINITY ? 0.0f : m_new;
-        const float alpha = fast_exp2(m - ref);
+        const float alpha = weight_of(m - ref);
         float w[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) w[i] = fast_exp2(s[i] - ref);
+        for (int i = 0; i < 4; i++) w[i] = weight_of(s[i] - ref);
         l = l * alpha + ((w[0] + w[1]) + (w[2] + w[3]));
         m = m_new;
         if (__ballot(alpha != 1.0f)) {
@@ -248,7 +252,7 @@ __global__ __launch_bounds__(kThreads) void attn_f32_kernel(const AttnF32Params 
             float lt = 0.0f;
 #pragma unroll
             for (int w = 0; w < kWaves; w++) {
-                const float f = fast_exp2(s_m[w][r] - ref);
+                const float f = weight_of(s_m[w][r] - ref);
                 // a wavefront without a score for the row has weight 0 and O 0
                 acc += *(const f32x4*)&s_o[w][r * OROW + d0] * f;
                 lt += s_l[w][r] * f;
@@ -292,7 +296,7 @@ __global__ __launch_bounds__(256) void attn_f32_merge_kernel(const AttnF32Params
         for (int k = 0; k < BATCH; k++) {
             if (s0 + SLOTS * k >= ns) break;
             const float mn = fmaxf(m, ml[k].x), ref = mn == -INFINITY ? 0.0f : mn;
-            const float a = fast_exp2(m - ref), w = fast_exp2(ml[k].x - ref);
+            const float a = weight_of(m - ref), w = weight_of(ml[k].x - ref);
             l = l * a + ml[k].y * w;
             o = o * a + os[k] * w;
             m = mn;
@@ -310,7 +314,7 @@ __global__ __launch_bounds__(256) void attn_f32_merge_kernel(const AttnF32Params
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int k = 0; k < SLOTS; k++) {
-            const float w = fast_exp2(s_ml[k].x - ref);
+            const float w = weight_of(s_ml[k].x - ref);
             lt += s_ml[k].y * w;
             acc += s_o[k][col] * w;
         }
@@ -379,6 +383,6 @@ int launch_attn_f32(ds5_hip_ctx* ctx, const GenericAttnLaunch& a) {
     p.max_ctx = a.max_ctx;
     p.chunk = plan.chunk;
     p.n_splits = plan.n_splits;
-    p.scale_log2 = a.scale * kLog2e;
+    p.scale = a.scale;
     return a.head_dim == 128 ? launch_d<128>(ctx, p, plan, a.n_kv_heads) : launch_d<64>(ctx, p, plan, a.n_kv_heads);
 }

@@ -92,6 +92,31 @@ def test_f32_non_finite_rows_stay_behind_the_mask(ctx, hip, T, pos, hq, hkv, d):
     assert np.all(np.isfinite(got[at - pos][:, [0, 1, 2, 4, 6]])) and np.all(np.isnan(got[at - pos + 1:]))
 
 
+@pytest.mark.parametrize("T,pos", [(1, 40), (1, 700), (600, 300)])  # one split, several, a wavefront per row tile
+@pytest.mark.parametrize("at", [0, 33, None])
+def test_f32_scores_near_the_largest_float(ctx, hip, T, pos, at):
+    """Scores of +-3e38 are finite: one such position takes all the weight; with every score
+    at -3e38 (at None) the positions share it."""
+    hq, hkv, d = 16, 4, 64
+    print(f"[attn_f32] scores of 3e38 T={T} pos={pos} at={at}", flush=True)
+    cap = pos + T
+    q, kc, vc = _inputs(T, pos, hq, hkv, d, cap)
+    q[:], kc[:] = 0, 0
+    q[:, :, 5], kc[:, slice(None) if at is None else at, 5] = 1e19, 3e19 if at is not None else -3e19
+    out = ctx.createBuffer(T * hq * d * 4)
+    hip.gqaAttention(ctx, hip.AttnArgs(ctx.from_numpy(q), ctx.from_numpy(kc), ctx.from_numpy(vc), hip.DTYPE_F32, out, pos, T,
+                                       hq, hkv, d, cap, 1.0))
+    got = ctx.to_numpy(out, np.float32, (T, hq, d))
+    for t in (0, T // 2, T - 1):
+        L = pos + t + 1
+        for h in range(hq):
+            v = vc[h // (hq // hkv), :L].astype(np.float64)
+            if at is not None:
+                assert np.array_equal(got[t, h], v[at].astype(np.float32))
+            else:  # sums of L terms, each rounded
+                assert np.all(np.abs(got[t, h] - v.mean(0)) <= (L + 8) * EPS24 * np.abs(v).mean(0))
+
+
 @pytest.mark.parametrize("kv", ["f32", "f16"])
 @pytest.mark.parametrize("T,pos,hq,hkv,d", [(1, 40, 32, 4, 128), (3, 0, 4, 2, 64), (19, 5, 6, 2, 96), (2, 9, 64, 4, 128),
                                             (2, 1, 3, 1, 256), (2, 1, 2, 1, 320)])
