@@ -1049,11 +1049,13 @@ static bool gemm_half_tiles(const ds5_hip_ctx* ctx, uint32_t m, uint32_t cols) {
     return ((uint64_t)m + 63) / 64 * cols <= cu + cu / 8;
 }
 
-// Split products: 32 columns a workgroup until 128 fill the CUs (m 17, n 2048, k 4096: 14
-// against 28 us; above, x would be read four times as often: n 65536, 805 MB of it).
+// Split products: 32 columns a workgroup while tiles of 128 would fill half of the CUs (us,
+// 32 / 128 columns, k 2048 and 4096: 64 such tiles, m 64, n 4096, 17 / 22 and 27 / 37; 128,
+// m 128, n 4096, 25 / 25 and 42 / 42; 144, m 33, n 9216, 27 / 23 and 50 / 39): above, x is
+// read four times as often and nothing is left idle.
 static bool gemm_narrow_tiles(const ds5_hip_ctx* ctx, uint32_t m, uint32_t cols) {
     const uint64_t cu = ctx->cu_count > 0 ? ctx->cu_count : 256;
-    return ((uint64_t)m + 31) / 32 * cols <= cu;
+    return ((uint64_t)m + 31) / 32 * cols <= cu / 2;
 }
 
 // The split x is made once and shared by the group's products.
@@ -1209,14 +1211,19 @@ static bool gemm_offsets_fit(uint32_t m, uint32_t k, uint64_t w_end) {
     return (uint64_t)m * k * 2 < (1ull << 32) && w_end + 2 < (1ull << 32);
 }
 
-// Few tokens on a matrix that is not huge: four groups of wavefronts split a tile's blocks,
-// as otherwise most CUs have no tile and the others wait for one block after the other
-// (m 32, n 2048, k 4096: 41 us unsplit, 15 split; m 64, n 5120, k 2048: 26 and 17; m 128, n
-// 2048, k 4096: 50 and 20). From 16384 columns there are tiles enough, and 32-row tiles would
-// only read the weights once more. Chosen from the product's own shape: in a group or in the
-// attention block it adds in the same order.
+// Up to 128 tokens, four groups of wavefronts split a tile's blocks while the 32 x 128 tiles
+// (one such workgroup fits a CU) are at most as many as the 256 CUs: unsplit, most CUs have
+// no tile and the others wait for one block after the other. us, split and unsplit:
+//   k 2048:  n 2048, m 32 (16 tiles) 14 and 29;  n 8192, m 128 (256) 29 and 32, m 129 (320)
+//            43 and 32;  n 16384, m 64 (256) 29 and 33, m 65 (384) 45 and 34;  n 30011, m 32
+//            (235) 30 and 34, m 33 (470) 49 and 34
+//   k 4096:  n 9216, m 96 (216) 44 and 57, m 128 (288) 79 and 57;  n 16384, m 65 (384) 76 and 59
+// Few blocks leave little to split: half as many tiles (k 96: n 300, m 64 (6) 8.4 and 9.5,
+// n 4096, m 128 (128) 9.2 and 9.8, n 9216, m 64 (144) 9.9 and 10.0, n 12288, m 64 (192) 10.2
+// and 10.2, n 30011, m 32 (235), k 256 12.1 and 11.3). Chosen from the product's own shape:
+// in a group or in the attention block it adds in the same order.
 static bool gemm_split(uint32_t m, uint32_t n, uint32_t k) {
-    return k >= 32 * 8 && (m <= 32 || (m <= 128 && n < 16384));
+    return m <= 128 && ((uint64_t)m + 31) / 32 * (((uint64_t)n + kGemmCols - 1) / kGemmCols) <= (k > 256 ? 256 : 128);
 }
 
 MatmulPath matmul_path(const MatmulLaunch& a, uint64_t w_len) {

@@ -27,7 +27,11 @@ def bound(x, w, extra=0.0):
 
 
 CASES = [(16, 128, 64), (17, 1, 32), (31, 127, 96), (33, 300, 2048), (63, 512, 160), (64, 129, 4096), (65, 4096, 256),
-         (127, 40, 224), (128, 256, 32 * 65), (129, 130, 2048), (200, 20000, 64), (300, 12000, 96)]
+         (127, 40, 224), (128, 256, 32 * 65), (129, 130, 2048), (200, 20000, 64), (300, 12000, 96),
+         # blocks split over groups: one without a block (nine and three blocks), one with a single one;
+         # 32 and 128 columns a workgroup; the last split tile counts and the first unsplit ones
+         (16, 5, 32), (33, 300, 96), (20, 40, 288), (128, 4096, 288), (128, 4097, 288), (65, 10880, 320), (31, 32700, 288),
+         (128, 8192, 288), (128, 8193, 288), (64, 8192, 96), (64, 8193, 96), (32, 32800, 288)]
 
 
 @pytest.mark.parametrize("m,n,k", CASES)
