@@ -378,8 +378,9 @@ int ds5_hip_matmul_add(ds5_hip_ctx* ctx, const ds5_matmul_add_args* args);
  * w_dtype, out[e], m, n[e], k), same results bit for bit. All entries are
  * checked (in order, each as matmul checks) before anything is enqueued. When
  * every entry takes the same kernel the group is one launch per pass of tokens
- * (from 16 Q8_0 tokens: one split of x, then one launch). count is
- * 1..DS5_MATMUL_GROUP_MAX, else ShapeMismatch. */
+ * (from 16 Q8_0 tokens: one split of x, then one launch, or two where entries of
+ * different sizes take the kernel's two forms). count is 1..DS5_MATMUL_GROUP_MAX,
+ * else ShapeMismatch. */
 #define DS5_MATMUL_GROUP_MAX 4u
 typedef struct ds5_matmul_group_args {
     ds5_buf x;        /* f32 [m, k], shared */

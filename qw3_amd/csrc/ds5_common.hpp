@@ -151,6 +151,7 @@ struct MatmulLaunch {
 // tile's blocks split over groups of wavefronts), or the serial one-thread-per-output
 // kernel that takes any shape and alignment.
 enum class MatmulPath { Generic, Rows, Gemm, GemmSplit };
+inline bool is_gemm(MatmulPath p) { return p == MatmulPath::Gemm || p == MatmulPath::GemmSplit; }
 MatmulPath matmul_path(const MatmulLaunch& a, uint64_t w_len);
 int launch_matmul(ds5_hip_ctx* ctx, const MatmulLaunch& a, MatmulPath path);
 // Up to kMatmulGroupMax products sharing x (and m, k, the weight dtype).
@@ -192,7 +193,7 @@ struct QkvPrepLaunch {
     void* ws;
     const float* norm_w;  // x normalised first, as MatmulGroupLaunch::norm_w (null: none)
     float norm_eps;
-    bool split;  // MatmulPath::GemmSplit for all three
+    bool split[3];  // MatmulPath::GemmSplit for wq, wk, wv
 };
 size_t qkv_prep_workspace_bytes(uint32_t m, uint32_t k, uint32_t head_dim);
 int launch_qkv_prep(ds5_hip_ctx* ctx, const QkvPrepLaunch& a);

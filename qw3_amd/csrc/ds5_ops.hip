@@ -856,8 +856,7 @@ int ds5_hip_attention_block(ds5_hip_ctx* ctx, const ds5_attention_block_args* a)
     // every projection takes one of them; otherwise rmsNorm writes h to the context's
     // second buffer first and the block runs on h.
     const bool all_rows = paths[0] == MatmulPath::Rows && paths[1] == MatmulPath::Rows && paths[2] == MatmulPath::Rows;
-    const bool all_gemm = paths[0] == paths[1] && paths[1] == paths[2] &&
-                          (paths[0] == MatmulPath::Gemm || paths[0] == MatmulPath::GemmSplit);
+    const bool all_gemm = is_gemm(paths[0]) && is_gemm(paths[1]) && is_gemm(paths[2]);
     const bool norm_inside = norm && a->hidden > kRmsSerialMaxDim && aligned16(a->x_norm) && (all_rows || all_gemm);
     if (norm && !norm_inside) {
         void* h = nullptr;
@@ -915,7 +914,7 @@ int ds5_hip_attention_block(ds5_hip_ctx* ctx, const ds5_attention_block_args* a)
     qp.ws = (char*)ws + q16_bytes;
     qp.norm_w = gl.norm_w;
     qp.norm_eps = gl.norm_eps;
-    qp.split = paths[0] == MatmulPath::GemmSplit;
+    for (int e = 0; e < 3; e++) qp.split[e] = paths[e] == MatmulPath::GemmSplit;
     if (int rc = launch_qkv_prep(ctx, qp)) return rc;
     PrefillLaunch l{};
     l.q16 = (const f16*)ws;

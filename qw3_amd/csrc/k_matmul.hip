@@ -1058,17 +1058,18 @@ static bool gemm_narrow_tiles(const ds5_hip_ctx* ctx, uint32_t m, uint32_t cols)
     return ((uint64_t)m + 31) / 32 * cols <= cu / 2;
 }
 
-// The split x is made once and shared by the group's products.
-template <int TM, int W, int KS>
-int launch_gemm(ds5_hip_ctx* ctx, const MatmulGroupLaunch& a) {
-    void* ws = nullptr;
-    if (int rc = ds5_workspace(ctx, x_split_bytes(a.m, a.k), &ws)) return rc;
+// The split x: made once, shared by a group's products.
+struct XPlanes {
+    uint16_t *hi, *lo;
+    int* row_exp;
+};
+XPlanes x_planes(void* ws, uint32_t m, uint32_t k) {
     uint16_t* hi = (uint16_t*)ws;
-    uint16_t* lo = hi + (size_t)a.m * a.k;
-    int* row_exp = (int*)(lo + (size_t)a.m * a.k);
-    DS5_TIMED_LAUNCH(ctx, "matmul_x_split_kernel", matmul_x_split_kernel<false>, dim3(a.m), dim3(kSplitThreads), 0,
-                     ctx->stream, a.x, hi, lo, row_exp, a.k, XSplitRope{}, RopeTable{}, a.norm_w, a.norm_eps);
-    if (int rc = ds5_after_launch(ctx, "matmul_x_split_kernel")) return rc;
+    return XPlanes{hi, hi + (size_t)m * k, (int*)(hi + 2 * (size_t)m * k)};
+}
+
+template <int TM, int W, int KS>
+int launch_gemm(ds5_hip_ctx* ctx, const MatmulGroupLaunch& a, const XPlanes& xp) {
     WeightGroup g{};
     uint32_t tiles = 0;
     for (uint32_t e = 0; e < a.count; e++) {
@@ -1082,8 +1083,8 @@ int launch_gemm(ds5_hip_ctx* ctx, const MatmulGroupLaunch& a) {
     }
     if (tiles == 0) return DS5_OK;
     DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<TM, W, KS, 0>),
-                     dim3(tiles, gemm_row_tiles(a.m, 32 * TM)), dim3(64 * W * KS), 0, ctx->stream, hi, lo, row_exp, g, a.m,
-                     a.k, AttnPrepEpi{}, MoeGemmTiles{});
+                     dim3(tiles, gemm_row_tiles(a.m, 32 * TM)), dim3(64 * W * KS), 0, ctx->stream, xp.hi, xp.lo, xp.row_exp,
+                     g, a.m, a.k, AttnPrepEpi{}, MoeGemmTiles{});
     return ds5_after_launch(ctx, "matmul_q8_mfma_kernel");
 }
 
@@ -1160,37 +1161,40 @@ size_t qkv_prep_workspace_bytes(uint32_t m, uint32_t k, uint32_t head_dim) {
 }
 
 int launch_qkv_prep(ds5_hip_ctx* ctx, const QkvPrepLaunch& a) {
-    uint16_t* hi = (uint16_t*)a.ws;
-    uint16_t* lo = hi + (size_t)a.m * a.k;
-    int* row_exp = (int*)(lo + (size_t)a.m * a.k);
+    const XPlanes xp = x_planes(a.ws, a.m, a.k);
     float* cs = (float*)((char*)a.ws + qkv_prep_cs_offset(a.m, a.k));
     XSplitRope rope{a.positions, cs, a.head_dim / 2, a.freq_scale};
     DS5_TIMED_LAUNCH(ctx, "matmul_x_split_kernel", matmul_x_split_kernel<true>, dim3(a.m), dim3(kSplitThreads), 0,
-                     ctx->stream, a.x, hi, lo, row_exp, a.k, rope, *a.table, a.norm_w, a.norm_eps);
+                     ctx->stream, a.x, xp.hi, xp.lo, xp.row_exp, a.k, rope, *a.table, a.norm_w, a.norm_eps);
     if (int rc = ds5_after_launch(ctx, "matmul_x_split_kernel")) return rc;
-    WeightGroup g{};
     const uint32_t ns[3] = {a.n_q_heads * a.head_dim, a.n_kv_heads * a.head_dim, a.n_kv_heads * a.head_dim};
     const uint8_t* ws[3] = {a.wq, a.wk, a.wv};
-    uint32_t tiles = 0;
-    for (int e = 0; e < 3; e++) {
-        g.w[e] = ws[e];
-        g.n[e] = ns[e];
-        g.wg0[e] = tiles;
-        tiles += ns[e] / kGemmCols;
-    }
-    g.count = 3;
     AttnPrepEpi ep{a.q_norm, a.k_norm, cs, a.q16, a.k_cache, a.v_cache, a.pos, a.n_q_heads, a.max_ctx, a.eps, a.q_scale};
-    auto launch = [&](auto tm, auto ks) {
-        constexpr int TM = decltype(tm)::value, KS = decltype(ks)::value;
-        DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<TM, 4, KS, 1>),
-                         dim3(tiles, gemm_row_tiles(a.m, 32 * TM)), dim3(256 * KS), 0, ctx->stream, hi, lo, row_exp, g, a.m,
-                         a.k, ep, MoeGemmTiles{});
-    };
-    using std::integral_constant;
-    if (a.split) launch(integral_constant<int, 1>{}, integral_constant<int, 4>{});
-    else if (gemm_half_tiles(ctx, a.m, tiles)) launch(integral_constant<int, 2>{}, integral_constant<int, 1>{});
-    else launch(integral_constant<int, 4>{}, integral_constant<int, 1>{});
-    return ds5_after_launch(ctx, "matmul_q8_mfma_kernel");
+    // one launch, or two where the weights' sizes put some on the split form and some not
+    for (int split = 0; split < 2; split++) {
+        WeightGroup g{};
+        uint32_t tiles = 0;
+        for (int e = 0; e < 3; e++) {  // all three keep their places: the epilogue goes by them
+            g.w[e] = ws[e];
+            g.n[e] = ns[e];
+            g.wg0[e] = tiles;
+            if (a.split[e] == (split != 0)) tiles += ns[e] / kGemmCols;
+        }
+        g.count = 3;
+        if (tiles == 0) continue;
+        auto launch = [&](auto tm, auto ks) {
+            constexpr int TM = decltype(tm)::value, KS = decltype(ks)::value;
+            DS5_TIMED_LAUNCH(ctx, "matmul_q8_mfma_kernel", (matmul_q8_mfma_kernel<TM, 4, KS, 1>),
+                             dim3(tiles, gemm_row_tiles(a.m, 32 * TM)), dim3(256 * KS), 0, ctx->stream, xp.hi, xp.lo,
+                             xp.row_exp, g, a.m, a.k, ep, MoeGemmTiles{});
+        };
+        using std::integral_constant;
+        if (split) launch(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+        else if (gemm_half_tiles(ctx, a.m, tiles)) launch(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+        else launch(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+        if (int rc = ds5_after_launch(ctx, "matmul_q8_mfma_kernel")) return rc;
+    }
+    return DS5_OK;
 }
 
 // Tokens from which Q8_0 products run on the matrix cores (below, the row
@@ -1249,17 +1253,52 @@ static int launch_generic(ds5_hip_ctx* ctx, const float* x, const uint8_t* w, bo
     return ds5_after_launch(ctx, "matmul_generic_kernel");
 }
 
+// The part of a group that takes `path`.
+static MatmulGroupLaunch group_part(const MatmulGroupLaunch& a, const MatmulPath* paths, MatmulPath path) {
+    MatmulGroupLaunch p = a;
+    p.count = 0;
+    for (uint32_t e = 0; e < a.count; e++)
+        if (paths[e] == path) {
+            p.w[p.count] = a.w[e];
+            p.out[p.count] = a.out[e];
+            p.res[p.count] = a.res[e];
+            p.n[p.count++] = a.n[e];
+        }
+    return p;
+}
+
+// A group on the matrix cores: x split once, then a launch for the split products and one
+// for the others.
+static int launch_gemms(ds5_hip_ctx* ctx, const MatmulGroupLaunch& a, const MatmulPath* paths) {
+    void* ws = nullptr;
+    if (int rc = ds5_workspace(ctx, x_split_bytes(a.m, a.k), &ws)) return rc;
+    const XPlanes xp = x_planes(ws, a.m, a.k);
+    DS5_TIMED_LAUNCH(ctx, "matmul_x_split_kernel", matmul_x_split_kernel<false>, dim3(a.m), dim3(kSplitThreads), 0,
+                     ctx->stream, a.x, xp.hi, xp.lo, xp.row_exp, a.k, XSplitRope{}, RopeTable{}, a.norm_w, a.norm_eps);
+    if (int rc = ds5_after_launch(ctx, "matmul_x_split_kernel")) return rc;
+    for (MatmulPath path : {MatmulPath::Gemm, MatmulPath::GemmSplit}) {
+        const MatmulGroupLaunch p = group_part(a, paths, path);
+        uint32_t cols = 0;
+        for (uint32_t e = 0; e < p.count; e++) cols += (p.n[e] + kGemmCols - 1) / kGemmCols;
+        if (cols == 0) continue;
+        int rc;
+        if (path == MatmulPath::Gemm)
+            rc = gemm_half_tiles(ctx, a.m, cols) ? launch_gemm<2, 4, 1>(ctx, p, xp) : launch_gemm<4, 4, 1>(ctx, p, xp);
+        else
+            rc = gemm_narrow_tiles(ctx, a.m, cols) ? launch_gemm<1, 1, 4>(ctx, p, xp) : launch_gemm<1, 4, 4>(ctx, p, xp);
+        if (rc) return rc;
+    }
+    return DS5_OK;
+}
+
 static int launch_same_path(ds5_hip_ctx* ctx, const MatmulGroupLaunch& a, MatmulPath path) {
     if (a.norm_w && (path == MatmulPath::Generic || a.k <= kRmsSerialMaxDim))
         return ds5_fail(ctx, DS5_DEVICE_FAILURE, "matmul: an in-kernel norm needs the row or GEMM path and k > %u",
                         kRmsSerialMaxDim);
     if (path == MatmulPath::Rows) return a.q8 ? launch_rows_q<true>(ctx, a) : launch_rows_q<false>(ctx, a);
-    if (path == MatmulPath::Gemm || path == MatmulPath::GemmSplit) {
-        uint32_t cols = 0;
-        for (uint32_t e = 0; e < a.count; e++) cols += (a.n[e] + kGemmCols - 1) / kGemmCols;
-        if (path == MatmulPath::Gemm)
-            return gemm_half_tiles(ctx, a.m, cols) ? launch_gemm<2, 4, 1>(ctx, a) : launch_gemm<4, 4, 1>(ctx, a);
-        return gemm_narrow_tiles(ctx, a.m, cols) ? launch_gemm<1, 1, 4>(ctx, a) : launch_gemm<1, 4, 4>(ctx, a);
+    if (is_gemm(path)) {
+        const MatmulPath paths[kMatmulGroupMax] = {path, path, path, path};
+        return launch_gemms(ctx, a, paths);
     }
     for (uint32_t e = 0; e < a.count; e++)
         if (a.n[e])
@@ -1290,13 +1329,20 @@ int launch_add(ds5_hip_ctx* ctx, const void* x, const void* y, void* out, uint64
     return ds5_after_launch(ctx, "add_kernel");
 }
 
-// One launch for the whole group when every entry takes the same kernel;
-// otherwise each entry on its own kernel, in order.
+// One launch for the whole group when every entry takes the same kernel (the matrix cores'
+// two forms: one x split, a launch each); otherwise each entry on its own kernel, in order.
 int launch_matmul_group(ds5_hip_ctx* ctx, const MatmulGroupLaunch& a, const MatmulPath* paths) {
     if (a.m == 0 || a.count == 0) return DS5_OK;
-    bool same = true;
-    for (uint32_t e = 1; e < a.count; e++) same = same && paths[e] == paths[0];
+    bool same = true, gemm = true;
+    for (uint32_t e = 0; e < a.count; e++) {
+        same = same && paths[e] == paths[0];
+        gemm = gemm && is_gemm(paths[e]);
+    }
     if (same) return launch_same_path(ctx, a, paths[0]);
+    if (a.norm_w && !(gemm && a.k > kRmsSerialMaxDim))
+        return ds5_fail(ctx, DS5_DEVICE_FAILURE, "matmul: an in-kernel norm needs one kernel for the group and k > %u",
+                        kRmsSerialMaxDim);
+    if (gemm) return launch_gemms(ctx, a, paths);
     for (uint32_t e = 0; e < a.count; e++) {
         MatmulGroupLaunch one{};
         one.x = a.x;

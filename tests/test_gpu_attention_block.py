@@ -28,6 +28,9 @@ CASES = {
     "t100_pos37": (100, 37, 32, 4, 128, 1024, "q8", True, True),   # ragged row tile, continuation
     "t300_64q": (300, 0, 64, 4, 128, 512, "q8", True, True),       # three row tiles, 16-head groups
     "t130_2group": (130, 3, 8, 4, 128, 256, "q8", True, True),     # 2-head groups
+    # q unsplit, k and v split products: one x split, a launch for each form
+    "t100_128q": (100, 20, 128, 4, 128, 512, "q8", 2, True),
+    "t33_256q": (33, 0, 256, 8, 128, 288, "q8", 2, True),
     "c2_hidden2048": (2048, 0, 32, 4, 128, 2048, "q8", True, False),  # the C2 prefill with its projections
     "t8_rows": (8, 0, 32, 4, 128, 512, "q8", False, True),         # row kernel: the two calls
     "t1_decode": (1, 20, 32, 4, 128, 512, "q8", False, True),      # decode: the two calls
@@ -97,8 +100,8 @@ def test_attention_block_equals_the_two_calls(ctx, hip, oracle, case):
     block = hip.AttentionBlockArgs(inp.xb, *inp.wb, inp.dtype, hidden, blk)
     counts = _counted(ctx, lambda: hip.attentionBlock(ctx, block))
     print(f"  launches: { {k: c for k, c in counts.items() if c} }", flush=True)
-    if fused:  # the pre-pass is the GEMM's epilogue: no prep launch, one split and one GEMM
-        assert counts["matmul_q8_mfma_kernel"] == 1 and counts["matmul_x_split_kernel"] == 1
+    if fused:  # the pre-pass is the GEMM's epilogue: no prep launch, one split and one GEMM (or two)
+        assert counts["matmul_q8_mfma_kernel"] == int(fused) and counts["matmul_x_split_kernel"] == 1
         assert counts["prefill_prep_kernel"] == 0 and counts["prefill_attention_kernel"] == 1
     else:
         assert counts["prefill_prep_kernel"] + counts["decode_split_kernel"] + counts["rms_norm_rows_kernel"] >= 1
@@ -154,7 +157,7 @@ def test_attention_block_errors(ctx, hip, oracle):
 
 
 @pytest.mark.parametrize("case", ["t16", "t300_64q", "c2_hidden2048", "t8_rows", "t1_decode", "f32_weights",
-                                  "t130_2group", "d64", "t1_hidden2048"])
+                                  "t130_2group", "d64", "t1_hidden2048", "t100_128q", "t33_256q"])
 def test_attention_block_with_norm(ctx, hip, oracle, case):
     """The block with x_norm (attn_norm applied first) equals ds5_hip_rms_norm(x -> h) then
     the block on h, bit for bit (output and every cache row): the norm inside the row

@@ -55,6 +55,27 @@ def test_gemm_tile_edges(ctx, hip, m, n, k, residual):
     assert np.all(np.abs(got - want) <= lim + 1e-30), float(np.max(np.abs(got - want) / (lim + 1e-30)))
 
 
+@pytest.mark.parametrize("m", [64, 65, 128])
+def test_mixed_group_is_its_products(ctx, hip, m):
+    """A group whose products take both matrix-core forms (from 65 tokens: 16384 columns unsplit,
+    the others split): each entry's bits are its own matmul's, x is split once."""
+    print(f"[gemm] mixed group m={m}", flush=True)
+    k, ns = 512, (130, 16384, 512)
+    g = np.random.default_rng(m)
+    xb = ctx.from_numpy(g.standard_normal((m, k)).astype(np.float32))
+    wb = [ctx.from_numpy(np.concatenate([q8_rows(g, n, k)[0].reshape(-1), np.zeros(4, np.uint8)])) for n in ns]
+    got, want = ([ctx.createBuffer(m * n * 4) for n in ns] for _ in range(2))
+    ctx.set_kernel_timing(True)
+    hip.matmulGroup(ctx, hip.MatmulGroupArgs.of(xb, hip.DTYPE_Q8_0, m, k, list(zip(wb, got, ns))))
+    ctx.submit()
+    launches = [ctx.kernel_time(name)[0] for name in ("matmul_x_split_kernel", "matmul_q8_mfma_kernel")]
+    ctx.set_kernel_timing(False)
+    assert launches == [1, 2 if m > 64 else 1]
+    for w, a, b, n in zip(wb, got, want, ns):
+        hip.matmul(ctx, hip.MatmulArgs(xb, w, hip.DTYPE_Q8_0, b, m, n, k))
+        assert np.array_equal(ctx.to_numpy(a, np.uint32, (m, n)), ctx.to_numpy(b, np.uint32, (m, n)))
+
+
 @pytest.mark.parametrize("T,E,K,dim,ffn", [(22, 16, 1, 256, 96), (44, 16, 1, 512, 64), (60, 24, 4, 2048, 768)])
 def test_grouped_experts_few_pairs(ctx, hip, T, E, K, dim, ffn):
     """Few pairs per expert (below, at and above the grouped threshold of 11 per 8 experts) against
