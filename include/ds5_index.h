@@ -55,6 +55,11 @@ void ds5_index_gemm_q(uint32_t wave, uint32_t threads, uint32_t nq, uint32_t w_r
  * A q tile row's token. */
 uint32_t ds5_index_prefill_tile(uint32_t head_dim, int v, uint32_t key0, uint32_t kv_end, uint32_t* off);
 uint32_t ds5_index_pf_q_token(uint32_t q0, uint32_t row, uint32_t n_tokens);
+/* The parts a launch's keys are split into; a q tile's key tiles and a part's first one. */
+uint32_t ds5_index_prefill_splits(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads,
+                                  uint32_t n_kv_heads, uint32_t head_dim);
+uint32_t ds5_index_pf_key_tiles(uint32_t pos, uint32_t qt, uint32_t n_tokens);
+uint32_t ds5_index_pf_split_first(uint32_t n, uint32_t s, uint32_t n_splits);
 
 /* attn_f32_kernel: a launch's plan, out = [row tiles, positions per split, splits, 1 if a
  * wavefront takes a row tile]; the first query row of a wavefront; a load's position; what a

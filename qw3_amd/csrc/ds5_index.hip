@@ -125,6 +125,17 @@ uint32_t ds5_index_pf_q_token(uint32_t q0, uint32_t row, uint32_t n_tokens) {
 }
 
 
+uint32_t ds5_index_prefill_splits(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads,
+                                  uint32_t n_kv_heads, uint32_t head_dim) {
+    return prefill_splits(cu_count, pos, n_tokens, n_q_heads, n_kv_heads, head_dim);
+}
+uint32_t ds5_index_pf_key_tiles(uint32_t pos, uint32_t qt, uint32_t n_tokens) {
+    return ds5idx::pf_key_tiles(pos, qt, n_tokens);
+}
+uint32_t ds5_index_pf_split_first(uint32_t n, uint32_t s, uint32_t n_splits) {
+    return ds5idx::pf_split_first(n, s, n_splits);
+}
+
 // The f32 attention: its plan, and the rows, positions and stores of a split.
 void ds5_index_attn_f32_plan(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads,
                              uint32_t head_dim, uint32_t* out) {

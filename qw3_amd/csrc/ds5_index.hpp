@@ -162,6 +162,11 @@ DS5_HD uint32_t pf_clamped_off(uint32_t off, uint32_t key0, uint32_t kv_end, int
     const uint32_t last_row = kv_end - key0 - 1;
     return umin(off / (2 * D), last_row) * (2 * D) + off % (2 * D);
 }
+// Key tiles that q tile qt needs, and the first of them of part s of n_splits.
+DS5_HD uint32_t pf_key_tiles(uint32_t pos, uint32_t qt, uint32_t n_tokens) {
+    return (pos + umin(n_tokens, qt * kPfQRows + kPfQRows) + kPfKTile - 1) / kPfKTile;
+}
+DS5_HD uint32_t pf_split_first(uint32_t n, uint32_t s, uint32_t n_splits) { return n * s / n_splits; }
 // A q tile's row `row` (< 32) reads token min(q0 + row, n_tokens - 1).
 DS5_HD uint32_t pf_q_token(uint32_t q0, uint32_t row, uint32_t n_tokens) { return umin(q0 + row, n_tokens - 1); }
 

@@ -194,9 +194,6 @@ struct PrefillParams {
     float2* part_ml;
 };
 
-// Key tiles [lo, hi) of part s of a q tile's n.
-__device__ __forceinline__ uint32_t split_first(uint32_t n, uint32_t s, uint32_t n_splits) { return n * s / n_splits; }
-
 template <int D>
 struct PGeo {
     static constexpr int KS = D / 16;              // k-steps of the S product
@@ -329,7 +326,7 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 // current half's exponentials and the current PV products beside the next half's
 // row max (see step), so its matrix-core and VALU work overlap in one instruction
 // stream.
-template <int D, int QM>
+template <int D, int QM, bool SPLIT>
 __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(PrefillParams p) {
     using G = PGeo<D>;
     constexpr int KS = G::KS, DT = G::DT, RSK = G::RSK, RSV = G::RSV;
@@ -351,14 +348,20 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(PrefillPara
     auto kv_end_of = [&](uint32_t qtile) -> uint32_t {  // keys the q tile needs (exclusive)
         return p.pos + min(p.n_tokens, qtile * kQRows + kQRows);
     };
-    // (split: this part's of them, from hk0 and lk0; a heavy tile has at least half of the
-    // keys' tiles and n_splits is at most that half, so H > 0)
-    const uint32_t Hn = (kv_end_of(heavy) + kKTile - 1) / kKTile, Ln = (kv_end_of(pair) + kKTile - 1) / kKTile;
-    const uint32_t split = blockIdx.y;
-    const uint32_t hk0 = split_first(Hn, split, p.n_splits), lk0 = split_first(Ln, split, p.n_splits);
-    const uint32_t H = split_first(Hn, split + 1, p.n_splits) - hk0;
-    // (the middle tile of an odd count is processed once)
-    const uint32_t L = pair < heavy ? split_first(Ln, split + 1, p.n_splits) - lk0 : 0;
+    uint32_t H = ds5idx::pf_key_tiles(p.pos, heavy, p.n_tokens);
+    uint32_t L = pair < heavy ? ds5idx::pf_key_tiles(p.pos, pair, p.n_tokens) : 0;  // (an odd count's middle tile: once)
+    // split: this part's of them, from hk0 and lk0; a heavy tile has at least half of the
+    // keys' tiles and n_splits is at most that half, so H > 0
+    // (a form of its own: in one kernel with the unsplit one the divisions and the scalar
+    // registers that this keeps cost unsplit launches 2 to 5%)
+    uint32_t hk0 = 0, lk0 = 0;
+    const uint32_t split = SPLIT ? blockIdx.y : 0;
+    if constexpr (SPLIT) {
+        hk0 = ds5idx::pf_split_first(H, split, p.n_splits);
+        lk0 = ds5idx::pf_split_first(L, split, p.n_splits);
+        H = ds5idx::pf_split_first(H, split + 1, p.n_splits) - hk0;
+        L = ds5idx::pf_split_first(L, split + 1, p.n_splits) - lk0;
+    }
     const bool has_light = L > 0;
     const uint32_t n_items = H + L;
     auto item_qt = [&](uint32_t i) -> uint32_t { return i < H ? heavy : pair; };
@@ -725,12 +728,11 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(PrefillPara
     constexpr int OBLK = (G::STAGE / 4) / (32 * OSTR) < DT ? (G::STAGE / 4) / (32 * OSTR) : DT;
     static_assert(OBLK >= 1 && DT % OBLK == 0, "whole passes");
     auto write_rows = [&](uint32_t qtile, char* area) {
-        const bool whole = p.n_splits == 1;  // uniform
-        const float inv_l = whole ? 1.0f / Lsum[0] : 1.0f;
+        const float inv_l = SPLIT ? 1.0f : 1.0f / Lsum[0];
         const uint32_t q0 = qtile * kQRows, lane = lane_here();
-        float* const dst = whole ? p.out : p.part_o + (uint64_t)split * D;
-        const uint64_t row_stride = whole ? D : (uint64_t)p.n_splits * D;
-        if (!whole && lane < 32 && live && q0 + lane < p.n_tokens)  // (a row without a key here: weight 0)
+        float* const dst = SPLIT ? p.part_o + (uint64_t)split * D : p.out;
+        const uint64_t row_stride = SPLIT ? (uint64_t)p.n_splits * D : D;
+        if (SPLIT && lane < 32 && live && q0 + lane < p.n_tokens)  // (a row without a key here: weight 0)
             p.part_ml[((uint64_t)(q0 + lane) * p.n_q_heads + hq) * p.n_splits + split] =
                 float2{Lsum[0] > 0.0f ? m_sh : -INFINITY, Lsum[0]};
 #pragma unroll
@@ -840,7 +842,7 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(PrefillPara
     // crosses a q tile's first row (key tile kt of q tile qt with 64 kt + 63 > pos +
     // 32 qt, i.e. kt >= first_masked).
     auto first_masked = [&](uint32_t qtile) -> uint32_t { return (p.pos + qtile * kQRows + 1) / kKTile; };
-    auto from = [](uint32_t a, uint32_t b) -> uint32_t { return a > b ? a - b : 0; };
+    auto from = [](uint32_t a, uint32_t b) -> uint32_t { return !SPLIT ? a : a > b ? a - b : 0; };
     const uint32_t mh = min(from(first_masked(heavy), hk0), H), ml = H + from(first_masked(pair), lk0);
     auto next_special = [&](uint32_t r) -> uint32_t {  // the first special round >= r
         uint32_t ns = n_items;
@@ -878,7 +880,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     const uint32_t c4 = 4 * (threadIdx.x % COLS);
     if (row >= (uint64_t)p.n_tokens * p.n_q_heads) return;
     const uint32_t qt = (uint32_t)(row / p.n_q_heads) / kQRows;
-    const uint32_t n = (p.pos + min(p.n_tokens, qt * kQRows + kQRows) + kKTile - 1) / kKTile;
+    const uint32_t n = ds5idx::pf_key_tiles(p.pos, qt, p.n_tokens);
     const float2* ml = p.part_ml + row * p.n_splits;
     const float* o = p.part_o + row * p.n_splits * D + c4;
     // B parts' loads at a time: the fold waits on memory, not on bandwidth, when the rows are
@@ -887,7 +889,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     // nothing; it is read and dropped.
     auto part = [&](uint32_t s) { return min(s, p.n_splits - 1); };
     auto used = [&](uint32_t s) {
-        return s < p.n_splits && split_first(n, s, p.n_splits) < split_first(n, s + 1, p.n_splits);
+        return s < p.n_splits && ds5idx::pf_split_first(n, s, p.n_splits) < ds5idx::pf_split_first(n, s + 1, p.n_splits);
     };
     float M = -INFINITY;
     for (uint32_t s0 = 0; s0 < p.n_splits; s0 += B) {
@@ -919,17 +921,23 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
 }
 }  // namespace
 
-// Parts of a launch's key tiles: as many as give each compute unit one workgroup (one fits a
-// unit), of at least 8 rounds (64 keys of a q tile, 0.72 us each; a workgroup's ends and the
-// merge cost ~7 us). Attention and merge, us,
-// unsplit and at the rule (q heads / kv heads 32 / 4, D 128 unless stated):
-//   203 tokens at 6000, 64 / 4   147 -> 57 + 7 (4 parts; 2 parts 84 + 5)
-//   203 tokens at 6000           142 -> 35 + 9 (8; 10 parts, more than units, 51 + 10)
-//   500 tokens at 1500            51 -> 27 + 8 (4)
-//   300 tokens at 3000, 16 / 2, D 64   59 -> 19 + 6 (8)
-//   700 tokens at 6000           172 -> 98 + 7 (2)
-// Splits of a launch that already has a workgroup per unit gain nothing (700 tokens at 2000,
-// 64 / 4: 81 unsplit, 74 to 84 at 2 to 16 parts without their merge).
+// Parts of a launch's key tiles: up to one workgroup per compute unit (one fits a unit), of at
+// least 8 rounds (64 keys of a q tile), and as many as save most: a round takes 0.72 us (D 64:
+// 0.52), the merge's launch 3.5 and the parts' way through memory 0.35 per MB. That fits 231
+// calls of 2 to 2000 tokens (7 head layouts), none of them slower than unsplit (one measured
+// later is, 48 tokens at 500, 128 / 8: 27.9 -> 28.5 with the pre-pass); by the rounds alone 13
+// were, by up to 31%. (The line at 8 rounds is on the safe side: 2 tokens at 900, 15 rounds,
+// 17 us unsplit, took 13 in 4 parts.) us, unsplit and split, merge included, 32 q / 4 kv heads
+// x 128 unless stated:
+//   2 tokens at 1022                     17 -> 15 (2 parts)
+//   203 tokens at 6000                  140 -> 42 (8; 10 parts, more than units, 62)
+//   203 tokens at 6000, 64 / 4          140 -> 63 (4; 2 parts 85)
+//   500 tokens at 1500                   51 -> 35 (4)
+//   100 tokens at 3000, 16 / 2, D 64     57 -> 21 (12)
+//   700 tokens at 2000                   62 -> 48 (2)
+// and not split, whose two parts were slower:
+//   1000 tokens at 0                     23, 30      500 at 600, 64 / 4    33, 36
+//   128 tokens at 500, 128 / 8           25, 30      1500 at 0, 16 / 2, D 64   21, 24
 constexpr uint32_t kSplitMinRounds = 8;
 uint32_t prefill_splits(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint32_t n_q_heads, uint32_t n_kv_heads,
                         uint32_t head_dim) {
@@ -938,9 +946,20 @@ uint32_t prefill_splits(uint32_t cu_count, uint32_t pos, uint32_t n_tokens, uint
     const uint64_t wgs = (uint64_t)n_kv_heads * hgroups * pairs, cu = cu_count ? cu_count : 256;
     const uint64_t tiles = ((uint64_t)pos + n_tokens + kKTile - 1) / kKTile;
     const uint64_t rounds = qtiles > 1 ? tiles + (pos + kQRows + kKTile - 1) / kKTile : tiles;
-    const uint64_t s = std::min<uint64_t>({cu / std::max<uint64_t>(wgs, 1), rounds / kSplitMinRounds, tiles / 2,
-                                           (uint64_t)ds5_max_splits((uint64_t)n_tokens * n_q_heads, head_dim)});
-    return (uint32_t)std::max<uint64_t>(s, 1);
+    const uint64_t row_bytes = (uint64_t)n_tokens * n_q_heads * (head_dim + 2) * sizeof(float);  // of one part
+    const uint64_t most = std::min<uint64_t>({cu / std::max<uint64_t>(wgs, 1), rounds / kSplitMinRounds, tiles / 2,
+                                              (uint64_t)ds5_max_splits((uint64_t)n_tokens * n_q_heads, head_dim)});
+    int64_t best = 0;  // what the split saves, in ns
+    uint32_t splits = 1;
+    for (uint64_t s = 2; s <= most; s++) {
+        const int64_t saved = (int64_t)(rounds * (s - 1) * (head_dim == 128 ? 720 : 520) / s) - 3500 -
+                              (int64_t)(row_bytes * s * 35 / 100000);
+        if (saved > best) {
+            best = saved;
+            splits = (uint32_t)s;
+        }
+    }
+    return splits;
 }
 
 bool prefill_prep_supported(uint32_t n_kv_heads, uint32_t head_dim) {
@@ -960,8 +979,12 @@ int launch_kv_prep(ds5_hip_ctx* ctx, const KvPrepLaunch& a) {
 
 template <int D, int QM>
 static void launch_prefill_k(ds5_hip_ctx* ctx, const PrefillParams& p) {
-    DS5_TIMED_LAUNCH(ctx, "prefill_attention_kernel", (prefill_attention_kernel<D, QM>), dim3(p.n_items, p.n_splits),
-                     dim3(kThreads), 0, ctx->stream, p);
+    if (p.n_splits > 1)
+        DS5_TIMED_LAUNCH(ctx, "prefill_attention_kernel", (prefill_attention_kernel<D, QM, true>),
+                         dim3(p.n_items, p.n_splits), dim3(kThreads), 0, ctx->stream, p);
+    else
+        DS5_TIMED_LAUNCH(ctx, "prefill_attention_kernel", (prefill_attention_kernel<D, QM, false>), dim3(p.n_items),
+                         dim3(kThreads), 0, ctx->stream, p);
 }
 
 template <int D>

@@ -43,6 +43,8 @@ def ix(hip):
         "ds5_index_gemm_x": ([u32] * 7 + [P], None), "ds5_index_gemm_q": ([u32] * 8 + [P] * 4, None),
         "ds5_index_gemm_x_rows": ([u32] * 7 + [P, P], None),
         "ds5_index_prefill_tile": ([u32, C.c_int, u32, u32, P], u32), "ds5_index_pf_q_token": ([u32] * 3, u32),
+        "ds5_index_prefill_splits": ([u32] * 6, u32), "ds5_index_pf_key_tiles": ([u32] * 3, u32),
+        "ds5_index_pf_split_first": ([u32] * 3, u32),
         "ds5_index_attn_f32_plan": ([u32] * 6 + [P], None), "ds5_index_af_row0": ([u32, u32, C.c_int], u32),
         "ds5_index_af_load_pos": ([u32] * 2, u32), "ds5_index_af_store": ([u32] * 3, u32),
         "ds5_index_af_row_splits": ([u32] * 2, u32),
@@ -65,7 +67,7 @@ def test_index_header_symbols_exported(hip):
     """Every function include/ds5_index.h declares is exported by the library."""
     text = open(os.path.join(ROOT, "include", "ds5_index.h")).read()
     names = set(re.findall(r"^\s*(?:void|uint32_t|uint64_t)\s+(ds5_index_\w+)\(", text, re.M))
-    assert len(names) == 22
+    assert len(names) == 25
     for n in names:
         assert getattr(hip.LIB, n) is not None
 
@@ -488,6 +490,41 @@ def check_prefill(ix, pos, T, hq, hkv, D, max_ctx):
 def test_prefill_dma_addresses(ix, pos, T, hq, hkv, D, cap):
     """C2 and the GPU parity suite's prefill shapes (chunked continuations, odd q-tile counts)."""
     assert check_prefill(ix, pos, T, hq, hkv, D, cap) > 0
+
+
+@pytest.mark.parametrize("hq,hkv,D", [(64, 4, 128), (32, 4, 128), (128, 8, 128), (16, 2, 64), (4, 2, 64), (5, 1, 128), (8, 8, 128)])
+def test_prefill_key_parts(ix, hq, hkv, D):
+    """A split launch: one workgroup per compute unit at most, 32 MiB of parts at most, and for
+    every q tile the parts that hold key tiles (those the merge folds) cover each tile once; a
+    workgroup's heavy tile has key tiles in every part."""
+    seen = set()
+    for T in (2, 17, 32, 33, 64, 65, 97, 203, 500, 700, 1000, 1600, 2048):
+        for pos in (0, 1, 63, 500, 1022, 1600, 3001, 6000, 20000):
+            s = ix.ds5_index_prefill_splits(256, pos, T, hq, hkv, D)
+            qtiles = -(-T // 32)
+            pairs = (qtiles + 1) // 2
+            assert s == 1 or s * hkv * -(-(hq // hkv) // 4) * pairs <= 256
+            assert s == 1 or s * T * hq * (D + 2) * 4 <= 32 << 20
+            if s == 1:
+                continue
+            seen.add(s)
+            for qt in range(qtiles):
+                n = ix.ds5_index_pf_key_tiles(pos, qt, T)
+                assert n == -(-(pos + min(T, 32 * qt + 32)) // 64)
+                first = [ix.ds5_index_pf_split_first(n, i, s) for i in range(s + 1)]
+                assert first[0] == 0 and first[s] == n and all(a <= b for a, b in zip(first, first[1:]))
+                if qt >= qtiles - pairs:  # a heavy tile
+                    assert all(a < b for a, b in zip(first, first[1:]))
+    assert 2 in seen and max(seen) >= 8
+
+
+@pytest.mark.parametrize("T,pos,hq,hkv,D,parts", [
+    (2, 959, 32, 4, 128, 2), (2, 957, 32, 4, 128, 1), (203, 6000, 32, 4, 128, 8), (203, 6000, 64, 4, 128, 4), (500, 1500, 32, 4, 128, 4),
+    (100, 3000, 16, 2, 64, 12), (700, 2000, 32, 4, 128, 2), (1000, 0, 32, 4, 128, 1), (500, 600, 64, 4, 128, 1),
+    (128, 500, 128, 8, 128, 1), (1500, 0, 16, 2, 64, 1), (2048, 0, 32, 4, 128, 1)])
+def test_prefill_split_rule(ix, T, pos, hq, hkv, D, parts):
+    """The rule at the calls its comment gives the times of."""
+    assert ix.ds5_index_prefill_splits(256, pos, T, hq, hkv, D) == parts
 
 
 # ---------------------------------------------------------------------------

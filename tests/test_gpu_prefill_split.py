@@ -1,22 +1,28 @@
 """Prefill attention whose key tiles are split over workgroups: short chunks over long
 contexts, where the launch would leave compute units idle. Against float64 at the attention
 gate of the f16 paths (max-abs 2e-3, cosine 0.99999), at parts that start inside a tile
-pair's masked rounds, odd tile counts, part-filled q tiles and the smallest split; and the
-allocation-free step against the step, whose partials live in different memory."""
+pair's masked rounds, odd tile counts, part-filled q tiles, 2 parts (the smallest split) to
+19 and the calls on either side of the rule's line; the allocation-free step against the
+step; and the attention block against the two calls it equals."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [  # T, pos, hq, hkv, d
-    (2, 1600, 64, 4, 128),    # one part-filled q tile, the smallest context that splits in two
-    (17, 3001, 32, 4, 128),
-    (33, 2047, 16, 2, 64),    # two q tiles, the light one full
-    (65, 5000, 5, 1, 128),    # an odd count of q tiles, a head group of one
-    (203, 6000, 64, 4, 128),
-    (100, 700, 4, 2, 64),
-    (1600, 0, 4, 1, 128),     # diagonal tiles in every part
-    (1000, 400, 2, 1, 64),
+SHAPES = [  # T, pos, hq, hkv, d, parts on 256 compute units
+    (2, 957, 64, 4, 128, 1),     # 15 key tiles of a part-filled q tile: unsplit
+    (2, 959, 64, 4, 128, 2),     # 16: two parts
+    (2, 959, 16, 2, 64, 2),
+    (2, 1600, 64, 4, 128, 3),
+    (17, 3001, 32, 4, 128, 6),
+    (33, 2047, 16, 2, 64, 8),    # two q tiles, the light one full
+    (65, 5000, 5, 1, 128, 19),   # an odd count of q tiles, a head group of one
+    (203, 500, 32, 4, 128, 2),
+    (203, 6000, 64, 4, 128, 4),
+    (128, 500, 128, 8, 128, 1),  # the parts' way through memory costs more than it saves
+    (100, 700, 4, 2, 64, 3),
+    (1600, 0, 4, 1, 128, 3),     # diagonal tiles in every part
+    (1000, 400, 2, 1, 64, 3),
 ]
 
 
@@ -35,8 +41,8 @@ def _f64(q, kc, vc, pos, scale):
     return out
 
 
-@pytest.mark.parametrize("T,pos,hq,hkv,d", SHAPES)
-def test_prefill_split(ctx, hip, T, pos, hq, hkv, d):
+@pytest.mark.parametrize("T,pos,hq,hkv,d,parts", SHAPES)
+def test_prefill_split(ctx, hip, T, pos, hq, hkv, d, parts):
     print(f"[prefill_split] T={T} pos={pos} hq={hq} hkv={hkv} d={d}", flush=True)
     g = np.random.default_rng(T + pos)
     cap = pos + T + 5
@@ -51,7 +57,8 @@ def test_prefill_split(ctx, hip, T, pos, hq, hkv, d):
                         cap, scale)
     ctx.set_kernel_timing(True)
     hip.gqaAttention(ctx, args)
-    assert ctx.kernel_time("prefill_merge_kernel")[0] == 1  # split, one merge
+    assert hip.LIB.ds5_index_prefill_splits(256, pos, T, hq, hkv, d) == parts
+    assert ctx.kernel_time("prefill_merge_kernel")[0] == (parts > 1)  # one merge
     ctx.set_kernel_timing(False)
     got = ctx.to_numpy(out, np.float32, (T, hq, d)).astype(np.float64)
     err = np.abs(got - want).max()
