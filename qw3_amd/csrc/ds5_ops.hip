@@ -283,13 +283,14 @@ static bool experts_fast(ds5_buf x, ds5_buf gate, ds5_buf up, ds5_buf down, uint
 }
 
 // The experts run grouped (sorted by expert, on the matrix cores) when their Q8_0
-// banks take the wavefront kernels and the pairs share experts: each expert's weights are
-// read once instead of once per pair. From 11 pairs per 8 experts on average where there are
-// enough pairs to pay for the four more launches (128 experts of 2048 x 768, the MoE call: 24
-// tokens x 8 pairs 271 us pair by pair, 234 grouped; 17 tokens 192 and 211), from two pairs
-// per expert in any case.
+// banks take the wavefront kernels and the pairs share experts: from two pairs per expert on
+// average, each expert's weights are read once instead of once per pair. (At 11 pairs per 8
+// experts 128 experts of 2048 x 768 gain already, the MoE call of 24 tokens 268 us pair by
+// pair and 227 grouped, but 32 experts of 1024 x 512 lose, 11 tokens x 4 43 and 50; and the
+// wavefront kernels take x and h in f32 where the grouped products take 22 bits of them: error
+// of the experts' sums against 64 bits 1.8e-7 and 2.9e-7, so those calls stay with f32.)
 static bool experts_grouped(bool fast, uint32_t dt, uint64_t P, uint64_t E, uint64_t dim, uint64_t ffn) {
-    return fast && dt == DS5_DTYPE_Q8_0 && E > 0 && E <= kMoeGroupedMaxExperts && (P >= 2 * E || (8 * P >= 11 * E && P >= 32)) &&
+    return fast && dt == DS5_DTYPE_Q8_0 && E > 0 && E <= kMoeGroupedMaxExperts && P >= 2 * E &&
            P * std::max(dim, ffn) * 2 < (1ull << 32) && row_bytes_of(dt, std::max(dim, ffn)) * std::max(dim, ffn) <
                                                                 (1ull << 31);
 }

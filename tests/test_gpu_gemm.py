@@ -76,10 +76,12 @@ def test_mixed_group_is_its_products(ctx, hip, m):
         assert np.array_equal(ctx.to_numpy(a, np.uint32, (m, n)), ctx.to_numpy(b, np.uint32, (m, n)))
 
 
-@pytest.mark.parametrize("T,E,K,dim,ffn", [(22, 16, 1, 256, 96), (44, 16, 1, 512, 64), (60, 24, 4, 2048, 768)])
-def test_grouped_experts_few_pairs(ctx, hip, T, E, K, dim, ffn):
-    """Few pairs per expert (below, at and above the grouped threshold of 11 per 8 experts) against
-    float64, twice: rows of one expert land in any order."""
+@pytest.mark.parametrize("T,E,K,dim,ffn,grouped", [
+    (31, 16, 1, 256, 96, 0), (32, 16, 1, 512, 64, 1), (24, 96, 8, 256, 96, 1), (23, 96, 8, 256, 96, 0), (22, 64, 4, 256, 64, 0),
+    (60, 24, 4, 2048, 768, 1)])
+def test_grouped_experts_few_pairs(ctx, hip, T, E, K, dim, ffn, grouped):
+    """Few pairs per expert, on both sides of the two per expert from which the experts run grouped
+    (below, x and h stay in f32), against float64, twice: rows of one expert land in any order."""
     print(f"[moe] few pairs T={T} E={E} K={K}", flush=True)
     g = np.random.default_rng(T)
     (G, Gf), (U, Uf), (D, Df) = (q8_rows(g, E * a, b) for a, b in ((ffn, dim), (ffn, dim), (dim, ffn)))
@@ -102,10 +104,15 @@ def test_grouped_experts_few_pairs(ctx, hip, T, E, K, dim, ffn):
     lim += (K + 2) * 2.0 ** -23 * np.abs(want)
     bufs = [ctx.from_numpy(np.concatenate([v.reshape(-1), np.zeros(4, np.uint8)])) for v in (G, U, D)]
     runs = []
+    ctx.set_kernel_timing(True)
     for _ in range(2):
         out = ctx.createBuffer(T * dim * 4)
         hip.expertMlpSwiglu(ctx, ctx.from_numpy(x), *bufs, hip.DTYPE_Q8_0, pairs, out, T, dim, ffn, E)
         runs.append(ctx.to_numpy(out, np.float32, (T, dim)))
+    ctx.submit()
+    sorts = ctx.kernel_time("moe_sort_kernel")[0]
+    ctx.set_kernel_timing(False)
+    assert sorts == 2 * grouped
     assert np.all(np.abs(runs[0] - want) <= lim), float(np.max(np.abs(runs[0] - want) / lim))
     assert np.array_equal(runs[0], runs[1])
 
