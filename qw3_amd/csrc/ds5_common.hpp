@@ -221,12 +221,16 @@ struct RouterLaunch {
     float* h_out;
 };
 int launch_router(ds5_hip_ctx* ctx, const RouterLaunch& a);
-// The router's logits run in token x expert tiles (router_logits_tile_kernel) from
-// this many tokens, for f32 or f16 rows (dim % 4 == 0, x 16-byte and the rows 16- or
-// 8-byte aligned) without an in-kernel norm: with the norm's own launch 22 us at 24 tokens
-// x 128 experts x 2048 against 23 per token with the norm inside, 22 against 21 at 16.
-constexpr uint32_t kRouterTileMinTokens = 24;
-bool router_tiled(uint32_t w_dtype, uint32_t n_tokens, uint32_t dim, const void* x, const void* w);
+// The router's logits run in token x expert tiles (router_logits_tile_kernel) from 32 tokens,
+// and from 24 where there are kRouterTileMinWork products, for f32 or f16 rows (dim % 4 == 0,
+// x 16-byte and the rows 16- or 8-byte aligned) without an in-kernel norm. The tiles need the
+// norm's own launch and a chain of dim adds, the per-token kernel grows with the products:
+// MoE call with small experts, us, per token and in tiles, 24 tokens: 128 experts x 2048 77.7
+// and 76.6 (20 tokens 73.0 and 76.2), 128 x 4096 162 and 119, 512 x 2048 136 and 97, but 32 x
+// 1024 44.2 and 48.9, 64 x 512 40.5 and 42.6.
+constexpr uint32_t kRouterTileTokens = 32, kRouterTileMinTokens = 24;
+constexpr uint64_t kRouterTileMinWork = 5500000;
+bool router_tiled(uint32_t w_dtype, uint32_t n_tokens, uint32_t dim, uint32_t n_experts, const void* x, const void* w);
 
 // SwiGLU experts over device dispatch pairs; out accumulates. Token t's pairs
 // are order[offsets[t] .. offsets[t + 1]) in list order, or t*top_k .. when

@@ -487,7 +487,8 @@ int ds5_hip_moe(ds5_hip_ctx* ctx, const ds5_moe_args* a) {
     const bool norm_inside = norm && a->dim > kRmsSerialMaxDim && a->dim % 4 == 0 &&
                              a->router_dtype == DS5_DTYPE_F32 && aligned16(a->x) && aligned16(a->router_w) &&
                              aligned16(a->x_norm) &&
-                             !router_tiled(a->router_dtype, a->n_tokens, a->dim, ds5_ptr(a->x), ds5_ptr(a->router_w));
+                             !router_tiled(a->router_dtype, a->n_tokens, a->dim, a->n_experts, ds5_ptr(a->x),
+                                           ds5_ptr(a->router_w));
     if (norm && !norm_inside) {
         void* h = nullptr;
         const uint64_t bytes = (uint64_t)a->n_tokens * a->dim * 4;

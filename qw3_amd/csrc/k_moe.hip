@@ -958,9 +958,11 @@ static int launch_router_dt(ds5_hip_ctx* ctx, const RouterLaunch& a) {
     return launch_router_t<DT, 1>(ctx, a);
 }
 
-bool router_tiled(uint32_t w_dtype, uint32_t n_tokens, uint32_t dim, const void* x, const void* w) {
+bool router_tiled(uint32_t w_dtype, uint32_t n_tokens, uint32_t dim, uint32_t n_experts, const void* x, const void* w) {
     const uintptr_t wa = (uintptr_t)w;
-    return n_tokens >= kRouterTileMinTokens && dim % 4 == 0 && ((uintptr_t)x & 15u) == 0 &&
+    const bool many = n_tokens >= kRouterTileTokens ||
+                      (n_tokens >= kRouterTileMinTokens && (uint64_t)n_tokens * n_experts * dim >= kRouterTileMinWork);
+    return many && dim % 4 == 0 && ((uintptr_t)x & 15u) == 0 &&
            ((w_dtype == DS5_DTYPE_F32 && (wa & 15u) == 0) || (w_dtype == DS5_DTYPE_F16 && (wa & 7u) == 0));
 }
 
@@ -983,7 +985,7 @@ static int launch_router_tile(ds5_hip_ctx* ctx, const RouterLaunch& a) {
 int launch_router(ds5_hip_ctx* ctx, const RouterLaunch& a) {
     if (a.n_tokens == 0) return DS5_OK;
     int rc;
-    if (!a.x_norm_w && router_tiled(a.w_dtype, a.n_tokens, a.dim, a.x, a.w))
+    if (!a.x_norm_w && router_tiled(a.w_dtype, a.n_tokens, a.dim, a.n_experts, a.x, a.w))
         rc = a.w_dtype == DS5_DTYPE_F32 ? launch_router_tile<DS5_DTYPE_F32>(ctx, a)
                                         : launch_router_tile<DS5_DTYPE_F16>(ctx, a);
     else
