@@ -39,16 +39,17 @@ uint32_t ds5_index_plan_items(uint32_t len, uint32_t chunk);
 uint32_t ds5_index_plan_whole(uint32_t len, uint32_t chunk);
 uint32_t ds5_index_plan_partial(uint32_t len, uint32_t chunk);
 
-/* matmul_q8_mfma_kernel: a wavefront's x-plane offsets [nx][64] and raw-q dword
- * index, tile row and even/odd-block offsets [nq][64]. */
+/* matmul_q8_mfma_kernel: a wavefront's x-plane offsets [nx][64] and the first of the four
+ * dwords, the tile row and the even/odd-block offsets of its raw-q loads [2][64]; the blocks
+ * of group `group` of ks, out = [iterations, first, count, the last one (repeated past it)]. */
 void ds5_index_gemm_x(uint32_t wave, uint32_t W, uint32_t nx, uint32_t BM, uint32_t m0, uint32_t m, uint32_t k,
                       uint32_t* x_off);
 /* The grouped MoE form: tile row r reads plane row x_rows[min(m0 + r, m - 1)]. */
 void ds5_index_gemm_x_rows(uint32_t wave, uint32_t W, uint32_t nx, uint32_t BM, uint32_t m0, uint32_t m, uint32_t k,
                            const uint32_t* x_rows, uint32_t* x_off);
-void ds5_index_gemm_q(uint32_t wave, uint32_t threads, uint32_t nq, uint32_t w_rows, uint32_t row_dw, uint32_t n0,
-                      uint32_t n, uint32_t row_bytes, uint32_t* q_dw, uint32_t* q_row, uint32_t* q_even,
-                      uint32_t* q_odd);
+void ds5_index_gemm_q(uint32_t wave, uint32_t n0, uint32_t n, uint32_t row_bytes, uint32_t* q_dw, uint32_t* q_row,
+                      uint32_t* q_even, uint32_t* q_odd);
+void ds5_index_gemm_blocks(uint32_t nb, uint32_t group, uint32_t ks, uint32_t* out);
 
 /* prefill_attention_kernel: byte offsets [loads][64] of a K (v = 0) or V tile's
  * direct-to-LDS loads from key0 (clamped past kv_end); returns the load count.

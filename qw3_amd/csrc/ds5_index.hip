@@ -76,8 +76,9 @@ uint32_t ds5_index_plan_whole(uint32_t len, uint32_t chunk) { return ds5idx::pla
 uint32_t ds5_index_plan_partial(uint32_t len, uint32_t chunk) { return ds5idx::plan_partial(len, chunk); }
 
 // GEMM: the x-plane byte offsets (block 0) of wavefront `wave`'s nx loads
-// (x_off[i * 64 + lane]), and its nq raw-q loads' dword index, tile row and
-// even/odd-block offsets (q_*[i * 64 + lane]).
+// (x_off[i * 64 + lane]), and its two raw-q loads' first dword, tile row and
+// even/odd-block offsets (q_*[i * 64 + lane]); a group's [iterations, first block, blocks,
+// last block].
 void ds5_index_gemm_x(uint32_t wave, uint32_t W, uint32_t nx, uint32_t BM, uint32_t m0, uint32_t m, uint32_t k,
                       uint32_t* x_off) {
     for (uint32_t i = 0; i < nx; i++)
@@ -93,16 +94,18 @@ void ds5_index_gemm_x_rows(uint32_t wave, uint32_t W, uint32_t nx, uint32_t BM, 
             x_off[i * 64 + lane] = ds5idx::gemm_x_off_row(r, lane, x_rows[ds5idx::umin(m0 + r, m - 1)], k);
         }
 }
-void ds5_index_gemm_q(uint32_t wave, uint32_t threads, uint32_t nq, uint32_t w_rows, uint32_t row_dw, uint32_t n0,
-                      uint32_t n, uint32_t row_bytes, uint32_t* q_dw, uint32_t* q_row, uint32_t* q_even,
-                      uint32_t* q_odd) {
-    for (uint32_t i = 0; i < nq; i++)
+void ds5_index_gemm_q(uint32_t wave, uint32_t n0, uint32_t n, uint32_t row_bytes, uint32_t* q_dw, uint32_t* q_row,
+                      uint32_t* q_even, uint32_t* q_odd) {
+    for (uint32_t i = 0; i < 2; i++)
         for (uint32_t lane = 0; lane < 64; lane++) {
-            const uint32_t j = i * 64 + lane;
-            q_dw[j] = ds5idx::gemm_q_dword(i, lane, w_rows, row_dw);
-            q_row[j] = ds5idx::gemm_q_row(q_dw[j], wave, threads, row_dw);
-            ds5idx::gemm_q_off(q_dw[j], q_row[j], n0, n, row_bytes, row_dw, q_even[j], q_odd[j]);
+            const uint32_t j = i * 64 + lane, u = ds5idx::gemm_q_unit(i, lane);
+            q_dw[j] = ds5idx::gemm_q_dword(u);
+            q_row[j] = ds5idx::gemm_q_row(u, wave);
+            ds5idx::gemm_q_off(q_dw[j], q_row[j], n0, n, row_bytes, q_even[j], q_odd[j]);
         }
+}
+void ds5_index_gemm_blocks(uint32_t nb, uint32_t group, uint32_t ks, uint32_t* out) {
+    ds5idx::gemm_group_blocks(nb, group, ks, out[0], out[1], out[2], out[3]);
 }
 
 // Prefill: the byte offsets (from the tile's first key row) of every lane of

@@ -117,10 +117,10 @@ DS5_HD uint32_t plan_partial(uint32_t len, uint32_t chunk) { return (len == 0 ||
 // matmul_q8_mfma_kernel: block b's direct-to-LDS loads.
 // x: load i of wavefront `wave` fills stage bytes o = 1024 (wave + W i) + 16 lane;
 //    its plane byte offset (block 0) is row min(m0 + r, m - 1), swizzled chunk c.
-// raw q: dword d % 9 of a row's block, counted from the dword boundary at or below it: the
-//    offsets from the block's scalar base (w + 34 b, or w + 34 b - 2 for odd b). The kernel
-//    loads dwords 0..3, 4..7 and 5..8 of each row; gemm_q_dword and gemm_q_row enumerate all
-//    nine of every row of a tile, as the host checks do.
+// raw q: row r of the wavefront's 32 takes 48 bytes, three 16-byte lanes with dwords 0..3,
+//    4..7 and 5..8 of the nine from the dword boundary at or below its block: unit u = 3 r +
+//    part, 96 of them in two loads (the second's other lanes repeat the last). The offsets are
+//    from the block's scalar base (w + 34 b, or w + 34 b - 2 for odd b).
 // ---------------------------------------------------------------------------
 DS5_HD uint32_t gemm_x_tile_row(uint32_t o, uint32_t BM) { return (o % (BM * 64)) / 64; }
 // the offset of tile row r's swizzled chunk in plane row `row`
@@ -131,18 +131,24 @@ DS5_HD uint32_t gemm_x_off(uint32_t o, uint32_t lane, uint32_t BM, uint32_t m0, 
     const uint32_t r = gemm_x_tile_row(o, BM);
     return gemm_x_off_row(r, lane, umin(m0 + r, m - 1), k);
 }
-DS5_HD uint32_t gemm_q_row(uint32_t d, uint32_t wave, uint32_t threads, uint32_t row_dw) {
-    const uint32_t lr = d / row_dw;
-    return 16 * wave + (threads / 4) * (lr / 16) + lr % 16;
-}
-DS5_HD uint32_t gemm_q_dword(uint32_t i, uint32_t lane, uint32_t w_rows, uint32_t row_dw) {
-    return umin(64u * i + lane, w_rows * row_dw - 1);
-}
-DS5_HD void gemm_q_off(uint32_t d, uint32_t row, uint32_t n0, uint32_t n, uint32_t row_bytes, uint32_t row_dw,
-                       uint32_t& even, uint32_t& odd) {
+DS5_HD uint32_t gemm_q_unit(uint32_t i, uint32_t lane) { return umin(64u * i + lane, 95u); }
+// the tile row and the first of the four dwords of unit u of wavefront `wave`
+DS5_HD uint32_t gemm_q_row(uint32_t u, uint32_t wave) { return 32 * wave + u / 3; }
+DS5_HD uint32_t gemm_q_dword(uint32_t u) { return u % 3 == 0 ? 0u : u % 3 + 3u; }
+DS5_HD void gemm_q_off(uint32_t d, uint32_t row, uint32_t n0, uint32_t n, uint32_t row_bytes, uint32_t& even,
+                       uint32_t& odd) {
     const uint32_t rb = umin(n0 + row, n - 1) * row_bytes;
-    even = (rb & ~3u) + 4 * (d % row_dw);
-    odd = ((rb + 2) & ~3u) + 4 * (d % row_dw);
+    even = (rb & ~3u) + 4 * d;
+    odd = ((rb + 2) & ~3u) + 4 * d;
+}
+// The blocks [first, first + count) of group `group` of ks (every group runs the same number
+// of iterations; one past its blocks, or without any, repeats block `last`).
+DS5_HD void gemm_group_blocks(uint32_t nb, uint32_t group, uint32_t ks, uint32_t& iters, uint32_t& first,
+                              uint32_t& count, uint32_t& last) {
+    iters = (nb + ks - 1) / ks;
+    first = umin(group * iters, nb - 1);
+    count = umin(iters, nb - umin(group * iters, nb));
+    last = first + umax(count, 1u) - 1;
 }
 
 // ---------------------------------------------------------------------------

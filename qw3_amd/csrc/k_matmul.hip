@@ -582,8 +582,10 @@ __global__ __launch_bounds__(64 * W * KS, W* KS <= 4 ? 2 : W * KS / 4) void matm
     const uint32_t smem_lds = gemm_lds_addr(ring);
     // this group's blocks [first, first + iters) below nb: every group runs iters iterations
     // (the barriers), those past its blocks without loads or products
-    const uint32_t iters = (nb + KS - 1) / KS, first = min(group * iters, nb - 1);
-    const uint32_t blocks = min(iters, nb - min(group * iters, nb));
+    // (past its end the last block is asked for again, so that every iteration has the same
+    // loads outstanding; the loop ends on a full wait)
+    uint32_t iters, first, blocks, bl;
+    ds5idx::gemm_group_blocks(nb, group, KS, iters, first, blocks, bl);
 
     // x: load i of this wavefront fills bytes [1024 (wave + W i), +1024) of a stage, lane L
     // the 16 bytes at +16 L: plane, row r, slot L % 4 holding chunk (L % 4) ^ ((r >> 2) & 3).
@@ -608,13 +610,14 @@ __global__ __launch_bounds__(64 * W * KS, W* KS <= 4 ? 2 : W * KS / 4) void matm
     };
     // raw q: row r of the wavefront's 32 takes 48 bytes, three 16-byte lanes with dwords
     // 0..3, 4..7 and 5..8 of the nine from the dword boundary at or below its block: 96
-    // lanes of two loads (the others repeat the last, into the area's padding). 34 b is 0 mod 4 for even b and 2 mod 4 for odd b:
-    // scalar base w + 34 b or w + 34 b - 2, lane offsets per parity.
+    // lanes of two loads (the others repeat the last, into the area's padding). 34 b is 0 mod
+    // 4 for even b and 2 mod 4 for odd b: scalar base w + 34 b or w + 34 b - 2, lane offsets
+    // per parity.
     uint32_t qe[2], qo[2];
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-        const uint32_t u = min(64u * i + lane, 95u), part = u % 3;
-        ds5idx::gemm_q_off(part == 0 ? 0u : part + 3u, 32 * wave + u / 3, n0, n, row_bytes, 9, qe[i], qo[i]);
+        const uint32_t u = ds5idx::gemm_q_unit(i, (uint32_t)lane);
+        ds5idx::gemm_q_off(ds5idx::gemm_q_dword(u), ds5idx::gemm_q_row(u, wave), n0, n, row_bytes, qe[i], qo[i]);
     }
     auto issue_q = [&](uint32_t b, uint32_t slot, int i) {
         const bool odd = b & 1;
@@ -679,9 +682,6 @@ __global__ __launch_bounds__(64 * W * KS, W* KS <= 4 ? 2 : W * KS / 4) void matm
     // four of the previous pair's scale multiply-adds (across blocks too): a wavefront keeps
     // the matrix core and the VALU busy by itself, the scheduling fences hold the order.
     constexpr int kAhead = 6;
-    // Past the end the last block is asked for again, so that every iteration has the same
-    // loads outstanding; the loop ends on a full wait.
-    const uint32_t bl = first + max(blocks, 1u) - 1;
     auto issue = [&](uint32_t b, uint32_t stage, uint32_t bq, uint32_t slot, int n) {
         if (n < NX) issue_x(b, stage, n);
         else if (n < NX + 2) issue_q(bq, slot, n - NX);
@@ -754,8 +754,7 @@ __global__ __launch_bounds__(64 * W * KS, W* KS <= 4 ? 2 : W * KS / 4) void matm
                 }
                 const float sc = p == 0 ? ps : sb;
 #pragma unroll
-                for (int e = 4 * (q % 4); e < 4 * (q % 4) + 4; e++)
-{
+                for (int e = 4 * (q % 4); e < 4 * (q % 4) + 4; e++) {
                     float v = __builtin_fmaf(sc, t[cur ^ 1][q / 4][e], acc[U * pp + q / 4][e]);
                     asm volatile("" : "+v"(v));  // here, not sunk into a later block
                     acc[U * pp + q / 4][e] = v;

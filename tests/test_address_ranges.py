@@ -4,7 +4,7 @@ kernels' own index arithmetic (no GPU).
 The kernels compute their per-lane offsets and clamps with the __host__ __device__
 helpers of qw3_amd/csrc/ds5_index.hpp; libds5hip.so exports host wrappers of the same
 helpers (include/ds5_index.h), and these tests call them for every tile, load and lane
-of a launch at the BASELINE shapes (C0-C4) and at the Q8_0 shapes whose blocks start 2
+of a launch at the benchmark shapes (C0-C4) and at the Q8_0 shapes whose blocks start 2
 bytes off a dword, then assert that every access stays inside its view (and that the
 paged plan covers every position exactly once). A change to a helper changes the kernel
 and what these tests see alike. A GPU memory fault once came from exactly such
@@ -40,7 +40,8 @@ def ix(hip):
         "ds5_index_page_first": ([i32, u32, u32, P], u64), "ds5_index_plan_bounds": ([u32, P, P], None),
         "ds5_index_plan_len": ([i32, u32], u32), "ds5_index_plan_items": ([u32, u32], u32),
         "ds5_index_plan_whole": ([u32, u32], u32), "ds5_index_plan_partial": ([u32, u32], u32),
-        "ds5_index_gemm_x": ([u32] * 7 + [P], None), "ds5_index_gemm_q": ([u32] * 8 + [P] * 4, None),
+        "ds5_index_gemm_x": ([u32] * 7 + [P], None), "ds5_index_gemm_q": ([u32] * 4 + [P] * 4, None),
+        "ds5_index_gemm_blocks": ([u32] * 3 + [P], None),
         "ds5_index_gemm_x_rows": ([u32] * 7 + [P, P], None),
         "ds5_index_prefill_tile": ([u32, C.c_int, u32, u32, P], u32), "ds5_index_pf_q_token": ([u32] * 3, u32),
         "ds5_index_prefill_splits": ([u32] * 6, u32), "ds5_index_pf_key_tiles": ([u32] * 3, u32),
@@ -67,7 +68,7 @@ def test_index_header_symbols_exported(hip):
     """Every function include/ds5_index.h declares is exported by the library."""
     text = open(os.path.join(ROOT, "include", "ds5_index.h")).read()
     names = set(re.findall(r"^\s*(?:void|uint32_t|uint64_t)\s+(ds5_index_\w+)\(", text, re.M))
-    assert len(names) == 25
+    assert len(names) == 26
     for n in names:
         assert getattr(hip.LIB, n) is not None
 
@@ -289,11 +290,11 @@ def gemm_path_ok(w_addr, n, k, w_len, m=1):
     return w_addr % 4 == 0 and ((w_addr + end) % 4 == 0 or w_len >= end + 2) and fits
 
 
-def check_gemm(ix, m, n, k, w_addr, w_len, BM, BN, WM, WN):
-    """Every x-plane and weight byte the GEMM's direct-to-LDS loads read, for each
-    block b of every tile (offsets from the kernel's helpers); returns one past the
-    highest weight byte read."""
-    W = WM * WN
+def check_gemm(ix, m, n, k, w_addr, TM, W):
+    """Every x-plane and weight byte the GEMM's direct-to-LDS loads read, for each block b of
+    every tile of 32 TM tokens x 32 W columns (offsets from the kernel's helpers); returns one
+    past the highest weight byte read."""
+    BM, BN = 32 * TM, 32 * W
     nb = k // 32
     row_bytes = nb * Q8
     b = np.arange(nb)[:, None]
@@ -312,33 +313,35 @@ def check_gemm(ix, m, n, k, w_addr, w_len, BM, BN, WM, WN):
                 assert (plane == plane[0]).all()  # one plane per load
                 byte = off[i * 64:(i + 1) * 64].astype(np.int64)[None, :] + 64 * b
                 assert byte.min() >= 0 and (byte + 16).max() <= m * k * 2
-    # raw q: the dwords of each row's block from the dword boundary at or below it, a
-    # scalar base (34 b, or 34 b - 2 for odd b) plus the lane's even/odd offset
-    threads = W * 64
-    b_per = BN * 4 // threads
-    w_rows = 16 * b_per
-    nq = (w_rows * 9 + 63) // 64
-    hi = None
+    # raw q: two loads of 16 bytes a lane per wavefront and block: a scalar base (34 b, or
+    # 34 b - 2 for odd b) plus the lane's even / odd offset
+    hi = 0
     for n0 in range(0, n, BN):
         for w in range(W):
-            dw, row, even, odd = (_u32s(nq * 64) for _ in range(4))
-            ix.ds5_index_gemm_q(w, threads, nq, w_rows, 9, n0, n, row_bytes, _ptr(dw), _ptr(row), _ptr(even),
-                                _ptr(odd))
+            dw, row, even, odd = (_u32s(128) for _ in range(4))
+            ix.ds5_index_gemm_q(w, n0, n, row_bytes, _ptr(dw), _ptr(row), _ptr(even), _ptr(odd))
             dw, row, even, odd = (a.astype(np.int64) for a in (dw, row, even, odd))
             base = Q8 * b - (b % 2) * 2                    # the scalar base (non-negative: b >= 1 when odd)
             assert base.min() >= 0
             byte = base + np.where(b % 2 == 0, even[None, :], odd[None, :])
             rb = np.minimum(n0 + row, n - 1) * row_bytes
-            # the bytes are those of the dword boundary at or below the block
-            want = (rb[None, :] + Q8 * b) // 4 * 4 + 4 * (dw % 9)[None, :]
+            # the bytes are those from the dword boundary at or below the block
+            want = (rb[None, :] + Q8 * b) // 4 * 4 + 4 * dw[None, :]
             assert (byte == want).all()
-            assert ((w_addr + byte) % 4 == 0).all()  # dword loads stay aligned
-            top = int((byte + 4).max())
-            hi = top if hi is None else max(hi, top)
-            # the wavefront loaded exactly the rows its threads convert (thread c: row c / 4)
-            conv = {(c + threads * u) // 4 for c in range(64 * w, 64 * w + 64) for u in range(b_per)}
-            assert set(row.tolist()) == conv
+            assert ((w_addr + byte) % 4 == 0).all()  # the loads stay on dwords
+            hi = max(hi, int((byte + 16).max()))
+            # LDS unit u = 64 i + lane of the wavefront's area: row u / 3 of its 32, whose three
+            # 16-byte units hold all nine dwords, four a unit
+            u = np.minimum(np.arange(128), 95)
+            assert (row == 32 * w + u // 3).all()
+            for r in range(32):
+                d = dw[3 * r:3 * r + 3]
+                assert {int(v) + e for v in d for e in range(4)} == set(range(9))
     return hi
+
+
+# the kernel's tiles, (32 rows, wavefronts of 32 columns): the split forms, unsplit ones and the experts'
+GEMM_TILES = [(1, 1), (1, 4), (2, 4), (4, 4)]
 
 
 @pytest.mark.parametrize("m,n,k", [
@@ -346,15 +349,30 @@ def check_gemm(ix, m, n, k, w_addr, w_len, BM, BN, WM, WN):
     (17, 256, 256), (16, 5, 32 * 3), (33, 129, 32 * 7),
     (128, 256, 32), (130, 128, 64), (256, 384, 96), (136, 200, 160),
 ])
-@pytest.mark.parametrize("tile", [(128, 128, 4, 2), (32, 64, 2, 2), (64, 128, 2, 2), (128, 128, 2, 2)])
+@pytest.mark.parametrize("tile", GEMM_TILES)
 def test_gemm_load_block_addresses(ix, m, n, k, tile):
-    """Both GEMM tiles; odd block counts put every other row's blocks at 2 mod 4."""
+    """Every GEMM tile; odd block counts put every other row's blocks at 2 mod 4."""
     end = n * (k // 32) * Q8
     for w_len in (end, end + 2):
         if not gemm_path_ok(0, n, k, w_len, m):
             continue  # matmul_path sends this view to the serial kernel
-        hi = check_gemm(ix, m, n, k, 0, w_len, *tile)
+        hi = check_gemm(ix, m, n, k, 0, *tile)
         assert hi <= w_len, (hi, w_len)
+
+
+@pytest.mark.parametrize("nb", [1, 2, 3, 4, 5, 7, 8, 9, 10, 11, 12, 64, 65, 257])
+@pytest.mark.parametrize("ks", [1, 4])
+def test_gemm_groups_cover_the_blocks(ix, nb, ks):
+    """The groups' ranges cover every block once; each group has the same iterations (they share
+    a barrier), and what it asks for past its blocks, or without any, is a block of the matrix."""
+    out, seen = _u32s(4), []
+    for g in range(ks):
+        ix.ds5_index_gemm_blocks(nb, g, ks, _ptr(out))
+        iters, first, count, last = (int(v) for v in out)
+        assert iters == -(-nb // ks) and count <= iters
+        assert 0 <= first <= last < nb and last == first + max(count, 1) - 1
+        seen += range(first, first + count)
+    assert seen == list(range(nb))
 
 
 def _moe_tiles(pairs_expert, E, rows):
@@ -368,14 +386,13 @@ def _moe_tiles(pairs_expert, E, rows):
 
 @pytest.mark.parametrize("T,K,E,dim,ffn", [(64, 8, 16, 2048, 768), (40, 8, 12, 512, 256), (24, 3, 8, 256, 96),
                                            (2048, 8, 128, 2048, 768)])
-@pytest.mark.parametrize("tile", [(64, 128, 2, 2), (128, 128, 4, 2)])
+@pytest.mark.parametrize("tile", GEMM_TILES[1:])
 def test_grouped_moe_gemm_x_rows(ix, hip, T, K, E, dim, ffn, tile):
     """The grouped MoE products' x loads: gate / up read sorted row r's token's row of the
     T-row x planes (x_rows = the pairs' tokens in sorted order), down the P-row h planes
     (no map); every load stays inside its planes, reads a row of the tile's own expert,
     and the tile count stays within moe_max_tiles (P / rows + E + 1)."""
-    BM, BN, WM, WN = tile
-    W = WM * WN
+    BM, W = 32 * tile[0], tile[1]
     g = np.random.default_rng(T + E)
     P = T * K
     tokens = np.repeat(np.arange(T), K)
@@ -412,7 +429,7 @@ def test_gemm_slack_rule_is_needed(ix):
     n, k = 129, 32 * 7
     end = n * (k // 32) * Q8
     assert end % 4 == 2 and not gemm_path_ok(0, n, k, end)
-    assert check_gemm(ix, 64, n, k, 0, end, 32, 64, 2, 2) == end + 2
+    assert check_gemm(ix, 64, n, k, 0, 1, 1) == end + 2
 
 
 # ---------------------------------------------------------------------------
