@@ -1,9 +1,9 @@
 #!/usr/bin/env python3
-"""Benchmark of the gfx950 attention path on the BASELINE configurations.
+"""Benchmark of the gfx950 attention path on its five configurations (C0-C4).
 
     python bench.py [--steps K] [--warmup W] [--gpus 1] [--no-cpu] [--only C1,C2,...]
 
-Prints ONE JSON line. The headline workload is config 1:
+Prints ONE JSON line. The headline workload is C1:
 one decode token through 48 independent layers' attention, Qwen3-30B-A3B shape
 (32 q / 4 kv heads, head_dim 128), f16 KV cache of 8192 tokens per layer. A
 "step" is that 48-layer sweep: per layer one fused attention step (q/k
@@ -28,7 +28,7 @@ roofline.achieved = algorithmic bytes of one decode_split_kernel launch (one
 cpu_baseline = the oracle on C1 layers, 1 core (per-config CPU figures are in
          configs.C*.cpu)
 
-configs.C0..C4 hold each BASELINE configuration's GPU figures, CPU figures
+configs.C0..C4 hold each configuration's GPU figures, CPU figures
 and parity; floors holds the measured cost of one dependent launch and of a
 bare once-read of a C1 layer's K/V; extra holds the projection / MoE legs
 (the rows after the attention path).
@@ -52,7 +52,7 @@ F16_MFMA_PEAK_TFLOPS = 2516.6
 BF16_MFMA_PEAK_TFLOPS = 2516.6  # dense bf16 matrix-core peak (same as f16)
 QKV_BYTES = 5120 * 64 * 34 + 2048 * 4 + 5120 * 4  # Qwen3-30B-A3B q/k/v weights + x + out per layer
 ROCPROF_JSON = os.path.join(ROOT, "profiles", "rocprof_kernel_us.json")
-OUT_ATOL, OUT_COS = 2e-3, 0.99999  # BASELINE attention-output gates
+OUT_ATOL, OUT_COS = 2e-3, 0.99999  # attention-output gates
 LOG = sys.stderr
 
 
@@ -751,7 +751,7 @@ def main():
     ap.add_argument("--leg-seconds", type=float, default=0.5,
                     help="minimum device time of each secondary timed leg (graph replays / eager kernel timing)")
     ap.add_argument("--only", default="C0,C1,C2,C3,C4,FLOOR,SIX,QKV,WO,MOE,LAYER,QKVP,BLK,MOEP",
-                    help="comma list of legs: C0-C4 (BASELINE configs; C1 is the headline), FLOOR (launch and "
+                    help="comma list of legs: C0-C4 (the configurations; C1 is the headline), FLOOR (launch and "
                          "bare-read floors), SIX (C1 through the six separate ops), QKV / QKVP (decode / prefill "
                          "q/k/v projections), WO (output projection + residual), MOE (decode MoE block), LAYER (48 whole "
                          "decode layers in the engine's fused order), BLK (prefill attention block: projections + "

@@ -25,7 +25,7 @@
 // One workgroup per (token, head) reading whole K rows per thread (the generic kernel,
 // which other head sizes keep) took 757 us at 3000 positions of 32 q / 4 kv heads x 128
 // and 480 us for a 500-token prompt; the attention blocks around them went from 782 to
-// 21 us and from 575 to 135 us (norm, rope and append in one launch included).
+// 21 us and from 575 to 117 us (norm, rope and append in one launch included).
 #include "ds5_common.hpp"
 
 namespace {

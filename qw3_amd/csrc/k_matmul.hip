@@ -221,10 +221,11 @@ __global__ __launch_bounds__(kMmThreads) void matmul_rows_kernel(const float* __
 // x' = x * 2^(14 - E) with 2^E <= max |x row| < 2^(E+1), so |x'| < 2^15 fits
 // f16, and split into two f16 parts, x' = hi + lo (lo the f16 rounding of
 // x' - hi): 22 significant bits, and no overflow or loss of range whatever
-// the row's magnitude. Per 32-element block and 16 x 16 output tile, two
-// v_mfma_f32_16x16x32_f16 (lo, then hi) into a zeroed temporary, then
-// acc += scale * tmp in f32 (the scale belongs to the weight row: one per lane
-// in the result layout); the epilogue undoes the row's power of two exactly.
+// the row's magnitude. Per 32-element block and 32 x 32 output tile, four
+// v_mfma_f32_32x32x16_f16 (lo, lo, hi, hi: two products of 16 elements each) into a
+// zeroed temporary, then acc += scale * tmp in f32 (the scale belongs to the weight
+// row: one per lane in the result layout); the epilogue undoes the row's power of two
+// exactly.
 //
 // matmul_x_split_kernel writes the two planes and the row exponents into the
 // context workspace; matmul_q8_mfma_kernel then only copies x tiles.
@@ -479,7 +480,7 @@ __device__ __forceinline__ void lds_dma(uint32_t off, uint64_t base, uint32_t ld
 }
 
 // EPI = 1: the attention block's q / k / v projections (entries 0, 1, 2 of the
-// group), 128 x 128 tiles: a tile is 128 tokens of one head's 128 dims, and
+// group), tiles of 128 columns: a tile is 32 TM tokens of one head's 128 dims, and
 // the epilogue turns it into what the prefill attention reads -- k: RMSNorm
 // (serial sum) and rotation, f16 into the cache row pos + t of its kv head; v:
 // f16 into the cache; q: RMSNorm, rotation, times q_scale, f16 into the q
@@ -816,9 +817,8 @@ __global__ __launch_bounds__(64 * W * KS, W* KS <= 4 ? 2 : W * KS / 4) void matm
     }
 
     if constexpr (EPI == 1) {
-        // One head (128 columns, four wavefronts) at a time goes through LDS; then thread t
-        // takes row t / 8 (+ 64, ...), dims k8 + [0, 8) and 64 + k8 + [0, 8) (8 rope
-        // pairs), k8 = 8 (t % 8).
+        // The tile's head goes through LDS; then thread t takes row t / 8 (+ kRowsPer, ...),
+        // dims k8 + [0, 8) and 64 + k8 + [0, 8) (8 rope pairs), k8 = 8 (t % 8).
         constexpr int D = 128, HALF = 64, TROW = kTileRow, kRowsPer = kGroupThreads * KS / 8;
         const int r0 = threadIdx.x / 8, k8 = 8 * (threadIdx.x % 8);
         const float* nw = entry == 0 ? ep.q_norm : ep.k_norm;
@@ -830,81 +830,78 @@ __global__ __launch_bounds__(64 * W * KS, W* KS <= 4 ? 2 : W * KS / 4) void matm
             *(float4*)&w1[4] = *(const float4*)(nw + HALF + k8 + 4);
         }
         float* tl = reinterpret_cast<float*>(smem);
-#pragma unroll 1
-        for (uint32_t hd = 0; hd < BN / D && n0 + D * hd < n; hd++) {  // uniform
-            const uint32_t head = tile * (BN / D) + hd;
-            __syncthreads();  // every wavefront's last read of the bytes
-            if (wave / 4 == hd && group == 0) {
+        const uint32_t head = tile;  // column tile j of an entry is head j
+        __syncthreads();  // every wavefront's last read of the bytes
+        if (group == 0) {
 #pragma unroll
-                for (int i = 0; i < TM; i++)
+            for (int i = 0; i < TM; i++)
 #pragma unroll
-                    for (int e = 0; e < 16; e++) {
-                        const int lr = 32 * i + 8 * (e / 4) + 4 * h + e % 4;
-                        tl[lr * TROW + (col & 127)] = __builtin_ldexpf(acc[i][e], s_sh[lr]);
-                    }
-            }
-            __syncthreads();
-#pragma unroll 1
-            for (int r = r0; r < BM; r += kRowsPer) {
-                const uint32_t tok = m0 + r;
-                if (m0 + (r - r0) >= m) break;  // uniform: no rows left
-                const bool ok = tok < m;
-                const float* trow = tl + r * TROW;
-                float x0[8], x1[8], c[8], sn[8];
-                if (entry != 2) {
-                    const float* cs = ep.cs + (uint64_t)min(tok, m - 1) * D;
-                    *(float4*)&c[0] = *(const float4*)(cs + k8);
-                    *(float4*)&c[4] = *(const float4*)(cs + k8 + 4);
-                    *(float4*)&sn[0] = *(const float4*)(cs + HALF + k8);
-                    *(float4*)&sn[4] = *(const float4*)(cs + HALF + k8 + 4);
+                for (int e = 0; e < 16; e++) {
+                    const int lr = 32 * i + 8 * (e / 4) + 4 * h + e % 4;
+                    tl[lr * TROW + col] = __builtin_ldexpf(acc[i][e], s_sh[lr]);
                 }
-                *(float4*)&x0[0] = *(const float4*)(trow + k8);
-                *(float4*)&x0[4] = *(const float4*)(trow + k8 + 4);
-                *(float4*)&x1[0] = *(const float4*)(trow + HALF + k8);
-                *(float4*)&x1[4] = *(const float4*)(trow + HALF + k8 + 4);
-                f16x8_t y0v, y1v;
-                f16* dst;
-                if (entry == 2) {  // v: f16 append
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int r = r0; r < BM; r += kRowsPer) {
+            const uint32_t tok = m0 + r;
+            if (m0 + (r - r0) >= m) break;  // uniform: no rows left
+            const bool ok = tok < m;
+            const float* trow = tl + r * TROW;
+            float x0[8], x1[8], c[8], sn[8];
+            if (entry != 2) {
+                const float* cs = ep.cs + (uint64_t)min(tok, m - 1) * D;
+                *(float4*)&c[0] = *(const float4*)(cs + k8);
+                *(float4*)&c[4] = *(const float4*)(cs + k8 + 4);
+                *(float4*)&sn[0] = *(const float4*)(cs + HALF + k8);
+                *(float4*)&sn[4] = *(const float4*)(cs + HALF + k8 + 4);
+            }
+            *(float4*)&x0[0] = *(const float4*)(trow + k8);
+            *(float4*)&x0[4] = *(const float4*)(trow + k8 + 4);
+            *(float4*)&x1[0] = *(const float4*)(trow + HALF + k8);
+            *(float4*)&x1[4] = *(const float4*)(trow + HALF + k8 + 4);
+            f16x8_t y0v, y1v;
+            f16* dst;
+            if (entry == 2) {  // v: f16 append
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    y0v[j] = (f16)x0[j];
+                    y1v[j] = (f16)x1[j];
+                }
+                dst = ep.v_cache + ((uint64_t)head * ep.max_ctx + ep.pos + tok) * D;
+            } else {
+                if (entry == 0) {
+                    // q: the thread's two quarters (pairs k8 .. k8 + 3 and k8 + 4 .. k8 + 7),
+                    // then the head's 8 threads in the balanced tree's order (xor 1, 2, 4)
+                    float ss = qk_quarter_sumsq(x0[0], x1[0], x0[1], x1[1], x0[2], x1[2], x0[3], x1[3]) +
+                               qk_quarter_sumsq(x0[4], x1[4], x0[5], x1[5], x0[6], x1[6], x0[7], x1[7]);
+#pragma unroll
+                    for (int mm = 1; mm < 8; mm <<= 1) ss += __shfl_xor(ss, mm, 64);
+                    const float r1 = rms_inv(ss, (float)D, ep.eps) * ep.q_scale;
 #pragma unroll
                     for (int j = 0; j < 8; j++) {
-                        y0v[j] = (f16)x0[j];
-                        y1v[j] = (f16)x1[j];
+                        _Float16 o0, o1;
+                        qk_q_pair(x0[j], x1[j], w0[j], w1[j], c[j], sn[j], r1, o0, o1);
+                        y0v[j] = o0;
+                        y1v[j] = o1;
                     }
-                    dst = ep.v_cache + ((uint64_t)head * ep.max_ctx + ep.pos + tok) * D;
-                } else {
-                    if (entry == 0) {
-                        // q: the thread's two quarters (pairs k8 .. k8 + 3 and k8 + 4 .. k8 + 7),
-                        // then the head's 8 threads in the balanced tree's order (xor 1, 2, 4)
-                        float ss = qk_quarter_sumsq(x0[0], x1[0], x0[1], x1[1], x0[2], x1[2], x0[3], x1[3]) +
-                                   qk_quarter_sumsq(x0[4], x1[4], x0[5], x1[5], x0[6], x1[6], x0[7], x1[7]);
+                } else {  // k: the reference's serial sum of the row
+                    const float inv = rms_inv(qk_serial_sumsq(trow, D), (float)D, ep.eps);
 #pragma unroll
-                        for (int mm = 1; mm < 8; mm <<= 1) ss += __shfl_xor(ss, mm, 64);
-                        const float r1 = rms_inv(ss, (float)D, ep.eps) * ep.q_scale;
-#pragma unroll
-                        for (int j = 0; j < 8; j++) {
-                            _Float16 o0, o1;
-                            qk_q_pair(x0[j], x1[j], w0[j], w1[j], c[j], sn[j], r1, o0, o1);
-                            y0v[j] = o0;
-                            y1v[j] = o1;
-                        }
-                    } else {  // k: the reference's serial sum of the row
-                        const float inv = rms_inv(qk_serial_sumsq(trow, D), (float)D, ep.eps);
-#pragma unroll
-                        for (int j = 0; j < 8; j++) {
-                            float y0, y1;
-                            qk_rotate(qk_norm_mul(x0[j], inv, w0[j]), qk_norm_mul(x1[j], inv, w1[j]), c[j], sn[j], y0,
-                                      y1);
-                            y0v[j] = (f16)y0;
-                            y1v[j] = (f16)y1;
-                        }
+                    for (int j = 0; j < 8; j++) {
+                        float y0, y1;
+                        qk_rotate(qk_norm_mul(x0[j], inv, w0[j]), qk_norm_mul(x1[j], inv, w1[j]), c[j], sn[j], y0,
+                                  y1);
+                        y0v[j] = (f16)y0;
+                        y1v[j] = (f16)y1;
                     }
-                    dst = entry == 0 ? ep.q16 + ((uint64_t)tok * ep.n_q_heads + head) * D
-                                     : ep.k_cache + ((uint64_t)head * ep.max_ctx + ep.pos + tok) * D;
                 }
-                if (ok) {
-                    *(f16x8_t*)(dst + k8) = y0v;
-                    *(f16x8_t*)(dst + HALF + k8) = y1v;
-                }
+                dst = entry == 0 ? ep.q16 + ((uint64_t)tok * ep.n_q_heads + head) * D
+                                 : ep.k_cache + ((uint64_t)head * ep.max_ctx + ep.pos + tok) * D;
+            }
+            if (ok) {
+                *(f16x8_t*)(dst + k8) = y0v;
+                *(f16x8_t*)(dst + HALF + k8) = y1v;
             }
         }
         return;
@@ -1207,8 +1204,8 @@ constexpr uint32_t kGemmMinM = 16;
 // the block starts on a dword boundary; for the last block that stays inside the
 // view only if the weights end on a dword boundary or the view has 2 more bytes.
 // The GEMM reads x as float4 (x 16-byte aligned), stores single floats (out
-// 4-byte aligned) and reads q in 8-byte runs from the dword boundary at or below
-// them, with the same end condition. Its loads address an x plane and the
+// 4-byte aligned) and reads q as 16-byte loads of dwords 0..3, 4..7 and 5..8 of the same
+// nine, with the same end condition. Its loads address an x plane and the
 // weights with 32-bit byte offsets from a scalar base.
 static bool gemm_offsets_fit(uint32_t m, uint32_t k, uint64_t w_end) {
     return (uint64_t)m * k * 2 < (1ull << 32) && w_end + 2 < (1ull << 32);

@@ -30,45 +30,45 @@ constexpr uint32_t kSerialMaxDim = kRmsSerialMaxDim;
 
 // The serial sum of a row's squares staged in LDS (16-byte aligned), in element order.
 __device__ __forceinline__ float staged_sumsq(const float* row, uint32_t dim) {
-            float sumsq = 0.0f;
-            // 32 squares per batch in two alternating register sets: a batch's reads are
-            // issued before the previous batch's adds (the scheduling fences keep them
-            // there), so the dependent chain never waits for LDS
-            constexpr int B = 8;  // float4 per batch
-            const uint32_t nb = dim / (4 * B), db = nb * 4 * B;
-            float4 ba[B], bb[B];
-            auto rd = [&](float4(&d)[B], uint32_t batch) {
-    #pragma unroll
-                for (int b = 0; b < B; b++) d[b] = *(const float4*)(row + 4 * B * batch + 4 * b);
-            };
-            auto add = [&](const float4(&d)[B]) {
-    #pragma unroll
-                for (int b = 0; b < B; b++) {
-                    sumsq += d[b].x;
-                    sumsq += d[b].y;
-                    sumsq += d[b].z;
-                    sumsq += d[b].w;
-                }
-            };
-            // pairs of batches, every read unconditional (a read under a branch makes the
-            // compiler's wait at the join count it as outstanding on both paths)
-            const uint32_t np = nb / 2;
-            if (np) rd(ba, 0);
-            for (uint32_t i = 0; i < np; i++) {
-                rd(bb, 2 * i + 1);
-                __builtin_amdgcn_sched_barrier(0);
-                add(ba);
-                __builtin_amdgcn_sched_barrier(0);
-                rd(ba, min(2 * i + 2, 2 * np - 1));
-                __builtin_amdgcn_sched_barrier(0);
-                add(bb);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            if (nb & 1) {
-                rd(ba, nb - 1);
-                add(ba);
-            }
-            for (uint32_t j = db; j < dim; j++) sumsq += row[j];
+    float sumsq = 0.0f;
+    // 32 squares per batch in two alternating register sets: a batch's reads are
+    // issued before the previous batch's adds (the scheduling fences keep them
+    // there), so the dependent chain never waits for LDS
+    constexpr int B = 8;  // float4 per batch
+    const uint32_t nb = dim / (4 * B), db = nb * 4 * B;
+    float4 ba[B], bb[B];
+    auto rd = [&](float4(&d)[B], uint32_t batch) {
+#pragma unroll
+        for (int b = 0; b < B; b++) d[b] = *(const float4*)(row + 4 * B * batch + 4 * b);
+    };
+    auto add = [&](const float4(&d)[B]) {
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            sumsq += d[b].x;
+            sumsq += d[b].y;
+            sumsq += d[b].z;
+            sumsq += d[b].w;
+        }
+    };
+    // pairs of batches, every read unconditional (a read under a branch makes the
+    // compiler's wait at the join count it as outstanding on both paths)
+    const uint32_t np = nb / 2;
+    if (np) rd(ba, 0);
+    for (uint32_t i = 0; i < np; i++) {
+        rd(bb, 2 * i + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        add(ba);
+        __builtin_amdgcn_sched_barrier(0);
+        rd(ba, min(2 * i + 2, 2 * np - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        add(bb);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (nb & 1) {
+        rd(ba, nb - 1);
+        add(ba);
+    }
+    for (uint32_t j = db; j < dim; j++) sumsq += row[j];
     return sumsq;
 }
 

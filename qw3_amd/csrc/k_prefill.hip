@@ -884,8 +884,8 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     const float2* ml = p.part_ml + row * p.n_splits;
     const float* o = p.part_o + row * p.n_splits * D + c4;
     // B parts' loads at a time: the fold waits on memory, not on bandwidth, when the rows are
-    // few (2 tokens at 8000, 10 parts: 7.1 us one by one, 5.4 by eights; 1000 tokens in 2
-    // parts: 9.5 by twos, 13 by eights). A part without a key tile of this row's q tile holds
+    // few (2 tokens at 8000, 15 parts: 7.8 us one by one, 5.3 by eights; 1000 tokens at 1000,
+    // 2 parts: 8.8 by twos, 12 by eights). A part without a key tile of this row's q tile holds
     // nothing; it is read and dropped.
     auto part = [&](uint32_t s) { return min(s, p.n_splits - 1); };
     auto used = [&](uint32_t s) {

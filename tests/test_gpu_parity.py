@@ -1,6 +1,6 @@
 """Parity of the gfx950 backend with the CPU oracle, through the C ABI.
 
-Gates (BASELINE): KV slot/page indexing bit-exact; cached K/V within 1 f16 ulp;
+Gates: KV slot/page indexing bit-exact; cached K/V within 1 f16 ulp;
 attention output max-abs <= 2e-3 and cosine >= 0.99999. Inputs are the same
 seeded host arrays for both sides. The reference's fixture tolerances apply to
 the vendored fixtures.
@@ -285,7 +285,7 @@ def test_decode_lengths_and_groups(ctx, hip, oracle, L, hq, hkv, hd):
 
 
 # ---------------------------------------------------------------------------
-# the fused step at the BASELINE configs
+# the fused step at the benchmark configurations
 # ---------------------------------------------------------------------------
 
 def _run_step(ctx, hip, q, k, v, qn, kn, positions, kc, vc, pos, s, fused):
